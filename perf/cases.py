@@ -337,3 +337,93 @@ _TOLERANCE = {
 def tolerance(case):
     by_kind = _TOLERANCE[case["dtype"]]
     return dict(by_kind.get(case["kind"], by_kind.get(None)))
+
+
+# ---------------------------------------------------------------- the same in 64 bits
+
+def _exact_norm(x):
+    centered = x - x.mean(-1, keepdim=True)
+    return centered / (centered.square().mean(-1, keepdim=True) + 1e-5).sqrt()
+
+
+def _exact_gelu(x):
+    return torch.nn.functional.gelu(x, approximate="tanh")
+
+
+def _exact_attention(q, k, v, mask):
+    scores = q @ k.transpose(-1, -2).contiguous() / math.sqrt(q.shape[-1]) + mask
+    return scores.softmax(-1) @ v
+
+
+def _exact_transformer(model, ids, heads):
+    batch, t = ids.shape
+    mask = torch.full((t, t), -1e4, device="cuda", dtype=torch.float64).triu(1)
+
+    def value(tensor):
+        return _view(tensor).double()
+
+    def linear(layer, x):
+        return x @ value(layer.weight) + value(layer.bias)
+
+    def norm(layer, x):
+        return _exact_norm(x) * (1 + value(layer.gain)) + value(layer.bias)
+
+    def split(x):
+        return x.reshape(batch, t, heads, -1).transpose(1, 2).contiguous()
+
+    x = value(model.table)[ids] + value(model.pos)[:t]
+    for block in model.blocks:
+        h = norm(block.ln1, x)
+        mixed = _exact_attention(split(linear(block.q, h)), split(linear(block.k, h)), split(linear(block.v, h)), mask)
+        x = x + linear(block.o, mixed.transpose(1, 2).reshape(x.shape))
+        x = x + linear(block.fc2, _exact_gelu(linear(block.fc1, norm(block.ln2, x))))
+    return linear(model.unembed, norm(model.ln_f, x))
+
+
+def _exact_train_step(s):
+    ids, targets = _view(s["ids"]), _view(s["targets"])
+    p = {name: _view(s["params"][name]["value"]).double().requires_grad_() for name in _PARAMETERS}
+    x = p["table"][ids]
+    f = (_exact_norm(x) * (1 + p["gain"]) + p["shift"]) @ p["w1"] + p["b1"]
+    y = x + _exact_gelu(f) @ p["w2"] + p["b2"]
+    loss = -(y @ p["wo"]).log_softmax(1).gather(1, targets[:, None]).sum()
+    loss.backward()
+    beta1, beta2, eps, decay, lr = torch.tensor([0.9, 0.999, 1e-8, 0.01, 1e-3], dtype=torch.float32).double().tolist()
+    out = {"loss": loss.detach().reshape([])}
+    for name in _PARAMETERS:
+        g = p[name].grad
+        m = beta1 * _view(s["params"][name]["m"]).double() + (1 - beta1) * g
+        v = beta2 * _view(s["params"][name]["v"]).double() + (1 - beta2) * g * g
+        moved = m / (1 - beta1 ** 10) / ((v / (1 - beta2 ** 10)).sqrt() + eps)
+        out[name + ".value"] = p[name].detach() * (1 - lr * decay) - lr * moved
+        out[name + ".m"], out[name + ".v"] = m, v
+    return out
+
+
+def exact(case, seed):
+    """What `run` returns for these inputs, in plain torch with 64-bit numbers and nothing rounded on the way.
+    None in the place of whole numbers that ties of rounded values decide."""
+    c, s = case, prepare(case, seed)
+    kind, half = c["kind"], c["dtype"] == "f16"
+    if kind == "transformer":
+        return _exact_transformer(s["model"], _view(s["ids"]), c["heads"])
+    if kind == "train_step":
+        return _exact_train_step(s)
+    v = {name: _view(t) for name, t in s.items() if isinstance(t, Tensor)}
+    v = {name: t if t.dtype == torch.int64 else t.double() for name, t in v.items()}
+    if kind == "small":
+        x = v["x"] + v["y"]
+        return [x, _exact_norm(x) * (v["gain"] + 1) + v["bias"]]
+    if kind == "matmul":
+        return (v["a"].t() if c["ta"] else v["a"]) @ (v["b"].t() if c["tb"] else v["b"])
+    if kind == "attention":
+        return _exact_attention(v["q"], v["k"], v["v"], v["mask"])
+    if kind == "row_ops":
+        h = _exact_gelu(v["x"] + v["bias"])
+        return {"h": h, "sum": h.sum(1), "max": h.max(1).values, "argmax": None if half else h.argmax(1)}
+    if kind == "embedding":
+        table = torch.zeros(c["vocab"], c["width"], dtype=torch.float64, device="cuda")
+        return [v["table"][v["ids"]], table.index_add_(0, v["ids"], v["grad"])]
+    ranked, order = v["logits"].sort(dim=1, descending=True, stable=True)
+    ranked = ranked.softmax(1)
+    return {"order": order, "ranked": ranked, "cumulative": ranked.cumsum(1)}
