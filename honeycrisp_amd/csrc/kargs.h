@@ -203,13 +203,14 @@ typedef struct {
 } hck_scan_args;
 
 /* argsort of axes longer than one block sorts at once: sorted runs of (key, index) pairs, one
- * array of each per line ([lines, reduce], line = outer * inner + inner index), merged pairwise. */
+ * array of each per line ([lines, reduce], line = outer * inner + inner index), merged 16 at a time.
+ * Keys are uint32_t for float types, uint64_t for int64. */
 typedef struct {
-  const void* in;          /* chunk pass: the tensor; emit pass: unused */
-  void* out;               /* emit pass: int64 result */
-  const uint64_t* keys_in; /* merge pass: runs of length `run` */
+  const void* in;          /* chunk pass: the tensor */
+  void* out;               /* last rank pass: int64 result, else null */
+  const void* keys_in;     /* rank pass: runs of length `run` */
   const uint32_t* idx_in;
-  uint64_t* keys_out;      /* chunk and merge passes */
+  void* keys_out;          /* chunk pass, rank passes before the last */
   uint32_t* idx_out;
   uint32_t outer, reduce, inner;
   uint32_t run, descending, pad;

@@ -9,9 +9,9 @@
 // to fill the chip, the axis is cut into segments: totals per segment, a small scan of the
 // totals, then the segments are scanned starting from what precedes them.
 //
-// argsort (BackendCPU.swift:888-920): one block per (outer, inner) pair sorts (key, index)
-// pairs with a bitonic network in LDS, up to 4096 elements; longer axes are sorted in runs of
-// 4096 that are then merged pairwise (merge path through LDS, 2048 outputs per workgroup). Keys are mapped to unsigned
+// argsort (BackendCPU.swift:888-920): one block per (outer, inner) pair merge-sorts (key, index)
+// pairs in LDS, up to 4096 elements; longer axes are sorted in runs of
+// 4096 that are then merged 16 at a time (every entry counts what goes before it in the other runs). Keys are mapped to unsigned
 // integers that order like the values (-0 counts as +0), inverted for descending order; the
 // source index breaks ties, so the sort is stable, which the reference's `stable` flag
 // asks for and its unstable variant permits.
@@ -215,111 +215,103 @@ template <bool WIDE> struct SortBuf {
   }
 };
 
-// Bitonic sort of N = 2^G * (workgroup size) entries in LDS with 2^G entries per lane held in
-// registers: a lane picks entries that differ only in G chosen index bits, so the G
-// compare-exchange stages whose strides are those bits run without touching LDS. A merge of
-// runs of length k/2 (log2 k stages) therefore costs ceil(log2 k / G) round trips, and all the
-// merges up to k = 2^G together cost one: 21 round trips instead of 78 stages for 4096 entries.
-template <bool WIDE, int G> __device__ __forceinline__ void bitonic_sort_regs(const SortBuf<WIDE>& buf, uint32_t N) {
-  constexpr int E = 1 << G;
+template <bool WIDE> __device__ __forceinline__ bool entry_before(uint64_t ka, uint32_t ia, uint64_t kb, uint32_t ib) {
+  return ka < kb || (WIDE && ka == kb && ia < ib);
+}
+
+// Merge sort of E entries per lane, E * 256 in all, of which the first `count` are wanted: a lane sorts its E
+// entries in registers (bitonic network on constant indices), then runs of E, 2 E, ... are merged
+// pairwise through LDS: a lane finds by bisection where the merge path crosses its first output and
+// merges E entries from there, one LDS read per entry. A level costs at most 11 + E dependent LDS reads
+// and two barriers, whatever the run length; a bitonic network needs log2(run) stages for the same merge
+// (13 runs of 4096 x 8 lines, fp32: 38 -> 28 us). Bound by the latency of those reads, one wave per SIMD.
+template <bool WIDE, int E> __device__ __forceinline__ void merge_sort_lds(const SortBuf<WIDE>& buf, uint32_t count) {
   uint64_t kx[E];
   uint32_t ix[E];
-  const uint32_t t = threadIdx.x;
-  // entries idx0 | (e << L), e = 0 .. E-1
-  auto load = [&](uint32_t idx0, uint32_t L) {
+  const uint32_t first = threadIdx.x * E;
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-      const uint32_t slot = sort_slot(idx0 | ((uint32_t)e << L));
-      kx[e] = buf.keys[slot];
-      if (WIDE) ix[e] = buf.idxs[slot];
-    }
-  };
-  auto store = [&](uint32_t idx0, uint32_t L) {
+  for (int e = 0; e < E; e++) {
+    const uint32_t slot = sort_slot(first + e);
+    kx[e] = buf.keys[slot];
+    if (WIDE) ix[e] = buf.idxs[slot];
+  }
 #pragma unroll
-    for (int e = 0; e < E; e++) {
-      const uint32_t slot = sort_slot(idx0 | ((uint32_t)e << L));
+  for (int k = 2; k <= E; k <<= 1)
+#pragma unroll
+    for (int s = k >> 1; s > 0; s >>= 1)
+#pragma unroll
+      for (int e = 0; e < E; e++) {
+        const int f = e ^ s;
+        if (f < e) continue;
+        const bool e_after_f = entry_before<WIDE>(kx[f], WIDE ? ix[f] : 0, kx[e], WIDE ? ix[e] : 0);
+        const bool swap = e_after_f == ((e & k) == 0);
+        const uint64_t klo = swap ? kx[f] : kx[e], khi = swap ? kx[e] : kx[f];
+        kx[e] = klo;
+        kx[f] = khi;
+        if (WIDE) {
+          const uint32_t ilo = swap ? ix[f] : ix[e], ihi = swap ? ix[e] : ix[f];
+          ix[e] = ilo;
+          ix[f] = ihi;
+        }
+      }
+  for (uint32_t run = E;; run <<= 1) {
+#pragma unroll
+    for (int e = 0; e < E; e++) {   // (every lane has read its inputs of the level before)
+      const uint32_t slot = sort_slot(first + e);
       buf.keys[slot] = kx[e];
       if (WIDE) buf.idxs[slot] = ix[e];
     }
-  };
-  // the g stages with strides 2^(L+g-1) .. 2^L of the merge into runs of length k
-  auto stages = [&](uint32_t idx0, uint32_t L, int g, uint32_t k) {
+    __syncthreads();
+    if (run >= count) return;
+    const uint32_t a0 = first & ~(2 * run - 1), b0 = a0 + run, d = first - a0;
+    uint32_t lo = d > run ? d - run : 0, hi = d < run ? d : run;
+    while (lo < hi) {
+      const uint32_t x = (lo + hi) >> 1, sa = sort_slot(a0 + x), sb = sort_slot(b0 + d - x - 1);
+      if (entry_before<WIDE>(buf.keys[sa], WIDE ? buf.idxs[sa] : 0, buf.keys[sb], WIDE ? buf.idxs[sb] : 0)) lo = x + 1;
+      else hi = x;
+    }
+    uint32_t x = a0 + lo, y = b0 + d - lo;         // next entry of either run
+    const uint32_t x_end = b0, y_end = b0 + run;   // (an entry past its run's end is never taken; its slot is clamped)
+    const uint32_t last = E * HCK_BLOCK - 1;
+    uint32_t sa = sort_slot(x), sb = sort_slot(y < last ? y : last);
+    uint64_t ka = buf.keys[sa], kb = buf.keys[sb];
+    uint32_t ia = WIDE ? buf.idxs[sa] : 0, ib = WIDE ? buf.idxs[sb] : 0;
 #pragma unroll
-    for (int b = G - 1; b >= 0; b--) {
-      if (b < g) {
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-          if (e & (1 << b)) continue;
-          const int f = e | (1 << b);
-          const bool ascending = ((idx0 | ((uint32_t)e << L)) & k) == 0;
-          const bool e_after_f = kx[e] > kx[f] || (WIDE && kx[e] == kx[f] && ix[e] > ix[f]);
-          const bool swap = e_after_f == ascending;
-          const uint64_t klo = swap ? kx[f] : kx[e], khi = swap ? kx[e] : kx[f];
-          kx[e] = klo;
-          kx[f] = khi;
-          if (WIDE) {
-            const uint32_t ilo = swap ? ix[f] : ix[e], ihi = swap ? ix[e] : ix[f];
-            ix[e] = ilo;
-            ix[f] = ihi;
-          }
-        }
+    for (int e = 0; e < E; e++) {
+      const bool take_a = y >= y_end || (x < x_end && entry_before<WIDE>(ka, ia, kb, ib));
+      kx[e] = take_a ? ka : kb;
+      if (WIDE) ix[e] = take_a ? ia : ib;
+      x += take_a ? 1 : 0;
+      y += take_a ? 0 : 1;
+      const uint32_t next = take_a ? x : y, slot = sort_slot(next < last ? next : last);
+      const uint64_t k = buf.keys[slot];
+      ka = take_a ? k : ka;
+      kb = take_a ? kb : k;
+      if (WIDE) {
+        const uint32_t i = buf.idxs[slot];
+        ia = take_a ? i : ia;
+        ib = take_a ? ib : i;
       }
     }
-  };
-  // runs up to length E: E consecutive entries per lane
-  load(t << G, 0);
-#pragma unroll
-  for (int m = 1; m <= G; m++) stages(t << G, 0, m, 1u << m);
-  store(t << G, 0);
-  __syncthreads();
-  for (uint32_t m = G + 1; (1u << m) <= N; m++) {
-    uint32_t left = m;  // stages left in this merge: strides 2^(left-1) .. 1
-    while (left > 0) {
-      const int g = left < (uint32_t)G ? (int)left : G;
-      const uint32_t L = left - g;
-      const uint32_t idx0 = ((t >> L) << (L + G)) | (t & ((1u << L) - 1));
-      load(idx0, L);
-      stages(idx0, L, g, 1u << m);
-      store(idx0, L);
-      __syncthreads();
-      left -= g;
-    }
+    __syncthreads();
   }
 }
 
-// The same network one stage at a time, for fewer entries than two per lane.
-template <bool WIDE> __device__ __forceinline__ void bitonic_sort_small(const SortBuf<WIDE>& buf, uint32_t N) {
-  const uint32_t half = N >> 1, t = threadIdx.x;
-  for (uint32_t k = 2; k <= N; k <<= 1) {
-    for (uint32_t s = k >> 1; s > 0; s >>= 1) {
-      if (t < half) {
-        const uint32_t lo = ((t & ~(s - 1)) << 1) | (t & (s - 1));
-        const uint32_t pa = sort_slot(lo), pb = sort_slot(lo + s);
-        const uint64_t ka = buf.keys[pa], kb = buf.keys[pb];
-        const uint32_t ia = WIDE ? buf.idxs[pa] : 0, ib = WIDE ? buf.idxs[pb] : 0;
-        const bool a_after_b = ka > kb || (WIDE && ka == kb && ia > ib);
-        if (a_after_b == ((lo & k) == 0)) {
-          buf.keys[pa] = kb;
-          buf.keys[pb] = ka;
-          if (WIDE) {
-            buf.idxs[pa] = ib;
-            buf.idxs[pb] = ia;
-          }
-        }
-      }
-      __syncthreads();
-    }
-  }
+// entries per lane that a sort of `count` <= ARGSORT_MAX entries runs with: 1, 2, 4, 8 or 16
+__device__ __forceinline__ uint32_t sort_entries(uint32_t count) {
+  uint32_t e = 1;
+  while (e * HCK_BLOCK < count) e <<= 1;
+  return e;
 }
 
-// N: a power of two, 2 <= N <= ARGSORT_MAX
-template <bool WIDE> __device__ __forceinline__ void bitonic_sort_lds(const SortBuf<WIDE>& buf, uint32_t N) {
+template <bool WIDE> __device__ __forceinline__ void sort_lds(const SortBuf<WIDE>& buf, uint32_t count) {
   static_assert(ARGSORT_MAX == 16 * HCK_BLOCK, "entries per lane below assume 4096 entries and 256 lanes");
-  if (N == 16 * HCK_BLOCK) bitonic_sort_regs<WIDE, 4>(buf, N);
-  else if (N == 8 * HCK_BLOCK) bitonic_sort_regs<WIDE, 3>(buf, N);
-  else if (N == 4 * HCK_BLOCK) bitonic_sort_regs<WIDE, 2>(buf, N);
-  else if (N == 2 * HCK_BLOCK) bitonic_sort_regs<WIDE, 1>(buf, N);
-  else bitonic_sort_small<WIDE>(buf, N);
+  const uint32_t e = sort_entries(count);
+  if (e == 16) merge_sort_lds<WIDE, 16>(buf, count);
+  else if (e == 8) merge_sort_lds<WIDE, 8>(buf, count);
+  else if (e == 4) merge_sort_lds<WIDE, 4>(buf, count);
+  else if (e == 2) merge_sort_lds<WIDE, 2>(buf, count);
+  else merge_sort_lds<WIDE, 1>(buf, count);
 }
 
 // descending order = ascending order of the inverted key
@@ -337,23 +329,23 @@ template <typename T> __device__ __forceinline__ void argsort_impl(const hck_sca
   const size_t base = (size_t)i * p.reduce * p.inner + j;
   const T* in = (const T*)p.in + base;
   int64_t* out = (int64_t*)p.out + base;
-  uint32_t N = 2;
-  while (N < p.reduce) N <<= 1;
+  const uint32_t N = sort_entries(p.reduce) * HCK_BLOCK;
   const uint64_t flip = key_flip<C>(p.reverse);
   for (uint32_t t = threadIdx.x; t < N; t += HCK_BLOCK) {
     if (t < p.reduce) buf.put(t, sort_key((C)to_arith(in[(size_t)t * p.inner])) ^ flip, t);
     else buf.pad(t);
   }
   __syncthreads();
-  bitonic_sort_lds<WIDE>(buf, N);
+  sort_lds<WIDE>(buf, p.reduce);
   for (uint32_t t = threadIdx.x; t < p.reduce; t += HCK_BLOCK) out[(size_t)t * p.inner] = (int64_t)buf.idx(t);
 }
 
 // Long axes, pass 1: block (line, chunk) sorts elements [chunk * ARGSORT_MAX, ...) of its line
-// and stores the sorted (key, index) run.
-template <typename T> __device__ __forceinline__ void argsort_chunks_impl(const hck_sort_args& p) {
+// and stores the sorted run: keys (32 bits, or 64 for int64 tensors) and indices.
+template <typename T, typename K> __device__ __forceinline__ void argsort_chunks_impl(const hck_sort_args& p) {
   typedef typename Arith<T>::type C;
   constexpr bool WIDE = sizeof(C) == 8;
+  static_assert(sizeof(K) == sizeof(C), "keys have the size of the arithmetic type");
   __shared__ uint64_t keys[SORT_SLOTS];
   __shared__ uint32_t idxs[WIDE ? SORT_SLOTS : 1];
   const SortBuf<WIDE> buf{keys, idxs};
@@ -369,116 +361,85 @@ template <typename T> __device__ __forceinline__ void argsort_chunks_impl(const 
     else buf.pad(t);
   }
   __syncthreads();
-  bitonic_sort_lds<WIDE>(buf, ARGSORT_MAX);
+  sort_lds<WIDE>(buf, count);
   const size_t dst = (size_t)line * p.reduce + first;
   for (uint32_t t = threadIdx.x; t < count; t += HCK_BLOCK) {
-    p.keys_out[dst + t] = buf.key(t);
+    ((K*)p.keys_out)[dst + t] = (K)buf.key(t);
     p.idx_out[dst + t] = buf.idx(t);
   }
 }
 
-// Long axes, pass 2..: runs of length `run` are merged pairwise. A workgroup produces
-// MERGE_TILE consecutive outputs of one pair of runs: two of its waves find where the merge
-// path crosses the tile's first and last output (a 64-way search: every lane probes one
-// candidate per round, so a run of any length needs at most a few dependent loads), the
-// workgroup copies the two input windows into LDS, and every lane bisects to its own first
-// output there and merges MERGE_SEG entries. (key, index) pairs are all distinct, so the
-// result does not depend on how ties would be broken.
-constexpr uint32_t MERGE_SEG = 8;
-constexpr uint32_t MERGE_TILE = MERGE_SEG * HCK_BLOCK;
+// Long axes, pass 2..: ARGSORT_WAYS neighbouring runs of length `run` (a power of two times 256) become one. The
+// place of an entry is its place in its own run plus, for every other run of the group, the number of
+// entries that go before it, found by bisection. The runs lie in index order, so ties go by the run: equal
+// keys of an earlier run go before. A lane owns an entry and bisects in 8 runs at a time, 8 independent loads
+// per step; neighbouring lanes own neighbouring keys and mostly read the same lines. The pass that
+// completes the line writes the index straight to its place in the result.
+// One such pass does what four passes of pairwise merging and one that wrote the result did, each of them a launch
+// that moved every entry through memory: [8, 50257] fp32 54 -> 36 us. Bound by the address path: lanes of a load
+// go to different lines, four lanes a cycle.
+constexpr uint32_t ARGSORT_WAYS = 16;
 
-__device__ __forceinline__ bool pair_before(uint64_t ka, uint32_t ia, uint64_t kb, uint32_t ib) {
-  return ka < kb || (ka == kb && ia < ib);
-}
-
-HC_KERNEL void hc_argsort_merge(hck_sort_args p) {
-  __shared__ uint64_t sk[MERGE_TILE];
-  __shared__ uint32_t si[MERGE_TILE];
-  __shared__ uint32_t split[2];
-  const uint32_t tiles = (p.reduce + MERGE_TILE - 1) / MERGE_TILE;
+template <typename K> __device__ __forceinline__ void argsort_rank_impl(const hck_sort_args& p) {
+  const uint32_t tiles = (p.reduce + HCK_BLOCK - 1) / HCK_BLOCK;
   const uint32_t line = blockIdx.x / tiles, tile = blockIdx.x - line * tiles;
-  const size_t base = (size_t)line * p.reduce;
-  const uint32_t pos = tile * MERGE_TILE;                // first output position in the line
-  const uint32_t pair = pos / (2 * p.run) * (2 * p.run); // start of this pair of runs
-  const uint32_t a0 = pair, a1 = min(pair + p.run, p.reduce);
-  const uint32_t b0 = a1, b1 = min(pair + 2 * p.run, p.reduce);
-  const uint32_t na = a1 - a0, nb = b1 - b0;
-  const uint32_t d0 = pos - pair, d1 = min(d0 + MERGE_TILE, na + nb);
-  const uint64_t* ka = p.keys_in + base + a0;
-  const uint64_t* kb = p.keys_in + base + b0;
-  const uint32_t* ia = p.idx_in + base + a0;
-  const uint32_t* ib = p.idx_in + base + b0;
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  if (wave < 2) {
-    // smallest x (entries taken from run A before diagonal d) with A[x] not before B[d - x - 1]
-    const uint32_t d = wave == 0 ? d0 : d1;
-    uint32_t lo = d > nb ? d - nb : 0, hi = d < na ? d : na;
-    while (lo < hi) {
-      const uint32_t step = (hi - lo + 63) / 64;
-      const uint32_t x = lo + lane * step;
-      const bool before = x < hi && pair_before(ka[x], ia[x], kb[d - x - 1], ib[d - x - 1]);
-      const uint32_t cnt = (uint32_t)__popcll(__ballot(before));  // the candidates that hold form a prefix
-      if (cnt == 0) {
-        hi = lo;
-      } else {
-        const uint32_t next = lo + cnt * step;
-        lo = lo + (cnt - 1) * step + 1;
-        hi = next < hi ? next : hi;
+  const K* keys = (const K*)p.keys_in + (size_t)line * p.reduce;
+  const uint32_t pos = tile * HCK_BLOCK + threadIdx.x;
+  const uint32_t own_start = tile * HCK_BLOCK / p.run * p.run;  // a tile lies inside one run
+  const uint32_t group = (uint32_t)((uint64_t)own_start / ((uint64_t)ARGSORT_WAYS * p.run) * ARGSORT_WAYS * p.run);
+  const bool valid = pos < p.reduce;
+  const K key = valid ? keys[pos] : (K)0;
+  uint32_t rank = pos - own_start;
+  for (uint32_t w0 = 0; w0 < ARGSORT_WAYS; w0 += 8) {
+    if ((uint64_t)group + (uint64_t)w0 * p.run >= p.reduce) break;
+    uint32_t start[8], len[8], before[8];
+    bool ties[8];
+#pragma unroll
+    for (int w = 0; w < 8; w++) {
+      const uint64_t s = (uint64_t)group + (uint64_t)(w0 + w) * p.run;
+      const bool other = s < p.reduce && s != own_start;
+      start[w] = other ? (uint32_t)s : 0;
+      len[w] = !other ? 0 : p.reduce - (uint32_t)s < p.run ? p.reduce - (uint32_t)s : p.run;
+      ties[w] = s < own_start;
+      before[w] = 0;
+    }
+    for (uint32_t step = p.run; step > 0; step >>= 1) {
+      K k[8];
+#pragma unroll
+      for (int w = 0; w < 8; w++) {
+        const uint32_t next = before[w] + step;
+        k[w] = keys[start[w] + (next <= len[w] ? next - 1 : 0)];
+      }
+      // (all eight loads are out before the first is waited for: the compiler would make eight
+      // branches of them, each with a load and a wait)
+      asm volatile("" : "+v"(k[0]), "+v"(k[1]), "+v"(k[2]), "+v"(k[3]), "+v"(k[4]), "+v"(k[5]), "+v"(k[6]), "+v"(k[7]));
+#pragma unroll
+      for (int w = 0; w < 8; w++) {
+        const uint32_t next = before[w] + step;
+        const bool goes_before = (k[w] < key) | (ties[w] & (k[w] == key));
+        before[w] = (next <= len[w]) & goes_before ? next : before[w];
       }
     }
-    if (lane == 0) split[wave] = lo;
+#pragma unroll
+    for (int w = 0; w < 8; w++) rank += before[w];
   }
-  __syncthreads();
-  const uint32_t x0 = split[0], x1 = split[1], y0 = d0 - x0, y1 = d1 - x1;
-  const uint32_t ca = x1 - x0, cb = y1 - y0;  // ca + cb = d1 - d0 <= MERGE_TILE
-  for (uint32_t t = threadIdx.x; t < ca + cb; t += HCK_BLOCK) {
-    sk[t] = t < ca ? ka[x0 + t] : kb[y0 + t - ca];
-    si[t] = t < ca ? ia[x0 + t] : ib[y0 + t - ca];
-  }
-  __syncthreads();
-  const uint32_t d = threadIdx.x * MERGE_SEG;  // diagonal inside the tile
-  if (d >= ca + cb) return;
-  const uint64_t* la = sk;
-  const uint64_t* lb = sk + ca;
-  const uint32_t* ja = si;
-  const uint32_t* jb = si + ca;
-  uint32_t lo = d > cb ? d - cb : 0, hi = d < ca ? d : ca;
-  while (lo < hi) {
-    const uint32_t x = (lo + hi) / 2, y = d - x - 1;
-    if (pair_before(la[x], ja[x], lb[y], jb[y])) lo = x + 1;
-    else hi = x;
-  }
-  uint32_t x = lo, y = d - lo;
-  const uint32_t n = min(MERGE_SEG, ca + cb - d);
-  const size_t o0 = base + pair + d0 + d;
-  for (uint32_t o = 0; o < n; o++) {
-    bool take_a;
-    if (x >= ca) take_a = false;
-    else if (y >= cb) take_a = true;
-    else take_a = pair_before(la[x], ja[x], lb[y], jb[y]);
-    p.keys_out[o0 + o] = take_a ? la[x] : lb[y];
-    p.idx_out[o0 + o] = take_a ? ja[x] : jb[y];
-    if (take_a) x++;
-    else y++;
+  if (!valid) return;
+  const uint32_t place = group + rank, idx = p.idx_in[(size_t)line * p.reduce + pos];
+  if (p.out != nullptr) {
+    const uint32_t i = line / p.inner, j = line - i * p.inner;
+    ((int64_t*)p.out)[((size_t)i * p.reduce + place) * p.inner + j] = (int64_t)idx;
+  } else {
+    ((K*)p.keys_out)[(size_t)line * p.reduce + place] = key;
+    p.idx_out[(size_t)line * p.reduce + place] = idx;
   }
 }
 
-// Long axes, last pass: sorted indices to the int64 result, back in the tensor's layout.
-HC_KERNEL void hc_argsort_emit(hck_sort_args p) {
-  const uint64_t gid = (uint64_t)blockIdx.x * HCK_BLOCK + threadIdx.x;
-  const uint64_t total = (uint64_t)p.outer * p.inner * p.reduce;
-  if (gid >= total) return;
-  // gid walks the result in memory order: (i, t, j)
-  const uint32_t j = (uint32_t)(gid % p.inner);
-  const uint64_t r = gid / p.inner;
-  const uint32_t t = (uint32_t)(r % p.reduce), i = (uint32_t)(r / p.reduce);
-  const size_t line = (size_t)i * p.inner + j;
-  ((int64_t*)p.out)[gid] = (int64_t)p.idx_in[line * p.reduce + t];
-}
+HC_KERNEL void hc_argsort_rank_k32(hck_sort_args p) { argsort_rank_impl<uint32_t>(p); }
+HC_KERNEL void hc_argsort_rank_k64(hck_sort_args p) { argsort_rank_impl<uint64_t>(p); }
 
-HC_KERNEL void hc_argsort_chunks_f32(hck_sort_args p) { argsort_chunks_impl<float>(p); }
-HC_KERNEL void hc_argsort_chunks_f16(hck_sort_args p) { argsort_chunks_impl<half_t>(p); }
-HC_KERNEL void hc_argsort_chunks_i64(hck_sort_args p) { argsort_chunks_impl<int64_t>(p); }
+HC_KERNEL void hc_argsort_chunks_f32(hck_sort_args p) { argsort_chunks_impl<float, uint32_t>(p); }
+HC_KERNEL void hc_argsort_chunks_f16(hck_sort_args p) { argsort_chunks_impl<half_t, uint32_t>(p); }
+HC_KERNEL void hc_argsort_chunks_i64(hck_sort_args p) { argsort_chunks_impl<int64_t, uint64_t>(p); }
 HC_KERNEL void hc_argsort_f32(hck_scan_args p) { argsort_impl<float>(p); }
 HC_KERNEL void hc_argsort_f16(hck_scan_args p) { argsort_impl<half_t>(p); }
 HC_KERNEL void hc_argsort_i64(hck_scan_args p) { argsort_impl<int64_t>(p); }
