@@ -390,6 +390,7 @@ template <int OP, bool HALF> __device__ __forceinline__ float elemwise_apply(flo
     if (OP == E_EXP) return exp_hw(f);
     if (OP == E_SIGMOID) return sigmoid_hw(f);
     if (OP == E_GELU_APPROX) return gelu_approx<true>(f);
+    if (OP == E_GELU_APPROX_GRAD) return gelu_approx_grad<true>(f);
   }
   switch (OP) {
     case E_SIN: return sinf(f);
@@ -413,12 +414,7 @@ template <int OP, bool HALF> __device__ __forceinline__ float elemwise_apply(flo
     case E_ABS: return f < 0.0f ? -f : f;
     case E_ABS_GRAD: return f < 0.0f ? -1.0f : 1.0f;
     case E_GELU_APPROX: return gelu_approx<false>(f);
-    case E_GELU_APPROX_GRAD: {
-      float tanh_term = tanhf(0.035677408145115f * powf(f, 3.0f) + 0.797884561f * f);
-      return 0.5f * f * (1.0f - powf(tanh_term, 2.0f)) *
-                 (0.107032224435345f * powf(f, 2.0f) + 0.797884561f) +
-             0.5f * tanh_term + 0.5f;
-    }
+    case E_GELU_APPROX_GRAD: return gelu_approx_grad<false>(f);
     case E_GELU_EXACT: return f * 0.5f * (1.0f + fast_erf(f * 0.7071067811865475f));
     case E_GELU_EXACT_GRAD: {
       const float c = 0.7071067811865475f;

@@ -3,7 +3,7 @@ path's range, each against the CPU oracle (or a 64-bit computation where the ora
 import numpy as np
 import pytest
 
-from honeycrisp_amd.descriptors import DType
+from honeycrisp_amd.descriptors import DType, ElemwiseOp
 from honeycrisp_amd.tensor import Tensor
 from test_hip_parity import check_exact, rand
 
@@ -28,3 +28,24 @@ def test_argsort_at_the_ends_of_runs(hip_backend, oracle_backend, dtype, shape):
         f = rand(rng, shape, dtype)
         f[0, :2] = [np.inf, -np.inf]
         check_exact(hip_backend, oracle_backend, lambda: Tensor(data=f).argsort(1))
+
+
+@pytest.mark.parametrize("dtype", [F32, F16], ids=["f32", "f16"])
+def test_gelu_gradient_over_its_range(hip_backend, dtype):
+    """The tails, zero, and values whose cube and square leave the range of the type."""
+    x = np.concatenate([np.linspace(-12, 12, 100003), [0.0, -0.0, 300.0, -300.0, 60000.0, -60000.0]]).astype(dtype.numpy)
+    u = 0.797884561 * x.astype(np.float64) + 0.035677408145115 * x.astype(np.float64) ** 3
+    up, down = 1 / (1 + np.exp(np.minimum(-2 * u, 700))), 1 / (1 + np.exp(np.minimum(2 * u, 700)))
+    want = 2 * x.astype(np.float64) * up * down * (0.797884561 + 0.107032224435345 * x.astype(np.float64) ** 2) + up
+    with hip_backend.use():
+        xt = Tensor(data=x)
+        d = hip_backend.elemwise(xt.data, ElemwiseOp.geluApproxGrad, None, x.size, dtype)
+        got = Tensor(dataHandle=d, shape=[x.size], dtype=dtype).numpy().astype(np.float64)
+    # fp16: one rounding of the result (2^-11 relative, 2^-25 among subnormals); fp32: u of size |u| rounded to 2^-24 moves
+    # the result by |u| * 2^-24 of x^2, and 1 - tanh^2 loses what is below 2^-24
+    bound = np.abs(want) * 2.0 ** -10.9 + 2.0 ** -25 if dtype == F16 else np.abs(want) * 2.0 ** -20 + 2.0 ** -20
+    assert (np.abs(got - want) <= bound).all()
+    y = np.array([np.nan, np.inf, -np.inf], dtype=dtype.numpy)
+    with hip_backend.use():
+        d = hip_backend.elemwise(Tensor(data=y).data, ElemwiseOp.geluApproxGrad, None, 3, dtype)
+        assert np.isnan(Tensor(dataHandle=d, shape=[3], dtype=dtype).numpy()).all()
