@@ -431,6 +431,10 @@ __device__ __forceinline__ void stream_row_out(const T* row, T* out, uint32_t n,
 // it fits, else passes 2 and 3 re-read it (L2).
 // NaNs are skipped by the strict compare here and on the CPU alike; any NaN in the row then
 // turns the exp-sum, and with it the whole row, into NaN on both.
+// A block holds rows of up to 32 KiB (8 x 16 bytes per lane): passes over a row that is longer than its team's
+// registers read it again from L2 and bound the kernel there.
+template <typename T, int LANES> using SoftmaxRegs = RowRegs<T, LANES, LANES == 256 ? 8 : 4>;
+
 template <typename T, int LANES> __device__ __forceinline__ void log_softmax_rows_impl(const hck_reduce_args& p) {
   __shared__ float lds[HCK_BLOCK / 64];
   const uint32_t lane = Team<LANES>::lane(), row = Team<LANES>::row();
@@ -438,8 +442,8 @@ template <typename T, int LANES> __device__ __forceinline__ void log_softmax_row
   const uint32_t n = p.reduce;
   const T* in = (const T*)p.in + (size_t)row * n;
   T* out = (T*)p.out + (size_t)row * n;
-  if (RowRegs<T, LANES>::fits(n)) {
-    RowRegs<T, LANES> r;
+  if (SoftmaxRegs<T, LANES>::fits(n)) {
+    SoftmaxRegs<T, LANES> r;
     r.load(in, n, lane);
     float m = -INFINITY;
     r.each(n, lane, [&](float x) { if (x > m) m = x; });
@@ -586,7 +590,9 @@ HC_KERNEL void hc_softmax_chain_rows8_f32(hck_softmax_chain_args p) { softmax_ch
 HC_KERNEL void hc_softmax_chain_rows_f16(hck_softmax_chain_args p) { softmax_chain_rows_impl<half_t, 64>(p); }
 HC_KERNEL void hc_softmax_chain_rows8_f16(hck_softmax_chain_args p) { softmax_chain_rows_impl<half_t, 8>(p); }
 
-// logSoftmaxGrad (BackendCPU.swift:1040-1085): g - sum(g) * expf(x - (logf(sum exp(x - max)) + max)).
+// logSoftmaxGrad (BackendCPU.swift:1040-1085): g - sum(g) * softmax(x). The exponential of an element is computed once,
+// relative to the maximum, and scaled by sum(g) / sum(exp) at the end (a second exponential of x - logf(sum) - max costs
+// as much again and loses the digits of a long logarithm). RowRegs keeps them between the passes.
 template <typename T, int LANES>
 __device__ __forceinline__ void log_softmax_grad_rows_impl(const hck_reduce_args& p) {
   __shared__ float lds[HCK_BLOCK / 64];
@@ -596,8 +602,8 @@ __device__ __forceinline__ void log_softmax_grad_rows_impl(const hck_reduce_args
   const T* in = (const T*)p.in + (size_t)row * n;
   const T* grad = (const T*)p.in2 + (size_t)row * n;
   T* out = (T*)p.out + (size_t)row * n;
-  if (RowRegs<T, LANES>::fits(n)) {
-    RowRegs<T, LANES> r, g;
+  if (SoftmaxRegs<T, LANES>::fits(n)) {
+    SoftmaxRegs<T, LANES> r, g;
     r.load(in, n, lane);
     g.load(grad, n, lane);
     float m = -INFINITY, gs = 0.0f;
@@ -606,10 +612,17 @@ __device__ __forceinline__ void log_softmax_grad_rows_impl(const hck_reduce_args
     m = Team<LANES>::reduce(m, MaxOp(), lds);
     gs = Team<LANES>::reduce(gs, SumOp(), lds);
     float s = 0.0f;
-    r.each(n, lane, [&](float x) { s += expf(x - m); });
-    s = Team<LANES>::reduce(s, SumOp(), lds);
-    const float log_sum = logf(s) + m;
-    g.store2(out, n, lane, r, [&](float gv, float x) { return gv - gs * expf(x - log_sum); });
+    if constexpr (sizeof(T) == 4) {
+      r.update(n, lane, [&](float x) { const float e = expf(x - m); s += e; return e; });
+      s = Team<LANES>::reduce(s, SumOp(), lds);
+      const float scale = gs / s;
+      g.store2(out, n, lane, r, [&](float gv, float e) { return gv - scale * e; });
+    } else {
+      r.each(n, lane, [&](float x) { s += expf(x - m); });
+      s = Team<LANES>::reduce(s, SumOp(), lds);
+      const float scale = gs / s;
+      g.store2(out, n, lane, r, [&](float gv, float x) { return gv - scale * expf(x - m); });
+    }
     return;
   }
   float m = -INFINITY, gs = 0.0f;
@@ -620,9 +633,9 @@ __device__ __forceinline__ void log_softmax_grad_rows_impl(const hck_reduce_args
   float s = 0.0f;
   stream_row<T, LANES>(in, n, lane, [&](float x, uint32_t) { s += expf(x - m); });
   s = Team<LANES>::reduce(s, SumOp(), lds);
-  const float log_sum = logf(s) + m;
+  const float scale = gs / s;
   stream_row_out<T, LANES>(grad, out, n, lane,
-                           [&](float gv, uint32_t k) { return gv - gs * expf((float)in[k] - log_sum); });
+                           [&](float gv, uint32_t k) { return gv - scale * expf((float)in[k] - m); });
 }
 
 HC_KERNEL void hc_log_softmax_grad_rows_f32(hck_reduce_args p) { log_softmax_grad_rows_impl<float, 64>(p); }

@@ -81,6 +81,24 @@ template <typename T, int LANES, int NCHUNKS = 4> struct RowRegs {
         for (int i = 0; i < VEC; i++) f((float)v[c][i]);
       }
   }
+  // f(x, y) for every element and the one of `other` in the same place
+  template <typename F> __device__ __forceinline__ void each2(uint32_t n, uint32_t lane, const RowRegs& other, F f) const {
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++)
+      if ((lane + LANES * c) * VEC < n) {
+#pragma unroll
+        for (int i = 0; i < VEC; i++) f((float)v[c][i], (float)other.v[c][i]);
+      }
+  }
+  // x = f(x)
+  template <typename F> __device__ __forceinline__ void update(uint32_t n, uint32_t lane, F f) {
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++)
+      if ((lane + LANES * c) * VEC < n) {
+#pragma unroll
+        for (int i = 0; i < VEC; i++) v[c][i] = f((float)v[c][i]);
+      }
+  }
   template <typename F> __device__ __forceinline__ void store(T* row, uint32_t n, uint32_t lane, F f) const {
 #pragma unroll
     for (int c = 0; c < CHUNKS; c++) {
