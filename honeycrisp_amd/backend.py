@@ -710,6 +710,18 @@ class HIPBackend(Backend):
                                          s.innerCount, int(bool(s.indicesAreUnique))))
         return out
 
+    def normalizeGrad(self, input, outGrad, dims: ReduceDims, eps, dtype: DType) -> HIPData:
+        """One kernel for rows (innerCount == 1); the base-class composition otherwise, and for few long rows,
+        where its launches spread a row over the whole device."""
+        if dims.innerCount != 1 or not dtype.isFloat or (dims.outerCount < 32 and dims.reduceCount >= 32768):
+            return super().normalizeGrad(input, outGrad, dims, eps, dtype)
+        out = self.allocate(dims.inCount * dtype.byteSize)
+        ad, gd = self._dev(input), self._dev(outGrad)
+        self._check(self._lib.hc_normalize_grad(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(gd.ptr),
+                                                c_void_p(out.ptr), dims.outerCount, dims.reduceCount,
+                                                c_float(float(np.float32(eps)))))
+        return out
+
     def logSoftmaxGrad(self, a, outGrad, dims: ReduceDims, dtype: DType) -> HIPData:
         out = self.allocate(dims.inCount * dtype.byteSize)
         ad, gd = self._dev(a), self._dev(outGrad)

@@ -2282,6 +2282,33 @@ extern "C" int hc_log_softmax_grad(hc_ctx* ctx, int dtype, const void* in, const
 }
 
 
+extern "C" int hc_normalize_grad(hc_ctx* ctx, int dtype, const void* in, const void* out_grad, void* out, int64_t outer,
+                                 int64_t reduce, float eps) {
+  OpNote note({in, out_grad}, {out});
+  REQUIRE(ctx, "hc_normalize_grad: null context");
+  if (dtype != HC_F32 && dtype != HC_F16)
+    return fail(HC_ERR_UNSUPPORTED, "hc_normalize_grad: dtype %d is not a float type", dtype);
+  HC_TRY(check_dims("hc_normalize_grad", outer, reduce, 1));
+  if (outer * reduce == 0) return HC_OK;
+  REQUIRE(in && out_grad && out, "hc_normalize_grad: null pointer");
+  REQUIRE(aligned16(in) && aligned16(out_grad) && aligned16(out), "hc_normalize_grad: buffers must be 16-byte aligned");
+  const size_t el_size = dtype_size(dtype);
+  hck_reduce_args k;
+  memset(&k, 0, sizeof(k));
+  k.in = in;
+  k.in2 = out_grad;
+  k.out = out;
+  k.outer = (uint32_t)outer;
+  k.reduce = (uint32_t)reduce;
+  k.inner = 1;
+  k.eps = eps;
+  // 8 lanes per row for short rows, a wave per row while the row fits its registers (4 x 16 bytes per lane), else a block
+  const uint32_t lanes = (uint64_t)reduce * el_size <= 512 ? 8 : (uint64_t)reduce * el_size <= 64 * 16 * 4 ? 64 : 256;
+  char name[64];
+  snprintf(name, sizeof(name), "hc_normalize_grad_rows%s_%s", lanes == 8 ? "8" : lanes == 64 ? "" : "256", dtype_name(dtype));
+  return launch(ctx, name, ceil_div((uint64_t)outer, HCK_BLOCK / lanes), 1, &k, sizeof(k));
+}
+
 extern "C" int hc_normalize(hc_ctx* ctx, int dtype, const void* in, void* out, int64_t outer,
                             int64_t reduce, int64_t inner, float eps) {
   REQUIRE(ctx, "hc_normalize: null context");

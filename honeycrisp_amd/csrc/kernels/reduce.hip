@@ -701,6 +701,73 @@ HC_KERNEL void hc_normalize_rows8_f16(hck_reduce_args p) { normalize_rows_impl<h
 HC_KERNEL void hc_normalize_rows256_f32(hck_reduce_args p) { normalize_rows_impl<float, 256>(p); }
 HC_KERNEL void hc_normalize_rows256_f16(hck_reduce_args p) { normalize_rows_impl<half_t, 256>(p); }
 
+// normalizeGrad for inner == 1, fused: the base-class composition (Backend.swift:332-455)
+//   c = x - mean(x); n1 = (var + eps)^-0.5; n3 = (var + eps)^-1.5 / n; cov = sum(c * g);
+//   out = (g - mean(g)) * n1 - c * cov * n3
+// with every intermediate rounded to the tensor dtype where the composition stores it; what differs is the order of the
+// sums. Bound by its bytes (x and g read once, the result written) where the composition moves each of them
+// five times in 19 launches ([2048, 512] fp32: 62 us and 19 launches -> 6 us).
+template <typename T, int LANES> __device__ __forceinline__ void normalize_grad_rows_impl(const hck_reduce_args& p) {
+  __shared__ float lds[HCK_BLOCK / 64];
+  const uint32_t lane = Team<LANES>::lane(), row = Team<LANES>::row();
+  if (row >= p.outer) return;
+  const uint32_t n = p.reduce;
+  const T* in = (const T*)p.in + (size_t)row * n;
+  const T* grad = (const T*)p.in2 + (size_t)row * n;
+  T* out = (T*)p.out + (size_t)row * n;
+  const float inv_n = 1.0f / (float)n;
+  auto total = [&](float v) { return round_through<T>(Team<LANES>::reduce(v, SumOp(), lds)); };
+  float s = 0.0f, gs = 0.0f, sq = 0.0f, cov = 0.0f, mean = 0.0f;
+  auto centered = [&](float x) { return round_through<T>(x - mean); };
+  auto squares = [&](float x) {
+    const float c = centered(x);
+    sq += round_through<T>(pow_like(c, 2.0f));
+  };
+  auto products = [&](float x, float g) { cov += round_through<T>(centered(x) * g); };
+  float grad_mean, normer, normer3;
+  auto finish = [&]() {
+    sq = total(sq);
+    cov = total(cov);
+    grad_mean = round_through<T>(total(gs) * inv_n);
+    const float shifted = round_through<T>(round_through<T>(sq * inv_n) + p.eps);
+    normer = round_through<T>(pow_like(shifted, -0.5f));
+    normer3 = round_through<T>(inv_n * pow_like(shifted, -1.5f));
+  };
+  auto result = [&](float x, float g) {
+    const float direct = round_through<T>(round_through<T>(g - grad_mean) * normer);
+    return direct - round_through<T>(round_through<T>(centered(x) * cov) * normer3);
+  };
+  if (RowRegs<T, LANES>::fits(n)) {
+    RowRegs<T, LANES> r, g;
+    r.load(in, n, lane);
+    g.load(grad, n, lane);
+    r.each(n, lane, [&](float x) { s += x; });
+    g.each(n, lane, [&](float x) { gs += x; });
+    mean = round_through<T>(total(s) * inv_n);
+    r.each(n, lane, squares);
+    r.each2(n, lane, g, products);
+    finish();
+    r.store2(out, n, lane, g, result);
+    return;
+  }
+  stream_row<T, LANES>(in, n, lane, [&](float x, uint32_t) { s += x; });
+  mean = round_through<T>(total(s) * inv_n);
+  stream_row<T, LANES>(grad, n, lane, [&](float g, uint32_t k) {
+    const float x = (float)in[k];
+    gs += g;
+    squares(x);
+    products(x, g);
+  });
+  finish();
+  stream_row_out<T, LANES>(grad, out, n, lane, [&](float g, uint32_t k) { return result((float)in[k], g); });
+}
+HC_KERNEL void hc_normalize_grad_rows_f32(hck_reduce_args p) { normalize_grad_rows_impl<float, 64>(p); }
+HC_KERNEL void hc_normalize_grad_rows8_f32(hck_reduce_args p) { normalize_grad_rows_impl<float, 8>(p); }
+HC_KERNEL void hc_normalize_grad_rows256_f32(hck_reduce_args p) { normalize_grad_rows_impl<float, 256>(p); }
+HC_KERNEL void hc_normalize_grad_rows_f16(hck_reduce_args p) { normalize_grad_rows_impl<half_t, 64>(p); }
+HC_KERNEL void hc_normalize_grad_rows8_f16(hck_reduce_args p) { normalize_grad_rows_impl<half_t, 8>(p); }
+HC_KERNEL void hc_normalize_grad_rows256_f16(hck_reduce_args p) { normalize_grad_rows_impl<half_t, 256>(p); }
+
 // The chain [cast to fp32] -> normalize (fp32, a wave per row) [-> x * (gain [+ c]) + bias] [-> cast]
 // (a LayerNorm as Trainable.swift:787-829 issues it) in one pass. Elements are spread over the
 // lanes as the fp32 normalize kernel spreads them (lane l: the 4-element groups l, l + 64, ...) and

@@ -251,8 +251,8 @@ int hc_launch(hc_ctx* ctx, hc_function* fn, const uint32_t grid[3], const uint32
  * pointer into the middle of a block (a view) must at least be aligned to its element size, and
  *  - the contiguous maps and row kernels require 16-byte aligned buffers and return
  *    HC_ERR_INVALID otherwise: hc_binary_op_scalar, hc_compare_scalar, hc_cast, hc_pow,
- *    hc_elemwise, hc_fill, hc_adamw, hc_log_softmax, hc_log_softmax_grad, hc_normalize, hc_reduce
- *    with inner == 1, and hc_scatter (whose output is cleared with hc_fill);
+ *    hc_elemwise, hc_fill, hc_adamw, hc_log_softmax, hc_log_softmax_grad, hc_normalize,
+ *    hc_normalize_grad, hc_reduce with inner == 1, and hc_scatter (whose output is cleared with hc_fill);
  *  - everything else takes any element-aligned pointer and only loses its 16-byte vector
  *    accesses: the broadcasting ops (hc_broadcast, hc_binary_op, hc_bitwise_op, hc_compare,
  *    hc_mul_add, hc_add_mul, hc_when, hc_clamp), hc_reduce with inner > 1, hc_cumulative,
@@ -348,6 +348,11 @@ int hc_log_softmax(hc_ctx* ctx, int dtype, const void* in, void* out, int64_t ou
  * (var + eps)^-0.5, every intermediate rounded to `dtype`). */
 int hc_normalize(hc_ctx* ctx, int dtype, const void* in, void* out, int64_t outer,
                  int64_t reduce, int64_t inner, float eps);
+
+/* Backend.normalizeGrad (Backend.swift:332-455) over rows (inner == 1): the gradient of hc_normalize for
+ * its input and the gradient of its result, every intermediate rounded to `dtype`. */
+int hc_normalize_grad(hc_ctx* ctx, int dtype, const void* in, const void* out_grad, void* out, int64_t outer,
+                      int64_t reduce, float eps);
 
 /* Backend.gather (Backend.swift:609-616; CPU BackendCPU.swift:1108-1147) with
  * ScatterGatherIndices flattened (ScatterGather.swift:21-45):

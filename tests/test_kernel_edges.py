@@ -31,6 +31,39 @@ def test_argsort_at_the_ends_of_runs(hip_backend, oracle_backend, dtype, shape):
 
 
 @pytest.mark.parametrize("dtype", [F32, F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("shape", [(3, 1), (5, 7), (70, 128), (3, 256), (3, 260), (2, 1024), (2, 1028), (3, 2048), (2, 2056),
+                                   (2, 8192), (2, 8196), (2, 16384), (2, 16392), (1, 32771)], ids=str)
+def test_gradients_of_rows_at_the_ends_of_the_registers(hip_backend, dtype, shape):
+    """logSoftmax, its gradient and normalizeGrad: 1, 8 and 64 lanes and a block per row, held in registers or streamed."""
+    rng = np.random.default_rng(shape[1])
+    x, g = rand(rng, shape, dtype), rand(rng, shape, dtype)
+    x64, g64 = x.astype(np.float64), g.astype(np.float64)
+    n = shape[1]
+    logp = x64 - np.log(np.exp(x64).sum(1, keepdims=True))
+    c = x64 - x64.mean(1, keepdims=True)
+    shifted = (c * c).mean(1, keepdims=True) + 1e-3
+    want = {"logSoftmax": logp, "logSoftmaxGrad": g64 - g64.sum(1, keepdims=True) * np.exp(logp),
+            "normalizeGrad": (g64 - g64.mean(1, keepdims=True)) / np.sqrt(shifted)
+            - c * (c * g64).sum(1, keepdims=True) / shifted ** 1.5 / n}
+    with hip_backend.use():
+        xt, gt = Tensor(data=x), Tensor(data=g)
+        dims = xt.reduceDims(1)
+        got = {"logSoftmax": hip_backend.logSoftmax(xt.data, dims, dtype),
+               "logSoftmaxGrad": hip_backend.logSoftmaxGrad(xt.data, gt.data, dims, dtype),
+               "normalizeGrad": hip_backend.normalizeGrad(xt.data, gt.data, dims, 1e-3, dtype)}
+        got = {name: Tensor(dataHandle=d, shape=list(shape), dtype=dtype).numpy() for name, d in got.items()}
+    # a handful of roundings of values no larger than the largest input or result (sums of n terms: sqrt(n) / 16 more);
+    # normalizeGrad divides by a deviation of sqrt(1e-3) where a row has one element, and rounds its sums to the type
+    eps = 2.0 ** -11 if dtype == F16 else 2.0 ** -24
+    for name, value in want.items():
+        if name == "normalizeGrad":
+            size = max(np.abs(value).max(), np.abs(g64).max(), (np.abs(g64) / np.sqrt(shifted)).max())
+        else:
+            size = max(np.abs(value).max(), np.abs(x64).max(), np.abs(g64).max(), np.abs(g64.sum(1)).max() if dtype == F32 else 0)
+        assert np.abs(got[name] - value).max() <= 16 * eps * size * max(1, np.sqrt(n) / 16), name
+
+
+@pytest.mark.parametrize("dtype", [F32, F16], ids=["f32", "f16"])
 def test_gelu_gradient_over_its_range(hip_backend, dtype):
     """The tails, zero, and values whose cube and square leave the range of the type."""
     x = np.concatenate([np.linspace(-12, 12, 100003), [0.0, -0.0, 300.0, -300.0, 60000.0, -60000.0]]).astype(dtype.numpy)
