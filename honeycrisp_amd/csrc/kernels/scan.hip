@@ -340,6 +340,21 @@ template <typename T> __device__ __forceinline__ void argsort_impl(const hck_sca
   for (uint32_t t = threadIdx.x; t < p.reduce; t += HCK_BLOCK) out[(size_t)t * p.inner] = (int64_t)buf.idx(t);
 }
 
+// Which line, and which of its `parts` pieces, a block takes. Blocks go to the eight XCDs round robin in launch order, each
+// with an L2 of its own: the blocks of a line are given to blocks 8 apart, so that one L2 serves them all.
+// (Lines beyond the last whole group of 8: launch order.)
+__device__ __forceinline__ void line_on_xcd(uint32_t parts, uint32_t lines, uint32_t& line, uint32_t& part) {
+  const uint32_t grouped = lines / 8 * 8 * parts, l = blockIdx.x;
+  if (l < grouped) {
+    const uint32_t g = l / (8 * parts), r = l - g * 8 * parts;
+    line = 8 * g + (r & 7);
+    part = r >> 3;
+  } else {
+    line = l / parts;
+    part = l - line * parts;
+  }
+}
+
 // Long axes, pass 1: block (line, chunk) sorts elements [chunk * ARGSORT_MAX, ...) of its line
 // and stores the sorted run: keys (32 bits, or 64 for int64 tensors) and indices.
 template <typename T, typename K> __device__ __forceinline__ void argsort_chunks_impl(const hck_sort_args& p) {
@@ -350,7 +365,8 @@ template <typename T, typename K> __device__ __forceinline__ void argsort_chunks
   __shared__ uint32_t idxs[WIDE ? SORT_SLOTS : 1];
   const SortBuf<WIDE> buf{keys, idxs};
   const uint32_t chunks = (p.reduce + ARGSORT_MAX - 1) / ARGSORT_MAX;
-  const uint32_t line = blockIdx.x / chunks, chunk = blockIdx.x - line * chunks;
+  uint32_t line, chunk;
+  line_on_xcd(chunks, p.outer * p.inner, line, chunk);
   const uint32_t i = line / p.inner, j = line - i * p.inner;
   const T* in = (const T*)p.in + (size_t)i * p.reduce * p.inner + j;
   const uint32_t first = chunk * ARGSORT_MAX;
@@ -376,13 +392,15 @@ template <typename T, typename K> __device__ __forceinline__ void argsort_chunks
 // per step; neighbouring lanes own neighbouring keys and mostly read the same lines. The pass that
 // completes the line writes the index straight to its place in the result.
 // One such pass does what four passes of pairwise merging and one that wrote the result did, each of them a launch
-// that moved every entry through memory: [8, 50257] fp32 54 -> 36 us. Bound by the address path: lanes of a load
-// go to different lines, four lanes a cycle.
+// that moved every entry through memory: [8, 50257] fp32 54 -> 36 us, 34 with the blocks of a line on one XCD.
+// Bound by the address path: lanes of a load go to different lines, four lanes a cycle. Windows of the other runs in LDS
+// (found by a search for the block's first and last entry) were slower: 43 us, for the search, the copies and two barriers.
 constexpr uint32_t ARGSORT_WAYS = 16;
 
 template <typename K> __device__ __forceinline__ void argsort_rank_impl(const hck_sort_args& p) {
   const uint32_t tiles = (p.reduce + HCK_BLOCK - 1) / HCK_BLOCK;
-  const uint32_t line = blockIdx.x / tiles, tile = blockIdx.x - line * tiles;
+  uint32_t line, tile;
+  line_on_xcd(tiles, p.outer * p.inner, line, tile);
   const K* keys = (const K*)p.keys_in + (size_t)line * p.reduce;
   const uint32_t pos = tile * HCK_BLOCK + threadIdx.x;
   const uint32_t own_start = tile * HCK_BLOCK / p.run * p.run;  // a tile lies inside one run

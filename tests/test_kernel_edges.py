@@ -30,6 +30,22 @@ def test_argsort_at_the_ends_of_runs(hip_backend, oracle_backend, dtype, shape):
         check_exact(hip_backend, oracle_backend, lambda: Tensor(data=f).argsort(1))
 
 
+@pytest.mark.parametrize("dtype", [F32, I64], ids=["f32", "i64"])
+@pytest.mark.parametrize("length", [4096 * 3 + 257, 65536 + 4097])
+def test_argsort_of_runs_that_overlap_unevenly(hip_backend, oracle_backend, dtype, length):
+    """Keys of some runs of 4096 lie between two neighbouring entries of others, and a line that is sorted already; nine
+    lines, of which the first eight go to an XCD each, along rows and along columns."""
+    rng = np.random.default_rng(length)
+    run = np.arange(length) // 4096
+    x = rng.integers(-30000, 30001, size=(9, length)) * np.where(run % 3 == 0, 1000, 1)
+    x[1] = np.sort(x[1])
+    x = x.astype(dtype.numpy)
+    for descending in (False, True):
+        check_exact(hip_backend, oracle_backend, lambda: Tensor(data=x).argsort(1, descending=descending, stable=True))
+    columns = np.ascontiguousarray(x.T)
+    check_exact(hip_backend, oracle_backend, lambda: Tensor(data=columns).argsort(0))
+
+
 @pytest.mark.parametrize("dtype", [F32, F16], ids=["f32", "f16"])
 @pytest.mark.parametrize("shape", [(3, 1), (5, 7), (70, 128), (3, 256), (3, 260), (2, 1024), (2, 1028), (3, 2048), (2, 2056),
                                    (2, 8192), (2, 8196), (2, 16384), (2, 16392), (1, 32771)], ids=str)
