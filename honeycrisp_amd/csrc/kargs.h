@@ -244,6 +244,7 @@ typedef struct {
   uint32_t middle;    /* source rows per outer slice */
   uint32_t row_vecs;  /* vectors per row */
   uint32_t total_rows;
+  uint32_t streaming;  /* wide kernels: the result is stored past the caches */
   hck_bcast idx; /* operand 0 = index offset for a flat row number, vec = 1 */
 } hck_gather_rows_args;
 

@@ -122,6 +122,29 @@ __device__ __forceinline__ void store_vec(T* base, size_t off, const T (&src)[N]
   *reinterpret_cast<Vec<T, N>*>(base + off) = t;
 }
 
+// Whole 16-byte vectors past the caches, for data that a launch touches once and that is more than they hold
+// (the host's rule: `streams` in hchip.cpp). STREAM false: load_vec / store_vec.
+typedef uint32_t StreamWords __attribute__((ext_vector_type(4)));
+template <bool STREAM, typename T, int N> __device__ __forceinline__ void load_once(const T* base, T (&dst)[N]) {
+  static_assert(sizeof(dst) == 16, "one 16-byte vector");
+  if (STREAM) {
+    const StreamWords w = __builtin_nontemporal_load(reinterpret_cast<const StreamWords*>(base));
+    __builtin_memcpy(dst, &w, 16);
+  } else {
+    load_vec<T, N>(base, 0, 1, dst);
+  }
+}
+template <bool STREAM, typename T, int N> __device__ __forceinline__ void store_once(T* base, size_t off, const T (&src)[N]) {
+  static_assert(sizeof(src) == 16, "one 16-byte vector");
+  if (STREAM) {
+    StreamWords w;
+    __builtin_memcpy(&w, src, 16);
+    __builtin_nontemporal_store(w, reinterpret_cast<StreamWords*>(base + off));
+  } else {
+    store_vec<T, N>(base, off, src);
+  }
+}
+
 // n / d with the (magic, sh) pair the host derived from d (hck_fast_div_setup): exact for every
 // 32-bit n, five instructions instead of the division sequence.
 __device__ __forceinline__ uint32_t fast_div(uint32_t n, uint32_t magic, uint32_t sh) {

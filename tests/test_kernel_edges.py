@@ -98,3 +98,25 @@ def test_gelu_gradient_over_its_range(hip_backend, dtype):
     with hip_backend.use():
         d = hip_backend.elemwise(Tensor(data=y).data, ElemwiseOp.geluApproxGrad, None, 3, dtype)
         assert np.isnan(Tensor(dataHandle=d, shape=[3], dtype=dtype).numpy()).all()
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, I64], ids=["f32", "f16", "i64"])
+@pytest.mark.parametrize("vecs,rows", [(64, 65535), (64, 65536), (256, 16383), (256, 16384), (256, 16385)])
+def test_gather_and_scatter_of_rows_around_64_mib(hip_backend, dtype, vecs, rows):
+    """Results of 64 MiB and more pass the caches: gather of `rows` rows (a quarter and all of a wave's vectors), scatter whose
+    sources and result come to as much. Small whole numbers: every sum is exact in every type."""
+    rng = np.random.default_rng(rows)
+    width, buckets = vecs * 16 // dtype.byteSize, 301
+    table = rng.integers(-3, 4, size=(buckets, width)).astype(dtype.numpy)
+    ids = rng.integers(0, buckets, size=(rows,))
+    ids[: rows // 2] = np.arange(rows // 2) % 7          # half of the sources meet in a few rows
+    x = rng.integers(-1, 2, size=(rows - buckets, 8)).astype(dtype.numpy)
+    with hip_backend.use():
+        got = Tensor(data=table).gather(0, Tensor(data=ids)).numpy()
+        assert got.tobytes() == table[ids].tobytes()
+        wide = np.tile(x, (1, width // 8))
+        summed = Tensor(data=wide).scatter(0, buckets, Tensor(data=ids[: rows - buckets])).numpy()
+    want = np.zeros((buckets, 8))
+    np.add.at(want, ids[: rows - buckets], x.astype(np.float64))
+    assert np.abs(want).max() < 2048                     # (fp16 holds whole numbers up to 2048)
+    np.testing.assert_array_equal(summed, np.tile(want.astype(dtype.numpy), (1, width // 8)))
