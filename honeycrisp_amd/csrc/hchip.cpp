@@ -2243,6 +2243,29 @@ extern "C" int hc_log_softmax(hc_ctx* ctx, int dtype, const void* in, void* out,
     snprintf(name, sizeof(name), "hc_log_softmax_rows256_%s", dtype_name(dtype));
     return launch(ctx, name, (uint64_t)outer, 1, &k, sizeof(k));
   }
+  if (few_long_rows) {
+    // pieces of at least 1024 elements (an fp32 vector per lane), four blocks per CU in all
+    const uint64_t most = 4 * (uint64_t)ctx->props.multiProcessorCount / (uint64_t)outer;
+    const uint64_t wanted = std::min<uint64_t>(std::max<uint64_t>(most, 2), ceil_div((uint64_t)reduce, 1024));
+    hck_softmax_split_args sp;
+    memset(&sp, 0, sizeof(sp));
+    sp.in = in;
+    sp.out = out;
+    sp.outer = (uint32_t)outer;
+    sp.reduce = (uint32_t)reduce;
+    sp.seg_len = (uint32_t)(ceil_div(ceil_div((uint64_t)reduce, wanted), 64) * 64);
+    sp.segs = (uint32_t)ceil_div((uint64_t)reduce, sp.seg_len);
+    Scratch scratch(ctx);
+    void *maxima = nullptr, *sums = nullptr;
+    HC_TRY(scratch.get((uint64_t)outer * sp.segs * sizeof(float), &maxima));
+    HC_TRY(scratch.get((uint64_t)outer * sp.segs * sizeof(float), &sums));
+    sp.seg_max = (float*)maxima;
+    sp.seg_expsum = (float*)sums;
+    snprintf(name, sizeof(name), "hc_log_softmax_split_%s", dtype_name(dtype));
+    HC_TRY(launch(ctx, name, (uint64_t)outer * sp.segs, 1, &sp, sizeof(sp)));
+    snprintf(name, sizeof(name), "hc_log_softmax_split_write_%s", dtype_name(dtype));
+    return launch(ctx, name, (uint64_t)outer * sp.segs, 1, &sp, sizeof(sp));
+  }
   return softmax_cols(ctx, dtype, in, nullptr, out, outer, reduce, inner);
 }
 

@@ -175,6 +175,15 @@ typedef struct {
   uint32_t pad;
 } hck_reduce_cols_args;
 
+/* logSoftmax of few long rows: [outer, reduce] cut into `segs` pieces of `seg_len` elements per row. */
+typedef struct {
+  const void* in;
+  void* out;
+  float* seg_max;     /* [outer, segs] maximum of a piece, ... */
+  float* seg_expsum;  /* ... and its sum of exp(x - maximum) */
+  uint32_t outer, reduce, segs, seg_len;
+} hck_softmax_split_args;
+
 /* Column logSoftmax / logSoftmaxGrad, last step: every element combined with per-column
  * statistics ([outer, inner] floats). */
 typedef struct {

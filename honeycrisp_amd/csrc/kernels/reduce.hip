@@ -465,6 +465,62 @@ template <typename T, int LANES> __device__ __forceinline__ void log_softmax_row
   stream_row_out<T, LANES>(in, out, n, lane, [&](float x, uint32_t) { return x - log_sum; });
 }
 
+// Few long rows (fewer than two per CU): a block per piece of a row. The first launch leaves every piece's maximum and its
+// sum of exponentials relative to that; the second brings the pieces of its row together in every block (the
+// sums scaled by exp(own maximum - maximum)) and writes its piece. Bound by the latency of a handful of dependent steps per
+// launch: as columns of extent 1 (maximum, its end, exp-sum, its end, logarithm, write-out) this was six launches,
+// [8, 50257] fp32 19 us; now 7.6 us.
+// A piece of nothing but -infinity (or NaN) takes its exponentials relative to 0: its sum is 0 (NaN), and a row
+// of such pieces only still becomes NaN when they meet.
+template <typename T, typename F> __device__ __forceinline__ void split_piece(const T* piece, uint32_t n, bool vectors, F f) {
+  if (vectors) stream_row<T, HCK_BLOCK>(piece, n, threadIdx.x, f);
+  else {
+#pragma unroll 4
+    for (uint32_t k = threadIdx.x; k < n; k += HCK_BLOCK) f((float)piece[k], k);
+  }
+}
+template <typename T, bool WRITE> __device__ __forceinline__ void log_softmax_split_impl(const hck_softmax_split_args& p) {
+  __shared__ float lds[HCK_BLOCK / 64];
+  const uint32_t row = blockIdx.x / p.segs, seg = blockIdx.x - row * p.segs;
+  const uint32_t first = seg * p.seg_len, n = p.reduce - first < p.seg_len ? p.reduce - first : p.seg_len;
+  const size_t at = (size_t)row * p.reduce + first;
+  const T* piece = (const T*)p.in + at;
+  // (pieces are whole numbers of vectors where rows are)
+  const bool vectors = p.reduce % VecWidth<T>::value == 0;
+  typedef Team<HCK_BLOCK> Block;
+  float m = -INFINITY, s = 0.0f;
+  if (!WRITE) {
+    split_piece(piece, n, vectors, [&](float x, uint32_t) { if (x > m) m = x; });
+    m = Block::reduce(m, MaxOp(), lds);
+    const float base = m == -INFINITY ? 0.0f : m;
+    split_piece(piece, n, vectors, [&](float x, uint32_t) { s += expf(x - base); });
+    s = Block::reduce(s, SumOp(), lds);
+    if (threadIdx.x == 0) {
+      p.seg_max[blockIdx.x] = m;
+      p.seg_expsum[blockIdx.x] = s;
+    }
+    return;
+  }
+  const float* maxima = p.seg_max + (size_t)row * p.segs;
+  const float* sums = p.seg_expsum + (size_t)row * p.segs;
+  for (uint32_t i = threadIdx.x; i < p.segs; i += HCK_BLOCK) m = maxima[i] > m ? maxima[i] : m;
+  m = Block::reduce(m, MaxOp(), lds);
+  for (uint32_t i = threadIdx.x; i < p.segs; i += HCK_BLOCK) s += sums[i] * expf(maxima[i] - m);
+  s = Block::reduce(s, SumOp(), lds);
+  const float log_sum = logf(s) + m;
+  T* out = (T*)p.out + at;
+  if (vectors) {
+    stream_row_out<T, HCK_BLOCK>(piece, out, n, threadIdx.x, [&](float x, uint32_t) { return x - log_sum; });
+  } else {
+#pragma unroll 4
+    for (uint32_t k = threadIdx.x; k < n; k += HCK_BLOCK) out[k] = narrow<T>((float)piece[k] - log_sum);
+  }
+}
+HC_KERNEL void hc_log_softmax_split_f32(hck_softmax_split_args p) { log_softmax_split_impl<float, false>(p); }
+HC_KERNEL void hc_log_softmax_split_f16(hck_softmax_split_args p) { log_softmax_split_impl<half_t, false>(p); }
+HC_KERNEL void hc_log_softmax_split_write_f32(hck_softmax_split_args p) { log_softmax_split_impl<float, true>(p); }
+HC_KERNEL void hc_log_softmax_split_write_f16(hck_softmax_split_args p) { log_softmax_split_impl<half_t, true>(p); }
+
 // Columns (inner > 1): per-column maximum and exp-sum come from the split column reductions
 // above (R_MAXF, R_EXPSUMF), then one element-wise pass applies them.
 template <typename T, int VEC, bool GRAD> __device__ __forceinline__ void softmax_cols_apply_impl(const hck_softmax_cols_args& p) {

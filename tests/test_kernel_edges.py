@@ -120,3 +120,28 @@ def test_gather_and_scatter_of_rows_around_64_mib(hip_backend, dtype, vecs, rows
     np.add.at(want, ids[: rows - buckets], x.astype(np.float64))
     assert np.abs(want).max() < 2048                     # (fp16 holds whole numbers up to 2048)
     np.testing.assert_array_equal(summed, np.tile(want.astype(dtype.numpy), (1, width // 8)))
+
+
+@pytest.mark.parametrize("dtype", [F32, F16], ids=["f32", "f16"])
+@pytest.mark.parametrize("shape", [(1, 32768), (1, 32769), (8, 50257), (3, 65536 + 8), (511, 32772)], ids=str)
+def test_log_softmax_of_few_long_rows(hip_backend, dtype, shape):
+    """Rows cut into pieces: whole and broken vectors, a last piece of any length, two pieces a row up to one per 1024 elements;
+    masked pieces (-infinity) count nothing, a NaN anywhere and a row of -infinity only give NaN."""
+    rng = np.random.default_rng(shape[1])
+    x = rand(rng, shape, dtype)
+    x[0, : shape[1] - 1500] = -np.inf
+    x64 = x.astype(np.float64)
+    m = x64.max(1, keepdims=True)
+    want = x64 - m - np.log(np.exp(x64 - m).sum(1, keepdims=True))
+    with hip_backend.use():
+        got = Tensor(data=x).logSoftmax().numpy().astype(np.float64)
+        # the sum's and the logarithm's last bits, one rounding of log(sum) + max, one of the difference
+        eps = np.finfo(dtype.numpy).eps
+        finite = np.isfinite(want)
+        assert np.array_equal(got[~finite], want[~finite])
+        assert np.abs(got - want)[finite].max() <= 2 * eps * np.abs(want[finite]).max() + 4e-6
+        y = x.copy()
+        y[0, shape[1] // 2] = np.nan
+        assert np.isnan(Tensor(data=y).logSoftmax().numpy()[0]).all()
+        y[0] = -np.inf
+        assert np.isnan(Tensor(data=y).logSoftmax().numpy()[0]).all()
