@@ -2212,8 +2212,7 @@ extern "C" int hc_log_softmax(hc_ctx* ctx, int dtype, const void* in, void* out,
   k.reduce = (uint32_t)reduce;
   k.inner = (uint32_t)inner;
   char name[64];
-  // (few long rows: a block per row would leave most of the device idle; the column path cuts the
-  // axis over many blocks)
+  // (few long rows: a block per row would leave most of the device idle; they are cut over many blocks)
   const bool few_long_rows = inner == 1 && (uint64_t)outer < 2 * (uint64_t)ctx->props.multiProcessorCount && reduce >= 32768;
   OpNote note({in}, {out});
   auto tag_rows = [&](int lanes) {   // rows held in the registers of a team of `lanes` lanes
