@@ -2127,8 +2127,11 @@ extern "C" int hc_cumulative(hc_ctx* ctx, int op, int dtype, const void* in, voi
     HC_TRY(scratch.get(units * 8, &k.carry));
     snprintf(name, sizeof(name), "hc_cumulative_%s_%s_totals_%s", opn, form, tn);
     HC_TRY(launch(ctx, name, blocks, 1, &k, sizeof(k)));
-    snprintf(name, sizeof(name), "hc_cumulative_%s_carry_%s", opn, dtype == HC_I64 ? "i64" : "f32");
-    HC_TRY(launch(ctx, name, ceil_div((uint64_t)outer * (uint64_t)inner, HCK_BLOCK / 64), 1, &k, sizeof(k)));  // a wave per line
+    k.totals = inner == 1 && segs <= 256;
+    if (!k.totals) {
+      snprintf(name, sizeof(name), "hc_cumulative_%s_carry_%s", opn, dtype == HC_I64 ? "i64" : "f32");
+      HC_TRY(launch(ctx, name, ceil_div((uint64_t)outer * (uint64_t)inner, HCK_BLOCK / 64), 1, &k, sizeof(k)));  // a wave per line
+    }
   }
   snprintf(name, sizeof(name), "hc_cumulative_%s_%s_%s", opn, form, tn);
   return launch(ctx, name, blocks, 1, &k, sizeof(k));

@@ -208,7 +208,8 @@ typedef struct {
   void* carry;
   uint32_t outer, reduce, inner;
   uint32_t exclusive, reverse;
-  uint32_t segs, seg_len, pad;
+  uint32_t segs, seg_len;
+  uint32_t totals;  /* rows: carry still holds the totals, every segment scans those before it */
 } hck_scan_args;
 
 /* argsort of axes longer than one block sorts at once: sorted runs of (key, index) pairs, one

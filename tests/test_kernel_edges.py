@@ -145,3 +145,16 @@ def test_log_softmax_of_few_long_rows(hip_backend, dtype, shape):
         assert np.isnan(Tensor(data=y).logSoftmax().numpy()[0]).all()
         y[0] = -np.inf
         assert np.isnan(Tensor(data=y).logSoftmax().numpy()[0]).all()
+
+
+@pytest.mark.parametrize("shape", [(1, 4096), (3, 65 * 1024), (2, 64 * 1024 + 1), (1, 256 * 1024), (1, 257 * 1024), (1, 260 * 1024 + 3)], ids=str)
+def test_running_sums_of_segmented_rows(hip_backend, oracle_backend, shape):
+    """Rows of 4 to 260 segments: around 64 (a round of a segment's own scan of the totals) and around 256 (past which a launch of its
+    own scans them); whole numbers, so every order of the sums gives the same."""
+    rng = np.random.default_rng(shape[1])
+    x = rng.integers(-2, 3, size=shape)
+    for exclusive in (False, True):
+        for reverse in (False, True):
+            for values in (x, x.astype(np.float32)):
+                check_exact(hip_backend, oracle_backend,
+                            lambda: Tensor(data=values).cumulativeSum(1, exclusive=exclusive, reverse=reverse))
