@@ -29,12 +29,14 @@ KERNELS = [
     ("gemm_dma", "gemm_dma.hip", ["-ffp-contract=off"]),
     ("gemm_dma2", "gemm_dma2.hip", ["-ffp-contract=off"]),
     ("gemm_mi16", "gemm_mi16.hip", ["-ffp-contract=off"]),
-    # the same three sources once more: kernels named *_m whose write-out applies the operations a
+    ("gemm_ks", "gemm_ks.hip", ["-ffp-contract=off"]),
+    # the same four sources once more: kernels named *_m whose write-out applies the operations a
     # recording merged into the product (the plain kernels above contain none of that code)
     ("gemm_dma_m", "gemm_dma.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1"]),
     ("gemm_dma2_m_f16", "gemm_dma2.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1", "-DHC_GEMM_ONLY=16"]),
     ("gemm_dma2_m_f32", "gemm_dma2.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1", "-DHC_GEMM_ONLY=32"]),
     ("gemm_mi16_m", "gemm_mi16.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1"]),
+    ("gemm_ks_m", "gemm_ks.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1"]),
 ]
 DEVICE_FLAGS = [
     "--offload-arch=gfx950", "--genco", "-O3", "-std=c++17",
@@ -57,6 +59,7 @@ def _run(cmd):
 # sit at the 256-VGPR limit; the edge kernels' write-out needs a few registers more): up to 96 bytes
 # per lane in the plain kernels, up to 128 in the kernels with merged epilogues.
 NO_SCRATCH = {"gemm_dma": 96, "gemm_dma2": 96, "gemm_mi16": 96, "gemm_f16_fast": 16,
+              "gemm_ks": 0, "gemm_ks_m": 0,
               "gemm_dma_m": 128, "gemm_dma2_m_f16": 128, "gemm_dma2_m_f32": 128, "gemm_mi16_m": 128}
 
 
@@ -102,7 +105,7 @@ def build_kernel(name, src, extra):
     if bad:
         os.remove(out)
         raise RuntimeError("%s: kernels that must not use scratch memory do: %s" % (src, ", ".join(bad)))
-    bad = kernels_with_promoted_private_data(remarks) if check and name != "gemm_f16_fast" else []
+    bad = kernels_with_promoted_private_data(remarks) if check and not name.startswith(("gemm_f16_fast", "gemm_ks")) else []
     if bad:
         os.remove(out)
         raise RuntimeError("%s: private data was moved into LDS: %s" % (src, ", ".join(bad)))

@@ -35,10 +35,12 @@ extern const unsigned char hc_image_gemm_f16_fast[], hc_image_gemm_f16_fast_end[
 extern const unsigned char hc_image_gemm_dma[], hc_image_gemm_dma_end[];
 extern const unsigned char hc_image_gemm_dma2[], hc_image_gemm_dma2_end[];
 extern const unsigned char hc_image_gemm_mi16[], hc_image_gemm_mi16_end[];
+extern const unsigned char hc_image_gemm_ks[], hc_image_gemm_ks_end[];
 extern const unsigned char hc_image_gemm_dma_m[], hc_image_gemm_dma_m_end[];
 extern const unsigned char hc_image_gemm_dma2_m_f16[], hc_image_gemm_dma2_m_f16_end[];
 extern const unsigned char hc_image_gemm_dma2_m_f32[], hc_image_gemm_dma2_m_f32_end[];
 extern const unsigned char hc_image_gemm_mi16_m[], hc_image_gemm_mi16_m_end[];
+extern const unsigned char hc_image_gemm_ks_m[], hc_image_gemm_ks_m_end[];
 }
 
 // noalloc.hip: looks up this device's copy of the library's fixed scratch array (device current)
@@ -123,7 +125,7 @@ struct hc_graph {
 // thread that flips a switch never races a thread that launches.
 struct hc_switches {
   char gemm_tile[16] = "";      // HCHIP_GEMM_TILE=general|<BM>x<BN>: overrides the tile choice
-  char gemm_kernel[16] = "";    // HCHIP_GEMM_KERNEL=dma|dma2|mi16|staged: the pipeline
+  char gemm_kernel[16] = "";    // HCHIP_GEMM_KERNEL=dma|dma2|mi16|ks|staged: the pipeline
   char gemm_ring[8] = "";       // HCHIP_GEMM_RING=4|2: ring-of-four variant of the smallest tiles forced / off
   char gemm_one[8] = "";        // HCHIP_GEMM_ONE=0: no single-slice variants
   bool gemm_no_peel = false;    // HCHIP_GEMM_NO_PEEL: no body-plus-fringes split
@@ -331,10 +333,12 @@ extern "C" int hc_init(int device, hc_ctx** out) {
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma, hc_image_gemm_dma_end, "gemm_dma");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma2, hc_image_gemm_dma2_end, "gemm_dma2");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_mi16, hc_image_gemm_mi16_end, "gemm_mi16");
+  if (s == HC_OK) s = load_image(ctx, hc_image_gemm_ks, hc_image_gemm_ks_end, "gemm_ks");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma_m, hc_image_gemm_dma_m_end, "gemm_dma_m");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma2_m_f16, hc_image_gemm_dma2_m_f16_end, "gemm_dma2_m_f16");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma2_m_f32, hc_image_gemm_dma2_m_f32_end, "gemm_dma2_m_f32");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_mi16_m, hc_image_gemm_mi16_m_end, "gemm_mi16_m");
+  if (s == HC_OK) s = load_image(ctx, hc_image_gemm_ks_m, hc_image_gemm_ks_m_end, "gemm_ks_m");
   if (s == HC_OK && ctx->batch_idle_after > 0) s = alloc_batch_flag_locked(ctx);
   if (s != HC_OK) {
     hc_shutdown(ctx);
@@ -809,7 +813,7 @@ static int emit_recording_locked(hc_ctx* ctx, std::vector<hc_pending>& list, siz
     if (e.dropped || e.kind == hc_pending::FREE) continue;
     if (sent++ == mark_at && mark_fn) HC_TRY(launch_fn(ctx, mark_fn, 1, 1, 1, HCK_BLOCK, 0, mark_args, sizeof(*mark_args)));
     if (e.kind == hc_pending::KERNEL) {
-      HC_TRY(launch_fn(ctx, e.fn, e.grid[0], e.grid[1], 1, HCK_BLOCK, 0, e.args.data(), e.args.size()));
+      HC_TRY(launch_fn(ctx, e.fn, e.grid[0], e.grid[1], 1, e.block[0], 0, e.args.data(), e.args.size()));
     } else if (e.kind == hc_pending::RAW_KERNEL) {
       size_t n = e.args.size();
       void* config[] = {HIP_LAUNCH_PARAM_BUFFER_POINTER, e.args.data(), HIP_LAUNCH_PARAM_BUFFER_SIZE, &n,
@@ -1158,7 +1162,7 @@ static int batch_grew_locked(hc_ctx* ctx) {
 }
 
 // Adds a launch to the list in progress (caller holds the mutex).
-static void record_launch_locked(hc_ctx* ctx, const std::string& name, hipFunction_t fn, uint32_t gx, uint32_t gy,
+static void record_launch_locked(hc_ctx* ctx, const std::string& name, hipFunction_t fn, uint32_t gx, uint32_t gy, uint32_t threads,
                                  const void* args, size_t bytes) {
   hc_pending e;
   e.kind = hc_pending::KERNEL;
@@ -1166,6 +1170,7 @@ static void record_launch_locked(hc_ctx* ctx, const std::string& name, hipFuncti
   e.name = name;
   e.grid[0] = gx;
   e.grid[1] = gy;
+  e.block[0] = threads;
   e.args.assign((const char*)args, (const char*)args + bytes);
   if (OpNote* n = OpNote::current) {
     e.known = true;
@@ -1252,7 +1257,7 @@ static int find_kernel_locked(hc_ctx* ctx, const std::string& name, hipFunction_
 }
 
 static int launch(hc_ctx* ctx, const std::string& name, uint64_t blocks_x, uint32_t blocks_y,
-                  const void* args, size_t bytes) {
+                  const void* args, size_t bytes, uint32_t threads = HCK_BLOCK) {
   if (blocks_x == 0 || blocks_y == 0) return HC_OK;
   if (blocks_x > 0x7fffffffull)
     return fail(HC_ERR_TOO_LARGE, "%s: grid of %llu blocks exceeds the launch limit", name.c_str(),
@@ -1261,10 +1266,10 @@ static int launch(hc_ctx* ctx, const std::string& name, uint64_t blocks_x, uint3
   hipFunction_t fn = nullptr;
   HC_TRY(find_kernel_locked(ctx, name, &fn));
   if (ctx->lazy) {
-    record_launch_locked(ctx, name, fn, (uint32_t)blocks_x, blocks_y, args, bytes);
+    record_launch_locked(ctx, name, fn, (uint32_t)blocks_x, blocks_y, threads, args, bytes);
     return batch_grew_locked(ctx);
   }
-  return launch_fn(ctx, fn, (uint32_t)blocks_x, blocks_y, 1, HCK_BLOCK, 0, args, bytes);
+  return launch_fn(ctx, fn, (uint32_t)blocks_x, blocks_y, 1, threads, 0, args, bytes);
 }
 
 static inline uint64_t ceil_div(uint64_t a, uint64_t b) { return (a + b - 1) / b; }
