@@ -324,6 +324,274 @@ template <int TMAX, int LANES> __device__ __forceinline__ void attention_impl(co
 #endif
 }
 
+// The softmax chain over BQ rows of a score tile whose rows may end anywhere (n a multiple of VEC): the lanes' vectors
+// cover NCH * LANES * VEC scores, of which those behind n count as -infinity from the maximum on (an exponential of
+// 0, which changes no sum) and leave as probabilities of 0, so that the code has no branches around vectors. Per row
+// the arithmetic and its order are the row kernel's.
+template <int LANES, int NCH, uint32_t BQ, uint32_t SP>
+__device__ __forceinline__ void attention_softmax_ragged(const hck_attention_args& p, char* s_lds, const uint32_t n, const uint32_t z, const uint32_t m0) {
+  typedef half_t H8 __attribute__((ext_vector_type(8)));
+  constexpr uint32_t TEAMS = HCK_BLOCK / LANES;
+  constexpr int WANT = NCH <= 2 ? 8 : 4;               // rows of a team at a time: as many as the registers hold
+  constexpr int R = TEAMS * WANT <= BQ ? WANT : BQ / TEAMS;
+  static_assert(BQ % (TEAMS * R) == 0, "the teams' passes cover the tile exactly");
+  const uint32_t tl = threadIdx.x % LANES, team = threadIdx.x / LANES;
+  const bool then_exp = (p.flags & HCK_SM_EXP) != 0;
+  const float s = p.scale;
+  const half_t s16 = (half_t)s;
+  const bool packed_scale = (float)s16 == s;
+  float one = 1.0f, minus_zero = -0.0f;
+  asm("" : "+v"(one), "+v"(minus_zero));   // (constants that the compiler must not fold)
+  const bool last_in = (tl + LANES * (NCH - 1)) * 8 < n;   // only the last vector of a lane can lie behind n
+  for (uint32_t first = team * R; first < BQ; first += TEAMS * R) {
+    H8 x[R][NCH];
+#pragma unroll
+    for (int j = 0; j < R; j++)
+#pragma unroll
+      for (int c = 0; c < NCH; c++) x[j][c] = *reinterpret_cast<const H8*>(s_lds + (first + j) * SP + (tl + LANES * c) * 16);
+    if (p.flags & HCK_SM_SCALE) {
+      if (packed_scale) {   // (the same bits: see attention_softmax_rows)
+#pragma unroll
+        for (int j = 0; j < R; j++)
+#pragma unroll
+          for (int c = 0; c < NCH; c++) x[j][c] = x[j][c] * s16;
+      } else {
+#pragma unroll
+        for (int j = 0; j < R; j++)
+#pragma unroll
+          for (int c = 0; c < NCH; c++)
+#pragma unroll
+            for (int i = 0; i < 8; i++) x[j][c][i] = narrow<half_t>((float)x[j][c][i] * s);
+      }
+    }
+    if (p.flags & HCK_SM_MASK) {
+      H8 m[R][NCH];
+#pragma unroll
+      for (int j = 0; j < R; j++) {
+        const uint64_t row = (uint64_t)z * n + m0 + first + j;   // this row among all score rows
+        const half_t* mask = (const half_t*)p.mask + (size_t)(row % p.mask_rows) * n;
+#pragma unroll
+        for (int c = 0; c < NCH; c++) m[j][c] = *reinterpret_cast<const H8*>(mask + (c == NCH - 1 && !last_in ? 0 : (tl + LANES * c) * 8));
+      }
+#pragma unroll
+      for (int j = 0; j < R; j++)
+#pragma unroll
+        for (int c = 0; c < NCH; c++) x[j][c] = x[j][c] + m[j][c];
+    }
+    if (!last_in) {
+#pragma unroll
+      for (int j = 0; j < R; j++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) x[j][NCH - 1][i] = (half_t)-INFINITY;
+    }
+    // What bounds this is the number of vector instructions per score, so: the maximum of fp16 values in packed fp16
+    // (which of two zeros it returns changes nothing below), and differences and products of an fp16 value formed by
+    // v_fma_mix_f32, which takes it as it is: x * 1 - m and x * c - 0 are rounded once, like x - m and x * c.
+    float mx[R], sum[R];
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      H8 v = x[j][0];
+#pragma unroll
+      for (int c = 1; c < NCH; c++) v = __builtin_elementwise_max(v, x[j][c]);
+      half2_t w[4];
+      __builtin_memcpy(w, &v, 16);
+      w[0] = __builtin_elementwise_max(__builtin_elementwise_max(w[0], w[1]), __builtin_elementwise_max(w[2], w[3]));
+      mx[j] = fmaxf((float)w[0][0], (float)w[0][1]);
+    }
+    team_reduce_each<LANES, R>(mx, MaxOp());
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      sum[j] = 0.0f;
+#pragma unroll
+      for (int c = 0; c < NCH; c++)
+#pragma unroll
+        for (int i = 0; i < 8; i++) sum[j] += exp_hw(fmaf((float)x[j][c][i], one, -mx[j]));
+    }
+    team_reduce_each<LANES, R>(sum, SumOp());
+#pragma unroll
+    for (int j = 0; j < R; j++) {
+      const float log_sum = logf(sum[j]) + mx[j];
+#pragma unroll
+      for (int c = 0; c < NCH; c++) {
+        H8 o;
+#pragma unroll
+        for (int i = 0; i < 8; i++) {
+          const half_t ls = narrow<half_t>(fmaf((float)x[j][c][i], one, -log_sum));   // (pinned: rounded to fp32 first, as the row kernel does)
+          o[i] = then_exp ? (half_t)__builtin_amdgcn_exp2f(fmaf((float)ls, 1.4426950408889634f, minus_zero)) : ls;
+        }
+        // (behind n the product wants zeros; without the exponential there would be -infinity)
+        if (c == NCH - 1 && !last_in) o = H8{};
+        *reinterpret_cast<H8*>(s_lds + (first + j) * SP + (tl + LANES * c) * 16) = o;
+      }
+    }
+  }
+}
+
+// The fp16 kernel for every other form: rows of up to TMAX scores of any length that is a multiple of 8, heads of HD =
+// 32, 64 or 128. A workgroup owns 32 query rows, so that rows of 1024 scores (64 KiB) leave room for two workgroups per
+// compute unit. 64 heads of 64, 1024 x 1024: 127 us in three launches (scores and probabilities pass memory, 128 MiB
+// four times) -> 74 us; 32 x 2048 x 2048 505 -> 206; 100 heads of 304 x 304 51 -> 25. What bounds it is the softmax's vector
+// arithmetic, about 16 instructions' time per score of which 8 are the two exponentials: 45 of the 74 us with the products
+// left out. The keys take 23 (every wave reads 32 bytes of 32 rows per load, 33 cycles of the address path; 128 KiB per
+// workgroup) and the values 12, hardly beside the softmax of the other workgroup (starting half of the workgroups later
+// changed nothing). Heads of 128 fit one workgroup per compute unit at T > 512.
+//   phase 1: wave w takes the keys 128 i + 32 w .. + 31 straight from memory into operand registers, the next ones on
+//            their way; scores to LDS, [32, T]
+//   phase 2: the row teams' chain in place; the first values are on their way into registers
+//   phase 3: out[32, HD], k over the keys in chunks of CK: registers -> LDS (two buffers, a barrier per chunk), the next
+//            chunks on their way. v_mfma_f32_32x32x16_f16 like every product with at most 128 columns per matrix:
+//            wave w owns the columns 32 w .. + 31 (waves HD / 32 .. 3 only bring values)
+template <int TMAX, int LANES, int HD> __device__ __forceinline__ void attention_rows32_impl(const hck_attention_args& p) {
+  constexpr uint32_t BQ = 32, SP = TMAX * 2 + 16, VP = HD * 2 + 16;
+  constexpr uint32_t CK = HD == 32 ? 64 : 32;                  // keys per chunk of values
+  constexpr int PIECES = CK * HD / 8 / HCK_BLOCK;              // 16-byte pieces of a chunk per lane: 1 (2 for HD = 128)
+  constexpr int AHEAD = HD == 128 ? 4 : 8;                     // chunks on their way
+  constexpr int KS = HD / 16;                                  // MFMAs per block of 32 keys
+  __shared__ __attribute__((aligned(16))) char s_lds[BQ * SP];
+  __shared__ __attribute__((aligned(16))) char v_lds[2 * CK * VP];
+  const uint32_t T = p.T, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t l32 = lane & 31, lgrp = lane >> 5;
+  uint32_t z, qb;
+  attention_block(z, qb);
+  const uint32_t m0 = qb * BQ;
+  uint32_t zh = z, zl = 0;
+  if (p.bdiv != 0) {
+    zh = z / p.bdiv;
+    zl = z - zh * p.bdiv;
+  }
+  const half_t* Q = (const half_t*)p.q + zh * p.q_bs + zl * p.q_bs2;
+  const half_t* K = (const half_t*)p.k + zh * p.k_bs + zl * p.k_bs2;
+  const half_t* V = (const half_t*)p.v + zh * p.v_bs + zl * p.v_bs2;
+  half_t* O = (half_t*)p.out + zh * p.o_bs + zl * p.o_bs2;
+
+  // ---- phase 1
+  {
+    Chunk qf[KS], kf[2][KS];
+    const uint32_t qrow = m0 + l32 < T ? m0 + l32 : T - 1;
+#pragma unroll
+    for (int s = 0; s < KS; s++) qf[s] = *reinterpret_cast<const Chunk*>(Q + (size_t)qrow * p.q_rs + s * 16 + lgrp * 8);
+    auto fetch = [&](Chunk (&f)[KS], uint32_t nb) {   // (keys past the end: the last one again)
+      const uint32_t row = nb + l32 < T ? nb + l32 : T - 1;
+#pragma unroll
+      for (int s = 0; s < KS; s++) f[s] = *reinterpret_cast<const Chunk*>(K + (size_t)row * p.k_rs + s * 16 + lgrp * 8);
+    };
+    auto scores = [&](const Chunk (&f)[KS], uint32_t nb) {
+      floatx16 acc;
+#pragma unroll
+      for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+#pragma unroll
+      for (int s = 0; s < KS; s++)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, f[s]), __builtin_bit_cast(half8, qf[s]), acc, 0, 0, 0);
+      // lane: query row l32, keys nb + 8 g + 4 lgrp .. + 3 in registers 4 g .. 4 g + 3
+#pragma unroll
+      for (int g = 0; g < 4; g++) {
+        half4v h;
+#pragma unroll
+        for (int e = 0; e < 4; e++) h[e] = narrow<half_t>(acc[4 * g + e]);
+        *reinterpret_cast<half4v*>(s_lds + l32 * SP + (nb + 8 * g + 4 * lgrp) * 2) = h;
+      }
+    };
+    fetch(kf[0], wave * 32);
+    for (uint32_t nb = wave * 32; nb < T; nb += 256) {
+      fetch(kf[1], nb + 128);
+      scores(kf[0], nb);
+      fetch(kf[0], nb + 256);
+      if (nb + 128 < T) scores(kf[1], nb + 128);
+    }
+  }
+
+  // ---- the first values on their way (rows past the end read as zero)
+  const __amdgpu_buffer_rsrc_t vsrc = __builtin_amdgcn_make_buffer_rsrc((void*)V, 0, ((T - 1) * p.v_rs + HD) * 2, 0x00020000);
+  Chunk vf[AHEAD][PIECES];
+  auto fetch_values = [&](Chunk (&f)[PIECES], uint32_t chunk) {
+#pragma unroll
+    for (int i = 0; i < PIECES; i++) {
+      const uint32_t piece = i * HCK_BLOCK + tid, key = chunk * CK + piece / (HD / 8), c = piece % (HD / 8);
+      f[i] = __builtin_amdgcn_raw_buffer_load_b128(vsrc, key < T ? key * p.v_rs * 2 + c * 16 : 0xfffffff0u, 0, 0);
+    }
+  };
+#pragma unroll
+  for (int u = 0; u < AHEAD; u++) fetch_values(vf[u], u);
+  lds_barrier();
+
+  // ---- phase 2
+  {
+    constexpr int NCH = (TMAX + LANES * 8 - 1) / (LANES * 8);
+    static_assert(NCH <= 4, "rows of TMAX elements fit the team's registers");
+    constexpr uint32_t FULL = LANES * 8;   // scores per vector of the team
+    if (T > (NCH - 1) * FULL) attention_softmax_ragged<LANES, NCH, BQ, SP>(p, s_lds, T, z, m0);
+    else if (NCH > 1 && T > (NCH - 2) * FULL) attention_softmax_ragged<LANES, (NCH > 1 ? NCH - 1 : 1), BQ, SP>(p, s_lds, T, z, m0);
+    else if (NCH > 2 && T > (NCH - 3) * FULL) attention_softmax_ragged<LANES, (NCH > 2 ? NCH - 2 : 1), BQ, SP>(p, s_lds, T, z, m0);
+    else attention_softmax_ragged<LANES, 1, BQ, SP>(p, s_lds, T, z, m0);
+  }
+
+  // ---- phase 3: operands: probabilities rows l32 (k-contiguous), values columns 32 w + l32 through the transposing
+  // read (a group of 16 lanes: k-rows 8 (grp / 2) + 4 h + r / 4, columns 16 (grp % 2) + 4 (r % 4) .. + 3)
+  const uint32_t r16 = lane & 15, grp = lane >> 4;
+  floatx16 acc;
+#pragma unroll
+  for (int e = 0; e < 16; e++) acc[e] = 0.0f;
+  const char* prow = s_lds + l32 * SP + lgrp * 16;
+  const char* vcol = v_lds + (8 * (grp >> 1) + (r16 >> 2)) * VP + (wave * 32 + 16 * (grp & 1) + 4 * (r16 & 3)) * 2;
+  const uint32_t chunks = (T + CK - 1) / CK;
+  const bool computes = wave < HD / 32;
+  // (the MFMAs of a chunk are issued behind the next one's LDS reads, so that neither waits for the other)
+  Chunk pf[2][CK / 16], wf[2][CK / 16];
+  auto read = [&](uint32_t chunk, int half) {
+#pragma unroll
+    for (uint32_t s = 0; s < CK / 16; s++) {
+      pf[half][s] = *reinterpret_cast<const Chunk*>(prow + (chunk * CK + 16 * s) * 2);
+      typedef short short4v __attribute__((ext_vector_type(4)));
+      typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+      const char* v = vcol + half * (CK * VP) + 16 * s * VP;
+      const u32x2 lo = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS short4v*)v));
+      const u32x2 hi = __builtin_bit_cast(u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((LDS_AS short4v*)(v + 4 * VP)));
+      wf[half][s] = Chunk{lo[0], lo[1], hi[0], hi[1]};
+    }
+  };
+  auto multiply = [&](int half) {
+#pragma unroll
+    for (uint32_t s = 0; s < CK / 16; s++)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, wf[half][s]), __builtin_bit_cast(half8, pf[half][s]), acc, 0, 0, 0);
+  };
+  for (uint32_t c0 = 0; c0 < chunks; c0 += AHEAD) {
+#pragma unroll
+    for (int u = 0; u < AHEAD; u++) {
+      const uint32_t chunk = c0 + u;
+      if (chunk < chunks) {
+        char* buf = v_lds + (u & 1) * (CK * VP);
+#pragma unroll
+        for (int i = 0; i < PIECES; i++) {
+          const uint32_t piece = i * HCK_BLOCK + tid;
+          *reinterpret_cast<Chunk*>(buf + piece / (HD / 8) * VP + piece % (HD / 8) * 16) = vf[u][i];
+        }
+      }
+      fetch_values(vf[u], chunk + AHEAD);
+      if (chunk < chunks) {
+        lds_barrier();   // this chunk is there (and, the first time, the probabilities); nobody reads the one before any more
+        if (computes) {
+          read(chunk, u & 1);
+          if (chunk > 0) multiply((u & 1) ^ 1);
+        }
+      }
+    }
+  }
+  if (computes) {
+    if (chunks & 1) multiply(0);
+    else multiply(1);
+  }
+  // lane: query row l32, columns 32 w + 8 g + 4 lgrp .. + 3
+  if (computes && m0 + l32 < T) {
+#pragma unroll
+    for (int g = 0; g < 4; g++) {
+      half4v h;
+#pragma unroll
+      for (int e = 0; e < 4; e++) h[e] = narrow<half_t>(acc[4 * g + e]);
+      *reinterpret_cast<half4v*>(O + (size_t)(m0 + l32) * p.o_rs + wave * 32 + 8 * g + 4 * lgrp) = h;
+    }
+  }
+}
+
 // The same kernel for fp32 tensors, T <= 256. Both products run on v_mfma_f32_32x32x2_f32 as the tiled
 // fp32 kernels of the library run them (gemm_dma.hip, gemm_dma2.hip): the second operand of the product
 // first, and inside every 16 k the instructions take the pairs k = {0, 4}, {1, 5}, {2, 6}, {3, 7},
@@ -502,3 +770,17 @@ template <int TMAX> __device__ __forceinline__ void attention_f32_impl(const hck
 HC_KERNEL void hc_attention_f16_t256(hck_attention_args p) { attention_impl<256, 8>(p); }
 HC_KERNEL void hc_attention_f16_t512(hck_attention_args p) { attention_impl<512, 64>(p); }
 HC_KERNEL void hc_attention_f32_t256(hck_attention_args p) { attention_f32_impl<256>(p); }
+#define DEF_ATTENTION_ROWS32(TMAX, LANES, OCC)                                                                            \
+  extern "C" __global__ __launch_bounds__(HCK_BLOCK, OCC) void hc_attention_f16_rows32_t##TMAX##_h32(hck_attention_args p) {   \
+    attention_rows32_impl<TMAX, LANES, 32>(p);                                                                            \
+  }                                                                                                                       \
+  extern "C" __global__ __launch_bounds__(HCK_BLOCK, OCC) void hc_attention_f16_rows32_t##TMAX##_h64(hck_attention_args p) {   \
+    attention_rows32_impl<TMAX, LANES, 64>(p);                                                                            \
+  }                                                                                                                       \
+  extern "C" __global__ __launch_bounds__(HCK_BLOCK, OCC) void hc_attention_f16_rows32_t##TMAX##_h128(hck_attention_args p) {  \
+    attention_rows32_impl<TMAX, LANES, 128>(p);                                                                           \
+  }
+DEF_ATTENTION_ROWS32(256, 8, 2)
+DEF_ATTENTION_ROWS32(512, 64, 2)
+DEF_ATTENTION_ROWS32(1024, 64, 2)
+DEF_ATTENTION_ROWS32(2048, 64, 1)
