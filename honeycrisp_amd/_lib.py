@@ -3,6 +3,7 @@
 There is no fallback: if the library has not been built, importing this module raises.
 """
 import ctypes
+import functools
 import os
 from ctypes import (POINTER, Structure, c_char, c_char_p, c_float, c_int, c_int64, c_size_t,
                     c_uint32, c_uint64, c_void_p)
@@ -133,6 +134,13 @@ def load(path: str = LIB_PATH) -> ctypes.CDLL:
         fn.restype = restype
         fn.argtypes = argtypes
     return lib
+
+
+@functools.lru_cache(maxsize=4096)
+def packed_strides(shape, strides):
+    """The C descriptor of a (shape, strides) pair of tuples as an argument of the calls that read one. A program's calls
+    repeat a few of them: the descriptor is kept, by value, and never written again."""
+    return ctypes.byref(make_strides(shape, strides))
 
 
 def make_strides(shape, strides) -> hc_strides:

@@ -272,7 +272,7 @@ class HIPData:
         backend, ptr = self.backend, self.ptr
         self.ptr = None
         if ptr and backend is not None and backend._ctx:
-            backend._lib.hc_free(backend._ctx, c_void_p(ptr))
+            backend._lib.hc_free(backend._ctx, ptr)
 
 
 class PermutationData(HIPData):
@@ -484,21 +484,24 @@ class HIPBackend(Backend):
     # -- storage (DataAllocator, Backend.swift:894-896)
 
     def allocate(self, byteCount: int) -> HIPData:
+        byteCount = int(byteCount)
         ptr = c_void_p()
-        self._check(self._lib.hc_malloc(self._ctx, c_size_t(max(int(byteCount), 0)), byref(ptr)))
-        return HIPData(self, ptr.value, int(byteCount))
+        status = self._lib.hc_malloc(self._ctx, byteCount if byteCount > 0 else 0, byref(ptr))
+        if status != _lib.HC_OK:
+            self._raise(status)
+        return HIPData(self, ptr.value, byteCount)
 
     def upload(self, host: np.ndarray) -> HIPData:
         host = np.ascontiguousarray(host)
         data = self.allocate(host.nbytes)
         if host.nbytes:
-            self._check(self._lib.hc_memcpy_h2d(self._ctx, c_void_p(data.ptr),
+            self._check(self._lib.hc_memcpy_h2d(self._ctx, data.ptr,
                                                 host.ctypes.data_as(c_void_p), host.nbytes))
         return data
 
     def _dev(self, data) -> HIPData:
         """Device buffer for `data`; foreign data is uploaded (cf. BackendMPS.swift:585-620)."""
-        if isinstance(data, HIPData) and data.backend is self:
+        if (type(data) is HIPData or isinstance(data, HIPData)) and data.backend is self:
             return data
         if isinstance(data, np.ndarray):
             return self.upload(data)
@@ -508,14 +511,14 @@ class HIPBackend(Backend):
 
     @staticmethod
     def _s(strides: BroadcastStrides):
-        return _lib.make_strides(strides.shape, strides.strides)
+        return _lib.packed_strides(tuple(strides.shape), tuple(strides.strides))
 
     @staticmethod
     def _scalar(value, dtype: DType):
-        """(float32 value, int64 value) the way T.toFloat() / T.toInt64() would give them."""
+        """(float32 value, int64 value) the way T.toFloat() / T.toInt64() would give them (the call rounds a float once)."""
         if dtype == DType.int64:
-            return c_float(0.0), c_int64(int(value))
-        return c_float(float(np.float32(value))), c_int64(0)
+            return 0.0, c_int64(int(value))
+        return value if type(value) is float else float(np.float32(value)), 0
 
     # -- ops
 
@@ -531,14 +534,14 @@ class HIPBackend(Backend):
         vf, vi = self._scalar(value, dtype)
         if dtype != DType.int64:
             vf = c_float(float(np.float32(value)))
-        self._check(self._lib.hc_fill(self._ctx, int(dtype), vf, vi, c_void_p(out.ptr), count))
+        self._check(self._lib.hc_fill(self._ctx, dtype, vf, vi, out.ptr, count))
         return out
 
     def broadcast(self, a: BroadcastData, dtype: DType) -> HIPData:
         out = self.allocate(product(a.strides.shape) * dtype.byteSize)
         ad = self._dev(a.data)
         s = self._s(a.strides)
-        self._check(self._lib.hc_broadcast(self._ctx, int(dtype), c_void_p(ad.ptr), byref(s), c_void_p(out.ptr)))
+        self._check(self._lib.hc_broadcast(self._ctx, dtype, ad.ptr, s, out.ptr))
         return out
 
     def binaryOp(self, a, b, op: NumericBinaryOp, dtype: DType, count: Optional[int] = None) -> HIPData:
@@ -546,8 +549,8 @@ class HIPBackend(Backend):
             out = self.allocate(product(a.strides.shape) * dtype.byteSize)
             ad, bd = self._dev(a.data), self._dev(b.data)
             sa, sb = self._s(a.strides), self._s(b.strides)
-            self._check(self._lib.hc_binary_op(self._ctx, int(op), int(dtype), c_void_p(ad.ptr), byref(sa),
-                                               c_void_p(bd.ptr), byref(sb), c_void_p(out.ptr)))
+            self._check(self._lib.hc_binary_op(self._ctx, op, dtype, ad.ptr, sa,
+                                               bd.ptr, sb, out.ptr))
             return out
         if count is None:
             raise TypeError("binaryOp with a scalar needs count")
@@ -556,16 +559,16 @@ class HIPBackend(Backend):
         out = self.allocate(count * dtype.byteSize)
         td = self._dev(tensor)
         sf, si = self._scalar(scalar, dtype)
-        self._check(self._lib.hc_binary_op_scalar(self._ctx, int(op), int(dtype), c_void_p(td.ptr), sf, si,
-                                                  int(scalar_first), c_void_p(out.ptr), count))
+        self._check(self._lib.hc_binary_op_scalar(self._ctx, op, dtype, td.ptr, sf, si,
+                                                  int(scalar_first), out.ptr, count))
         return out
 
     def _fused(self, fn, x, y, z, dtype):
         out = self.allocate(product(x.strides.shape) * dtype.byteSize)
         xd, yd, zd = self._dev(x.data), self._dev(y.data), self._dev(z.data)
         sx, sy, sz = self._s(x.strides), self._s(y.strides), self._s(z.strides)
-        self._check(fn(self._ctx, int(dtype), c_void_p(xd.ptr), byref(sx), c_void_p(yd.ptr), byref(sy),
-                       c_void_p(zd.ptr), byref(sz), c_void_p(out.ptr)))
+        self._check(fn(self._ctx, dtype, xd.ptr, sx, yd.ptr, sy,
+                       zd.ptr, sz, out.ptr))
         return out
 
     def mulAdd(self, input: BroadcastData, coeff: BroadcastData, bias: BroadcastData, dtype: DType):
@@ -590,8 +593,8 @@ class HIPBackend(Backend):
             out = self.allocate(product(a.strides.shape))
             ad, bd = self._dev(a.data), self._dev(b.data)
             sa, sb = self._s(a.strides), self._s(b.strides)
-            self._check(self._lib.hc_compare(self._ctx, int(op), int(dtype), c_void_p(ad.ptr), byref(sa),
-                                             c_void_p(bd.ptr), byref(sb), c_void_p(out.ptr)))
+            self._check(self._lib.hc_compare(self._ctx, op, dtype, ad.ptr, sa,
+                                             bd.ptr, sb, out.ptr))
             return out
         if count is None:
             raise TypeError("compare with a scalar needs count")
@@ -600,15 +603,15 @@ class HIPBackend(Backend):
         out = self.allocate(count)
         td = self._dev(tensor)
         sf, si = self._scalar(scalar, dtype)
-        self._check(self._lib.hc_compare_scalar(self._ctx, int(op), int(dtype), c_void_p(td.ptr), sf, si,
-                                                int(scalar_first), c_void_p(out.ptr), count))
+        self._check(self._lib.hc_compare_scalar(self._ctx, op, dtype, td.ptr, sf, si,
+                                                int(scalar_first), out.ptr, count))
         return out
 
     def cast(self, a, count: int, inType: DType, outType: DType) -> HIPData:
         out = self.allocate(count * outType.byteSize)
         ad = self._dev(a)
-        self._check(self._lib.hc_cast(self._ctx, c_void_p(ad.ptr), int(inType), c_void_p(out.ptr),
-                                      int(outType), count))
+        self._check(self._lib.hc_cast(self._ctx, ad.ptr, inType, out.ptr,
+                                      outType, count))
         return out
 
     def pow(self, a, b: Scalar, scale: Scalar, scales, count: int, dtype: DType) -> HIPData:
@@ -617,30 +620,30 @@ class HIPBackend(Backend):
         sd = self._dev(scales) if scales is not None else None
         bf, bi = self._scalar(b, dtype)
         scf, sci = self._scalar(scale, dtype)
-        self._check(self._lib.hc_pow(self._ctx, int(dtype), c_void_p(ad.ptr), bf, scf, bi, sci,
-                                     c_void_p(sd.ptr) if sd else None, c_void_p(out.ptr), count))
+        self._check(self._lib.hc_pow(self._ctx, dtype, ad.ptr, bf, scf, bi, sci,
+                                     sd.ptr if sd else None, out.ptr, count))
         return out
 
     def elemwise(self, a, op: ElemwiseOp, scales, count: int, dtype: DType) -> HIPData:
         out = self.allocate(count * dtype.byteSize)
         ad = self._dev(a)
         sd = self._dev(scales) if scales is not None else None
-        self._check(self._lib.hc_elemwise(self._ctx, int(op), int(dtype), c_void_p(ad.ptr),
-                                          c_void_p(sd.ptr) if sd else None, c_void_p(out.ptr), count))
+        self._check(self._lib.hc_elemwise(self._ctx, op, dtype, ad.ptr,
+                                          sd.ptr if sd else None, out.ptr, count))
         return out
 
     def reduce(self, a, op: ReduceOp, dims: ReduceDims, dtype: DType) -> HIPData:
         outType = DType.int64 if op.isIntOut else dtype
         out = self.allocate(dims.outCount * outType.byteSize)
         ad = self._dev(a)
-        self._check(self._lib.hc_reduce(self._ctx, int(op), int(dtype), c_void_p(ad.ptr), c_void_p(out.ptr),
+        self._check(self._lib.hc_reduce(self._ctx, op, dtype, ad.ptr, out.ptr,
                                         dims.outerCount, dims.reduceCount, dims.innerCount))
         return out
 
     def logSoftmax(self, a, dims: ReduceDims, dtype: DType) -> HIPData:
         out = self.allocate(dims.inCount * dtype.byteSize)
         ad = self._dev(a)
-        self._check(self._lib.hc_log_softmax(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(out.ptr),
+        self._check(self._lib.hc_log_softmax(self._ctx, dtype, ad.ptr, out.ptr,
                                              dims.outerCount, dims.reduceCount, dims.innerCount))
         return out
 
@@ -649,7 +652,7 @@ class HIPBackend(Backend):
         innerCount == 1)."""
         out = self.allocate(dims.inCount * dtype.byteSize)
         ad = self._dev(input)
-        self._check(self._lib.hc_normalize(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(out.ptr),
+        self._check(self._lib.hc_normalize(self._ctx, dtype, ad.ptr, out.ptr,
                                            dims.outerCount, dims.reduceCount, dims.innerCount,
                                            c_float(float(np.float32(eps)))))
         return out
@@ -669,14 +672,14 @@ class HIPBackend(Backend):
                 perm, shape = [0] + [p + 1 for p in perm], [s.outerCount] + shape
             n = len(shape)
             if n <= 8:      # (hc_permute takes up to 8 axes; more fall through to the index gather)
-                self._check(self._lib.hc_permute(self._ctx, int(dtype), c_void_p(self._dev(a).ptr),
+                self._check(self._lib.hc_permute(self._ctx, dtype, self._dev(a).ptr,
                                                  (c_int64 * max(n, 1))(*perm), (c_int64 * max(n, 1))(*shape), n,
-                                                 s.innerCount, c_void_p(out.ptr)))
+                                                 s.innerCount, out.ptr))
                 return out
         ad, idx = self._dev(a), self._dev(s.indices.data)
         st = self._s(s.indices.strides)
-        self._check(self._lib.hc_gather(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(idx.ptr), byref(st),
-                                        c_void_p(out.ptr), s.outerCount, s.middleCount, s.outCount,
+        self._check(self._lib.hc_gather(self._ctx, dtype, ad.ptr, idx.ptr, st,
+                                        out.ptr, s.outerCount, s.middleCount, s.outCount,
                                         s.innerCount))
         return out
 
@@ -697,16 +700,16 @@ class HIPBackend(Backend):
         out = self.allocate(product(a.strides.shape) * dtype.byteSize)
         ad, bd = self._dev(a.data), self._dev(b.data)
         sa, sb = self._s(a.strides), self._s(b.strides)
-        self._check(self._lib.hc_bitwise_op(self._ctx, int(op), int(dtype), c_void_p(ad.ptr), byref(sa),
-                                            c_void_p(bd.ptr), byref(sb), c_void_p(out.ptr)))
+        self._check(self._lib.hc_bitwise_op(self._ctx, op, dtype, ad.ptr, sa,
+                                            bd.ptr, sb, out.ptr))
         return out
 
     def scatter(self, a, s: ScatterGatherIndices, dtype: DType) -> HIPData:
         out = self.allocate(s.gatherInCount * dtype.byteSize)
         ad, idx = self._dev(a), self._dev(s.indices.data)
         st = self._s(s.indices.strides)
-        self._check(self._lib.hc_scatter(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(idx.ptr), byref(st),
-                                         c_void_p(out.ptr), s.outerCount, s.middleCount, s.outCount,
+        self._check(self._lib.hc_scatter(self._ctx, dtype, ad.ptr, idx.ptr, st,
+                                         out.ptr, s.outerCount, s.middleCount, s.outCount,
                                          s.innerCount, int(bool(s.indicesAreUnique))))
         return out
 
@@ -732,23 +735,23 @@ class HIPBackend(Backend):
             return super().normalizeGrad(input, outGrad, dims, eps, dtype)
         out = self.allocate(dims.inCount * dtype.byteSize)
         ad, gd = self._dev(input), self._dev(outGrad)
-        self._check(self._lib.hc_normalize_grad(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(gd.ptr),
-                                                c_void_p(out.ptr), dims.outerCount, dims.reduceCount,
+        self._check(self._lib.hc_normalize_grad(self._ctx, dtype, ad.ptr, gd.ptr,
+                                                out.ptr, dims.outerCount, dims.reduceCount,
                                                 c_float(float(np.float32(eps)))))
         return out
 
     def logSoftmaxGrad(self, a, outGrad, dims: ReduceDims, dtype: DType) -> HIPData:
         out = self.allocate(dims.inCount * dtype.byteSize)
         ad, gd = self._dev(a), self._dev(outGrad)
-        self._check(self._lib.hc_log_softmax_grad(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(gd.ptr),
-                                                  c_void_p(out.ptr), dims.outerCount, dims.reduceCount,
+        self._check(self._lib.hc_log_softmax_grad(self._ctx, dtype, ad.ptr, gd.ptr,
+                                                  out.ptr, dims.outerCount, dims.reduceCount,
                                                   dims.innerCount))
         return out
 
     def _cumulative(self, op: int, a, dims: ReduceDims, exclusive: bool, reverse: bool, dtype: DType) -> HIPData:
         out = self.allocate(dims.inCount * dtype.byteSize)
         ad = self._dev(a)
-        self._check(self._lib.hc_cumulative(self._ctx, op, int(dtype), c_void_p(ad.ptr), c_void_p(out.ptr),
+        self._check(self._lib.hc_cumulative(self._ctx, op, int(dtype), ad.ptr, out.ptr,
                                             dims.outerCount, dims.reduceCount, dims.innerCount, int(bool(exclusive)),
                                             int(bool(reverse))))
         return out
@@ -763,7 +766,7 @@ class HIPBackend(Backend):
         """Always stable, which `stable=False` permits (Backend.swift:535-545)."""
         out = self.allocate(dims.inCount * 8)
         ad = self._dev(a)
-        self._check(self._lib.hc_argsort(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(out.ptr), dims.outerCount,
+        self._check(self._lib.hc_argsort(self._ctx, dtype, ad.ptr, out.ptr, dims.outerCount,
                                          dims.reduceCount, dims.innerCount, int(bool(descending))))
         return out
 
@@ -782,9 +785,9 @@ class HIPBackend(Backend):
         lod, hid = (self._dev(lo.data) if lo else None), (self._dev(hi.data) if hi else None)
         sl, sh = (self._s(lo.strides) if lo else None), (self._s(hi.strides) if hi else None)
         self._check(self._lib.hc_clamp(
-            self._ctx, int(dtype), c_void_p(ad.ptr), byref(sa),
-            c_void_p(lod.ptr) if lo else None, byref(sl) if lo else None,
-            c_void_p(hid.ptr) if hi else None, byref(sh) if hi else None, c_void_p(out.ptr)))
+            self._ctx, dtype, ad.ptr, sa,
+            lod.ptr if lo else None, sl,
+            hid.ptr if hi else None, sh, out.ptr))
         return out
 
     def adamW(self, param, grad, moment1, moment2, beta1, beta2, eps, weightDecay, lr, step, count,
@@ -793,8 +796,7 @@ class HIPBackend(Backend):
         outs = [self.allocate(count * dtype.byteSize) for _ in range(3)]
         ins = [self._dev(x) for x in (param, grad, moment1, moment2)]
         self._check(self._lib.hc_adamw(
-            self._ctx, int(dtype), *[c_void_p(x.ptr) for x in ins], c_float(beta1), c_float(beta2), c_float(eps),
-            c_float(weightDecay), c_float(lr), c_float(step), c_size_t(count), *[c_void_p(o.ptr) for o in outs]))
+            self._ctx, dtype, *[x.ptr for x in ins], beta1, beta2, eps, weightDecay, lr, step, count, *[o.ptr for o in outs]))
         return tuple(outs)
 
     def matmul(self, a, transA: bool, b, transB: bool, transOut: bool, rows: int, inner: int, cols: int,
@@ -805,15 +807,15 @@ class HIPBackend(Backend):
                       inner: int, cols: int, dtype: DType) -> HIPData:
         out = self.allocate(matrixCount * rows * cols * dtype.byteSize)
         ad, bd = self._dev(a), self._dev(b)
-        self._check(self._lib.hc_matmul(self._ctx, int(dtype), matrixCount, c_void_p(ad.ptr), int(transA),
-                                        c_void_p(bd.ptr), int(transB), int(transOut), rows, inner, cols,
-                                        c_void_p(out.ptr)))
+        self._check(self._lib.hc_matmul(self._ctx, dtype, matrixCount, ad.ptr, int(transA),
+                                        bd.ptr, int(transB), int(transOut), rows, inner, cols,
+                                        out.ptr))
         return out
 
     def triangular(self, a, batch: int, rows: int, cols: int, upper: bool, offset: int, dtype: DType):
         out = self.allocate(batch * rows * cols * dtype.byteSize)
         ad = self._dev(a)
-        self._check(self._lib.hc_triangular(self._ctx, int(dtype), c_void_p(ad.ptr), c_void_p(out.ptr), batch,
+        self._check(self._lib.hc_triangular(self._ctx, dtype, ad.ptr, out.ptr, batch,
                                             rows, cols, int(upper), offset))
         return out
 
@@ -824,7 +826,7 @@ class HIPBackend(Backend):
         n = len(devs)
         ptrs = (c_void_p * max(n, 1))(*[d.ptr for d in devs])
         counts = (c_int64 * max(n, 1))(*innerCounts)
-        self._check(self._lib.hc_concat(self._ctx, int(dtype), ptrs, counts, n, outerCount, c_void_p(out.ptr)))
+        self._check(self._lib.hc_concat(self._ctx, dtype, ptrs, counts, n, outerCount, out.ptr))
         return out
 
     # bytes of permutation index vectors kept for reuse

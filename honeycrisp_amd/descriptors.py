@@ -7,6 +7,8 @@ NumericBinaryOp (BinaryOps.swift:2-23), ElemwiseOp (Elemwise.swift:13-43),
 ComparisonOp (Comparison.swift:4-28), BackendError (Backend.swift:6-16).
 """
 import enum
+import functools
+import math
 from dataclasses import dataclass
 from typing import Any, List, Sequence
 
@@ -21,15 +23,15 @@ class DType(enum.IntEnum):
 
     @property
     def byteSize(self) -> int:
-        return (8, 1, 2, 4)[int(self)]
+        return (8, 1, 2, 4)[self]
 
     @property
     def isNumeric(self) -> bool:
-        return self != DType.bool
+        return self is not DType.bool
 
     @property
     def isFloat(self) -> bool:
-        return self in (DType.float16, DType.float32)
+        return self is DType.float16 or self is DType.float32
 
     @property
     def numpy(self):
@@ -136,15 +138,22 @@ class BackendError(Exception):
 
 
 def product(xs: Sequence[int]) -> int:
-    n = 1
-    for x in xs:
-        n *= int(x)
+    n = math.prod(xs)
+    if type(n) is not int:      # (numpy integers among them: their products wrap)
+        n = 1
+        for x in xs:
+            n *= int(x)
     return n
 
 
 def stridesForShape(shape: Sequence[int]) -> List[int]:
     """Row-major strides (Broadcast.swift:238-244)."""
-    return [product(shape[i + 1:]) for i in range(len(shape))]
+    strides, n = [], 1
+    for size in reversed(shape):
+        strides.append(n)
+        n *= int(size)
+    strides.reverse()
+    return strides
 
 
 class BroadcastStrides:
@@ -161,6 +170,15 @@ class BroadcastStrides:
     def contiguousForShape(shape: Sequence[int]) -> "BroadcastStrides":
         return BroadcastStrides(shape, stridesForShape(shape))
 
+    @staticmethod
+    def expanding(shape: Sequence[int], newShape: Sequence[int]) -> "BroadcastStrides":
+        """Dense data of `shape` seen as `newShape` (Broadcast.swift:148-170). A program's calls repeat a few pairs of
+        shapes, so what follows from a pair is kept (by value, 4096 pairs); the object and its lists are the caller's own."""
+        made = BroadcastStrides.__new__(BroadcastStrides)
+        newShape, strides, made.dataCount, made.isNoOp = _expanded(tuple(shape), tuple(newShape))
+        made.shape, made.strides = list(newShape), list(strides)
+        return made
+
     def __call__(self, i: int) -> int:
         """Virtual index -> data index (Broadcast.swift:72-90)."""
         if self.isNoOp:
@@ -173,6 +191,22 @@ class BroadcastStrides:
 
     def __repr__(self):
         return "BroadcastStrides(shape=%s, strides=%s)" % (self.shape, self.strides)
+
+
+@functools.lru_cache(maxsize=4096)
+def _expanded(shape, newShape):
+    assert len(newShape) >= len(shape), "cannot broadcast %s to shorter shape %s" % (list(shape), list(newShape))
+    extra = len(newShape) - len(shape)
+    strides = [0] * extra
+    for i, (oldSize, oldStride) in enumerate(zip(shape, stridesForShape(shape))):
+        newSize = newShape[i + extra]
+        if newSize != oldSize:
+            assert oldSize == 1, "axis %d cannot expand from size %d to %d" % (i, oldSize, newSize)
+            strides.append(0)
+        else:
+            strides.append(oldStride)
+    made = BroadcastStrides(newShape, strides)
+    return tuple(made.shape), tuple(made.strides), made.dataCount, made.isNoOp
 
 
 @dataclass

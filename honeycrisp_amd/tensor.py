@@ -210,7 +210,7 @@ class Tensor:
         if dataHandle is not None:
             self.data = dataHandle
             self.shape = list(shape)
-            self.dtype = DType(dtype)
+            self.dtype = dtype if type(dtype) is DType else DType(dtype)
             return
         if isinstance(data, np.ndarray):
             arr = data
@@ -304,8 +304,9 @@ class Tensor:
 
     def cast(self, newType) -> "Tensor":
         """Tensor.swift:802-819."""
-        newType = newType.dtype if isinstance(newType, Tensor) else DType(newType)
-        if newType == self.dtype:
+        if type(newType) is not DType:
+            newType = newType.dtype if isinstance(newType, Tensor) else DType(newType)
+        if newType is self.dtype:
             return self
         data = Backend.current().cast(self.data, product(self.shape), self.dtype, newType)
         return self._new(data, dtype=newType)
@@ -313,18 +314,7 @@ class Tensor:
     # -- broadcasting (Broadcast.swift:115-236)
 
     def expandStrides(self, newShape) -> BroadcastStrides:
-        newShape = list(newShape)
-        assert len(newShape) >= len(self.shape), "cannot broadcast %s to shorter shape %s" % (self.shape, newShape)
-        extra = len(newShape) - len(self.shape)
-        strides = [0] * extra
-        for i, (oldSize, oldStride) in enumerate(zip(self.shape, stridesForShape(self.shape))):
-            newSize = newShape[i + extra]
-            if newSize != oldSize:
-                assert oldSize == 1, "axis %d cannot expand from size %d to %d" % (i, oldSize, newSize)
-                strides.append(0)
-            else:
-                strides.append(oldStride)
-        return BroadcastStrides(newShape, strides)
+        return BroadcastStrides.expanding(self.shape, newShape)
 
     @staticmethod
     def broadcastShape(shapes) -> List[int]:
@@ -333,6 +323,8 @@ class Tensor:
             return shapes[0]
         if len(shapes) == 2:
             s0, s1 = shapes
+            if s0 == s1:
+                return s0
             while len(s0) < len(s1):
                 s0 = [1] + s0
             while len(s1) < len(s0):
@@ -388,7 +380,7 @@ class Tensor:
     def _binary(self, other, op: NumericBinaryOp, reverse=False) -> "Tensor":
         backend = Backend.current()
         assert self.dtype.isNumeric, "dtype %s cannot be used with arithmetic operators" % self.dtype.name
-        if isinstance(other, _SCALARS):
+        if type(other) is not Tensor and isinstance(other, _SCALARS):
             n = product(self.shape)
             if reverse:
                 # scalar + tensor and scalar * tensor are rewritten as tensor (op) scalar
