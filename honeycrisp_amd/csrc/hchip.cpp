@@ -2145,6 +2145,12 @@ extern "C" int hc_cumulative(hc_ctx* ctx, int op, int dtype, const void* in, voi
   return launch(ctx, name, blocks, 1, &k, sizeof(k));
 }
 
+// Whether lines (or the runs of long ones) are sorted by blocks of 1024 lanes instead of 256: while there are no more blocks than
+// compute units, a sort is a chain of LDS reads, which four times the lanes make shorter (rule and figures: scan.hip).
+static bool wide_sort(const hc_ctx* ctx, uint64_t blocks, uint64_t entries) {
+  return entries > 512 && blocks <= (uint64_t)ctx->props.multiProcessorCount;
+}
+
 extern "C" int hc_argsort(hc_ctx* ctx, int dtype, const void* in, void* out, int64_t outer, int64_t reduce,
                           int64_t inner, int descending) {
   OpNote note({in}, {out});
@@ -2185,8 +2191,10 @@ extern "C" int hc_argsort(hc_ctx* ctx, int dtype, const void* in, void* out, int
     s.keys_out = keys[0];
     s.idx_out = (uint32_t*)idx[0];
     char name[64];
-    snprintf(name, sizeof(name), "hc_argsort_chunks_%s", dtype_name(dtype));
-    HC_TRY(launch(ctx, name, lines * ceil_div((uint64_t)reduce, 4096), 1, &s, sizeof(s)));
+    const uint64_t chunks = lines * ceil_div((uint64_t)reduce, 4096);
+    const bool wide = wide_sort(ctx, chunks, 4096);
+    snprintf(name, sizeof(name), "hc_argsort_chunks%s_%s", wide ? "_wide" : "", dtype_name(dtype));
+    HC_TRY(launch(ctx, name, chunks, 1, &s, sizeof(s), wide ? 1024 : HCK_BLOCK));
     int cur = 0;
     for (uint64_t run = 4096; run < (uint64_t)reduce; cur ^= 1) {
       const uint32_t ways = ways_of(run);
@@ -2212,8 +2220,9 @@ extern "C" int hc_argsort(hc_ctx* ctx, int dtype, const void* in, void* out, int
   k.inner = (uint32_t)inner;
   k.reverse = descending != 0;
   char name[64];
-  snprintf(name, sizeof(name), "hc_argsort_%s", dtype_name(dtype));
-  return launch(ctx, name, (uint64_t)outer * (uint64_t)inner, 1, &k, sizeof(k));
+  const bool wide = wide_sort(ctx, (uint64_t)outer * (uint64_t)inner, (uint64_t)reduce);
+  snprintf(name, sizeof(name), "hc_argsort%s_%s", wide ? "_wide" : "", dtype_name(dtype));
+  return launch(ctx, name, (uint64_t)outer * (uint64_t)inner, 1, &k, sizeof(k), wide ? 1024 : HCK_BLOCK);
 }
 
 // Whether the rows go to the logSoftmax kernels whose blocks hold 8 vectors of 16 bytes per lane: rows of whole vectors,

@@ -209,6 +209,11 @@ __device__ __forceinline__ uint64_t sort_key(float x) {
 __device__ __forceinline__ uint64_t sort_key(int64_t x) { return (uint64_t)x ^ 0x8000000000000000ull; }
 
 constexpr int ARGSORT_MAX = 4096;
+// Lanes of a sorting block while there are no more blocks than compute units. What bounds a block alone is the chain of dependent
+// LDS reads: 26 per level and 8 levels with 16 entries per lane, 13 per level and 10 levels with 4. us, 256 lanes / 1024: 8 lines of
+// 600 fp32 11.1 / 9.9, of 1025 15.4 / 12.8, of 4096 24.8 / 19.8 (int64 34.9 / 25.7), of 50257 47.7 / 42.0; 256 lines of 4096 26.6 / 21.6,
+// but 512 33.0 / 33.4 and 1024 45.2 / 58.7, where blocks share a unit; 512 entries and fewer 7.6 / 8.2.
+constexpr uint32_t SORT_WIDE_BLOCK = 1024;
 
 // What the block sort orders. Keys of 32 significant bits (floats, halfs) travel with their
 // index in one 64-bit word (key in the high half), so one integer comparison orders by
@@ -269,7 +274,7 @@ __device__ __forceinline__ void count_before(const SortBuf<WIDE>& buf, uint32_t 
 // registers (bitonic network on constant indices). [256, n] fp32 in us, merged from single entries / a bitonic network in LDS / now: n = 64 5.3 / 5.2 /
 // 3.0 (argsort_impl alone), 128 6.0 / 5.9 / 4.5, 256 6.5 / 7.6 / 5.5, 512 8.1 / 7.6 / 7.4. (Two int64 entries per lane: counting costs two
 // comparisons more, 9.8 us at 512 against 9.5.)
-template <bool WIDE, int E> __device__ __forceinline__ void merge_sort_lds(const SortBuf<WIDE>& buf, uint32_t count) {
+template <bool WIDE, int E, uint32_t BLOCK> __device__ __forceinline__ void merge_sort_lds(const SortBuf<WIDE>& buf, uint32_t count) {
   constexpr bool COUNTED = E == 1 || (E == 2 && !WIDE);
   uint64_t kx[E];
   uint32_t ix[E], to[E];   // an entry, and its place
@@ -329,7 +334,7 @@ template <bool WIDE, int E> __device__ __forceinline__ void merge_sort_lds(const
     }
     uint32_t x = a0 + lo, y = b0 + d - lo;         // next entry of either run
     const uint32_t x_end = b0, y_end = b0 + run;   // (an entry past its run's end is never taken; its slot is clamped)
-    const uint32_t last = E * HCK_BLOCK - 1;
+    const uint32_t last = E * BLOCK - 1;
     uint32_t sa = sort_slot(x), sb = sort_slot(y < last ? y : last);
     uint64_t ka = buf.keys[sa], kb = buf.keys[sb];
     uint32_t ia = WIDE ? buf.idxs[sa] : 0, ib = WIDE ? buf.idxs[sb] : 0;
@@ -354,21 +359,23 @@ template <bool WIDE, int E> __device__ __forceinline__ void merge_sort_lds(const
   }
 }
 
-// entries per lane that a sort of `count` <= ARGSORT_MAX entries runs with: 1, 2, 4, 8 or 16
-__device__ __forceinline__ uint32_t sort_entries(uint32_t count) {
+// entries per lane that a sort of `count` <= ARGSORT_MAX entries runs with: a power of two up to ARGSORT_MAX / BLOCK
+template <uint32_t BLOCK> __device__ __forceinline__ uint32_t sort_entries(uint32_t count) {
   uint32_t e = 1;
-  while (e * HCK_BLOCK < count) e <<= 1;
+  while (e * BLOCK < count) e <<= 1;
   return e;
 }
 
-template <bool WIDE> __device__ __forceinline__ void sort_lds(const SortBuf<WIDE>& buf, uint32_t count) {
-  static_assert(ARGSORT_MAX == 16 * HCK_BLOCK, "entries per lane below assume 4096 entries and 256 lanes");
-  const uint32_t e = sort_entries(count);
-  if (e == 16) merge_sort_lds<WIDE, 16>(buf, count);
-  else if (e == 8) merge_sort_lds<WIDE, 8>(buf, count);
-  else if (e == 4) merge_sort_lds<WIDE, 4>(buf, count);
-  else if (e == 2) merge_sort_lds<WIDE, 2>(buf, count);
-  else merge_sort_lds<WIDE, 1>(buf, count);
+template <bool WIDE, uint32_t BLOCK> __device__ __forceinline__ void sort_lds(const SortBuf<WIDE>& buf, uint32_t count) {
+  static_assert(ARGSORT_MAX == 16 * HCK_BLOCK && (BLOCK == HCK_BLOCK || BLOCK == SORT_WIDE_BLOCK), "entries per lane below assume 4096 entries and 256 or 1024 lanes");
+  const uint32_t e = sort_entries<BLOCK>(count);
+  if constexpr (BLOCK == HCK_BLOCK) {
+    if (e == 16) return merge_sort_lds<WIDE, 16, BLOCK>(buf, count);
+    if (e == 8) return merge_sort_lds<WIDE, 8, BLOCK>(buf, count);
+  }
+  if (e == 4) merge_sort_lds<WIDE, 4, BLOCK>(buf, count);
+  else if (e == 2) merge_sort_lds<WIDE, 2, BLOCK>(buf, count);
+  else merge_sort_lds<WIDE, 1, BLOCK>(buf, count);
 }
 
 // descending order = ascending order of the inverted key
@@ -376,7 +383,7 @@ template <typename C> __device__ __forceinline__ uint64_t key_flip(uint32_t desc
   return descending ? ((sizeof(C) == 8) ? ~0ull : 0xffffffffull) : 0ull;
 }
 
-template <typename T> __device__ __forceinline__ void argsort_impl(const hck_scan_args& p) {
+template <typename T, uint32_t BLOCK> __device__ __forceinline__ void argsort_impl(const hck_scan_args& p) {
   typedef typename Arith<T>::type C;
   constexpr bool WIDE = sizeof(C) == 8;
   __shared__ uint64_t keys[SORT_SLOTS];
@@ -400,14 +407,14 @@ template <typename T> __device__ __forceinline__ void argsort_impl(const hck_sca
     out[(size_t)place[0] * p.inner] = (int64_t)t;
     return;
   }
-  const uint32_t N = sort_entries(p.reduce) * HCK_BLOCK;
-  for (uint32_t t = threadIdx.x; t < N; t += HCK_BLOCK) {
+  const uint32_t N = sort_entries<BLOCK>(p.reduce) * BLOCK;
+  for (uint32_t t = threadIdx.x; t < N; t += BLOCK) {
     if (t < p.reduce) buf.put(t, sort_key((C)to_arith(in[(size_t)t * p.inner])) ^ flip, t);
     else buf.pad(t);
   }
   __syncthreads();
-  sort_lds<WIDE>(buf, p.reduce);
-  for (uint32_t t = threadIdx.x; t < p.reduce; t += HCK_BLOCK) out[(size_t)t * p.inner] = (int64_t)buf.idx(t);
+  sort_lds<WIDE, BLOCK>(buf, p.reduce);
+  for (uint32_t t = threadIdx.x; t < p.reduce; t += BLOCK) out[(size_t)t * p.inner] = (int64_t)buf.idx(t);
 }
 
 // Which line, and which of its `parts` pieces, block `l` takes. Blocks go to the eight XCDs round robin in launch order, each
@@ -427,7 +434,7 @@ __device__ __forceinline__ void line_on_xcd(uint32_t l, uint32_t parts, uint32_t
 
 // Long axes, pass 1: block (line, chunk) sorts elements [chunk * ARGSORT_MAX, ...) of its line
 // and stores the sorted run: keys (32 bits, or 64 for int64 tensors) and indices.
-template <typename T, typename K> __device__ __forceinline__ void argsort_chunks_impl(const hck_sort_args& p) {
+template <typename T, typename K, uint32_t BLOCK> __device__ __forceinline__ void argsort_chunks_impl(const hck_sort_args& p) {
   typedef typename Arith<T>::type C;
   constexpr bool WIDE = sizeof(C) == 8;
   static_assert(sizeof(K) == sizeof(C), "keys have the size of the arithmetic type");
@@ -442,14 +449,14 @@ template <typename T, typename K> __device__ __forceinline__ void argsort_chunks
   const uint32_t first = chunk * ARGSORT_MAX;
   const uint32_t count = p.reduce - first < ARGSORT_MAX ? p.reduce - first : ARGSORT_MAX;
   const uint64_t flip = key_flip<C>(p.descending);
-  for (uint32_t t = threadIdx.x; t < ARGSORT_MAX; t += HCK_BLOCK) {
+  for (uint32_t t = threadIdx.x; t < ARGSORT_MAX; t += BLOCK) {
     if (t < count) buf.put(t, sort_key((C)to_arith(in[(size_t)(first + t) * p.inner])) ^ flip, first + t);
     else buf.pad(t);
   }
   __syncthreads();
-  sort_lds<WIDE>(buf, count);
+  sort_lds<WIDE, BLOCK>(buf, count);
   const size_t dst = (size_t)line * p.reduce + first;
-  for (uint32_t t = threadIdx.x; t < count; t += HCK_BLOCK) {
+  for (uint32_t t = threadIdx.x; t < count; t += BLOCK) {
     ((K*)p.keys_out)[dst + t] = (K)buf.key(t);
     p.idx_out[dst + t] = buf.idx(t);
   }
@@ -540,9 +547,13 @@ DEF_RANK(2)
 DEF_RANK(4)
 DEF_RANK(8)
 
-HC_KERNEL void hc_argsort_chunks_f32(hck_sort_args p) { argsort_chunks_impl<float, uint32_t>(p); }
-HC_KERNEL void hc_argsort_chunks_f16(hck_sort_args p) { argsort_chunks_impl<half_t, uint32_t>(p); }
-HC_KERNEL void hc_argsort_chunks_i64(hck_sort_args p) { argsort_chunks_impl<int64_t, uint64_t>(p); }
-HC_KERNEL void hc_argsort_f32(hck_scan_args p) { argsort_impl<float>(p); }
-HC_KERNEL void hc_argsort_f16(hck_scan_args p) { argsort_impl<half_t>(p); }
-HC_KERNEL void hc_argsort_i64(hck_scan_args p) { argsort_impl<int64_t>(p); }
+#define DEF_ARGSORT(T, TN, K)                                                                                                   \
+  HC_KERNEL void hc_argsort_chunks_##TN(hck_sort_args p) { argsort_chunks_impl<T, K, HCK_BLOCK>(p); }                           \
+  HC_KERNEL void hc_argsort_##TN(hck_scan_args p) { argsort_impl<T, HCK_BLOCK>(p); }                                            \
+  extern "C" __global__ __launch_bounds__(SORT_WIDE_BLOCK) void hc_argsort_chunks_wide_##TN(hck_sort_args p) {                  \
+    argsort_chunks_impl<T, K, SORT_WIDE_BLOCK>(p);                                                                              \
+  }                                                                                                                             \
+  extern "C" __global__ __launch_bounds__(SORT_WIDE_BLOCK) void hc_argsort_wide_##TN(hck_scan_args p) { argsort_impl<T, SORT_WIDE_BLOCK>(p); }
+DEF_ARGSORT(float, f32, uint32_t)
+DEF_ARGSORT(half_t, f16, uint32_t)
+DEF_ARGSORT(int64_t, i64, uint64_t)
