@@ -2254,7 +2254,8 @@ extern "C" int hc_log_softmax(hc_ctx* ctx, int dtype, const void* in, void* out,
   const bool few_long_rows = inner == 1 && (uint64_t)outer < 2 * (uint64_t)ctx->props.multiProcessorCount && reduce >= 32768;
   OpNote note({in}, {out});
   auto tag_rows = [&](int lanes) {   // rows held in the registers of a team of `lanes` lanes
-    if (reduce % (int64_t)(16 / el_size) != 0) return;
+    // (fp16 rows of 8 lanes only as whole vectors: of 256 ragged halfs a lane would load 32 one by one)
+    if (reduce % (int64_t)(16 / el_size) != 0 && dtype == HC_F16 && lanes == 8) return;
     note.tag = hc_pending::LOG_SOFTMAX;
     note.meta.dtype = dtype;
     note.meta.rows = (uint64_t)outer;

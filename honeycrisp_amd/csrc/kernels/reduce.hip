@@ -601,30 +601,24 @@ HC_KERNEL void hc_log_softmax_rows256x8_f16(hck_reduce_args p) { log_softmax_row
 // The chain [x * scale] [+ mask] -> logSoftmax [-> exp] (an attention softmax as a Honeycrisp
 // model writes it) in one pass over rows that fit the team's registers: the arithmetic of the
 // separate kernels, with every intermediate rounded to T where they would have stored it.
-template <typename T, int LANES> __device__ __forceinline__ void softmax_chain_rows_impl(const hck_softmax_chain_args& p) {
+// Row: RowRegs, or RaggedRow for rows that are no whole number of 16-byte vectors (24 x [201, 201] fp32:
+// the four launches 2.7, 4.4, 5.6 and 2.8 us and the gaps between them; six times in a forward pass of a model, 876 -> 817 us). Bound by the latency of the two
+// reductions and by memory.
+template <typename T, int LANES, typename Row> __device__ __forceinline__ void softmax_chain_rows_impl(const hck_softmax_chain_args& p) {
   __shared__ float lds[HCK_BLOCK / 64];
   const uint32_t lane = Team<LANES>::lane(), row = Team<LANES>::row();
   if (row >= p.outer) return;
   const uint32_t n = p.reduce;
-  constexpr int VEC = RowRegs<T, LANES>::VEC, CHUNKS = RowRegs<T, LANES>::CHUNKS;
-  RowRegs<T, LANES> r;
+  Row r;
   r.load((const T*)p.in + (size_t)row * n, n, lane);
   if (p.flags & HCK_SM_SCALE) {
     const float s = p.scale;
-#pragma unroll
-    for (int c = 0; c < CHUNKS; c++)
-#pragma unroll
-      for (int i = 0; i < VEC; i++) r.v[c][i] = narrow<T>((float)r.v[c][i] * s);
+    r.update(n, lane, [&](float x) { return narrow<T>(x * s); });
   }
   if (p.flags & HCK_SM_MASK) {
-    RowRegs<T, LANES> m;
+    Row m;
     m.load((const T*)p.mask + (size_t)(row % p.mask_rows) * n, n, lane);
-#pragma unroll
-    for (int c = 0; c < CHUNKS; c++)
-      if ((lane + LANES * c) * VEC < n) {
-#pragma unroll
-        for (int i = 0; i < VEC; i++) r.v[c][i] = narrow<T>((float)r.v[c][i] + (float)m.v[c][i]);
-      }
+    r.update2(n, lane, m, [&](float x, float y) { return narrow<T>(x + y); });
   }
   float mx = -INFINITY;
   r.each(n, lane, [&](float x) { if (x > mx) mx = x; });
@@ -642,10 +636,13 @@ template <typename T, int LANES> __device__ __forceinline__ void softmax_chain_r
     return (sizeof(T) == 2 ? exp_hw(stored) : expf(stored)) * 1.0f;
   });
 }
-HC_KERNEL void hc_softmax_chain_rows_f32(hck_softmax_chain_args p) { softmax_chain_rows_impl<float, 64>(p); }
-HC_KERNEL void hc_softmax_chain_rows8_f32(hck_softmax_chain_args p) { softmax_chain_rows_impl<float, 8>(p); }
-HC_KERNEL void hc_softmax_chain_rows_f16(hck_softmax_chain_args p) { softmax_chain_rows_impl<half_t, 64>(p); }
-HC_KERNEL void hc_softmax_chain_rows8_f16(hck_softmax_chain_args p) { softmax_chain_rows_impl<half_t, 8>(p); }
+HC_KERNEL void hc_softmax_chain_rows_f32(hck_softmax_chain_args p) { softmax_chain_rows_impl<float, 64, RowRegs<float, 64>>(p); }
+HC_KERNEL void hc_softmax_chain_ragged_rows_f32(hck_softmax_chain_args p) { softmax_chain_rows_impl<float, 64, RaggedRow<float, 64>>(p); }
+HC_KERNEL void hc_softmax_chain_rows8_f32(hck_softmax_chain_args p) { softmax_chain_rows_impl<float, 8, RowRegs<float, 8>>(p); }
+HC_KERNEL void hc_softmax_chain_ragged_rows8_f32(hck_softmax_chain_args p) { softmax_chain_rows_impl<float, 8, RaggedRow<float, 8>>(p); }
+HC_KERNEL void hc_softmax_chain_rows_f16(hck_softmax_chain_args p) { softmax_chain_rows_impl<half_t, 64, RowRegs<half_t, 64>>(p); }
+HC_KERNEL void hc_softmax_chain_ragged_rows_f16(hck_softmax_chain_args p) { softmax_chain_rows_impl<half_t, 64, RaggedRow<half_t, 64>>(p); }
+HC_KERNEL void hc_softmax_chain_rows8_f16(hck_softmax_chain_args p) { softmax_chain_rows_impl<half_t, 8, RowRegs<half_t, 8>>(p); }
 
 // logSoftmaxGrad (BackendCPU.swift:1040-1085): g - sum(g) * softmax(x), with exponentials relative to the maximum that are scaled by
 // sum(g) / sum(exp) at the end (exponentials of x - logf(sum) - max would lose the digits of a long logarithm). An fp32 row in

@@ -99,6 +99,15 @@ template <typename T, int LANES, int NCHUNKS = 4> struct RowRegs {
         for (int i = 0; i < VEC; i++) v[c][i] = f((float)v[c][i]);
       }
   }
+  // x = f(x, y), y the element of `other` in the same place
+  template <typename F> __device__ __forceinline__ void update2(uint32_t n, uint32_t lane, const RowRegs& other, F f) {
+#pragma unroll
+    for (int c = 0; c < CHUNKS; c++)
+      if ((lane + LANES * c) * VEC < n) {
+#pragma unroll
+        for (int i = 0; i < VEC; i++) v[c][i] = f((float)v[c][i], (float)other.v[c][i]);
+      }
+  }
   template <typename F> __device__ __forceinline__ void store(T* row, uint32_t n, uint32_t lane, F f) const {
 #pragma unroll
     for (int c = 0; c < CHUNKS; c++) {
@@ -123,6 +132,38 @@ template <typename T, int LANES, int NCHUNKS = 4> struct RowRegs {
         store_vec<T, VEC>(row, k, o);
       }
     }
+  }
+};
+
+// The same for rows of any length: lane l owns the elements l, l + LANES, ..., the order in which a streamed ragged row is
+// visited. Up to as many elements as RowRegs holds; loads and stores of single elements, a wave's side by side.
+template <typename T, int LANES> struct RaggedRow {
+  static constexpr int COUNT = 4 * VecWidth<T>::value;
+  T v[COUNT];
+  __device__ __forceinline__ void load(const T* row, uint32_t n, uint32_t lane) {
+#pragma unroll
+    for (int i = 0; i < COUNT; i++)
+      if (lane + LANES * i < n) v[i] = row[lane + LANES * i];
+  }
+  template <typename F> __device__ __forceinline__ void each(uint32_t n, uint32_t lane, F f) const {
+#pragma unroll
+    for (int i = 0; i < COUNT; i++)
+      if (lane + LANES * i < n) f((float)v[i]);
+  }
+  template <typename F> __device__ __forceinline__ void update(uint32_t n, uint32_t lane, F f) {
+#pragma unroll
+    for (int i = 0; i < COUNT; i++)
+      if (lane + LANES * i < n) v[i] = f((float)v[i]);
+  }
+  template <typename F> __device__ __forceinline__ void update2(uint32_t n, uint32_t lane, const RaggedRow& other, F f) {
+#pragma unroll
+    for (int i = 0; i < COUNT; i++)
+      if (lane + LANES * i < n) v[i] = f((float)v[i], (float)other.v[i]);
+  }
+  template <typename F> __device__ __forceinline__ void store(T* row, uint32_t n, uint32_t lane, F f) const {
+#pragma unroll
+    for (int i = 0; i < COUNT; i++)
+      if (lane + LANES * i < n) row[lane + LANES * i] = narrow<T>(f((float)v[i]));
   }
 };
 
