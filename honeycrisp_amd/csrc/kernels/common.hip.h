@@ -307,11 +307,17 @@ __device__ __forceinline__ const void* gemm_epilogue_operand(const hck_gemm_args
 }
 
 // One 16-byte piece of C (row `row`, columns col .. col + 16 / sizeof(T) - 1) leaves a tiled GEMM
-// kernel; `staged` is where the piece sits in LDS. Edge kernels skip pieces outside C. LOOSE (the
-// edge kernels of the ordinary build): a row of C may start at any element (in the access mode the
+// kernel; `staged` is where the piece sits in LDS. Edge kernels skip pieces outside C. LOOSE (see
+// gemm_loose_stores): a row of C may start at any element (in the access mode the
 // runtime sets, multi-dword stores need no alignment), and the piece that straddles N leaves
 // element by element, in a loop that stays rolled (it runs for one piece per row at most and must
 // not cost the write-out registers). Without LOOSE, N is a whole number of pieces.
+// Edge kernels of the ordinary build take any N and any alignment of C; those of the second build (*_m) only with tiles of up to
+// 128 x 128 (batched products whose head swaps a recording folds into them): the larger ones have no registers left for it
+// (256 x 256: 136 bytes of scratch per lane against 96 to 128).
+template <bool EDGE, uint32_t BM, uint32_t BN> __device__ constexpr bool gemm_loose_stores() {
+  return EDGE && (!HC_GEMM_IS_MERGED || BM * BN <= 128 * 128);
+}
 template <typename T, typename Chunk16, bool EDGE, bool LOOSE>
 __device__ __forceinline__ void gemm_store_piece(T* dst, uint32_t row, uint32_t col, uint32_t M, uint32_t N, Chunk16 v,
                                                  const char* staged) {

@@ -560,7 +560,7 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
           const uint32_t piece = it * 64 + lane, r = piece / UNITS, u = piece % UNITS;
           const Chunk v = *reinterpret_cast<const Chunk*>(slab + r * RB + ((u ^ unit_swz(r)) * 16));
           const uint32_t row = m0 + wm + i * 32 + r, col = n0 + wn + u * (16 / ES);
-          gemm_store_piece<T, Chunk, EDGE, EDGE && !HC_GEMM_IS_MERGED>(C + (size_t)row * p.c_rs + col, row, col, p.M, p.N, v, slab + r * RB + ((u ^ unit_swz(r)) * 16));
+          gemm_store_piece<T, Chunk, EDGE, gemm_loose_stores<EDGE, BM, BN>()>(C + (size_t)row * p.c_rs + col, row, col, p.M, p.N, v, slab + r * RB + ((u ^ unit_swz(r)) * 16));
         }
       }
 #ifdef HC_GEMM_MERGED
