@@ -102,7 +102,7 @@ int hc_get_device_info(hc_ctx* ctx, hc_device_info* out);
  * other threads launch through the context (an entry point works on a copy it takes when it
  * starts). `value` NULL or "" restores the default; for the on/off switches anything but "0"
  * means on. Names: HCHIP_GEMM_TILE (general | <BM>x<BN>), HCHIP_GEMM_KERNEL (dma | dma2 | mi16 |
- * staged), HCHIP_GEMM_RING (4 | 2), HCHIP_GEMM_ONE (0), and the on/off switches
+ * ks | staged), HCHIP_GEMM_RING (4 | 2), HCHIP_GEMM_ONE (0), and the on/off switches
  * HCHIP_GEMM_NO_PEEL, HCHIP_GEMM_NO_DIRECT, HCHIP_GEMM_NO_REPITCH, HCHIP_GEMM_BAND,
  * HCHIP_NO_FUSION (looked at when a capture begins), HCHIP_RECORDING_LOG,
  * HCHIP_GRAPH_AS_LAUNCHES (both looked at when a capture ends). HC_ERR_INVALID for any other name. */
