@@ -8,7 +8,6 @@ ComparisonOp (Comparison.swift:4-28), BackendError (Backend.swift:6-16).
 """
 import enum
 import functools
-import math
 from dataclasses import dataclass
 from typing import Any, List, Sequence
 
@@ -138,11 +137,11 @@ class BackendError(Exception):
 
 
 def product(xs: Sequence[int]) -> int:
-    n = math.prod(xs)
-    if type(n) is not int:      # (numpy integers among them: their products wrap)
-        n = 1
-        for x in xs:
-            n *= int(x)
+    # (numpy integers become Python's before they are multiplied: their products wrap, or refuse a factor of more than 64 bits.
+    # One pass over xs, which may be an iterator. math.prod(map(int, xs)) takes 1.3 to 1.6 times as long.)
+    n = 1
+    for x in xs:
+        n *= x if type(x) is int else int(x)
     return n
 
 

@@ -1,5 +1,6 @@
 """What the front-end works out per call and keeps by value: strides, products, packed descriptors, scalars."""
 import ctypes
+import warnings
 
 import numpy as np
 import pytest
@@ -40,6 +41,12 @@ def test_products_and_strides():
     assert product([]) == 1 and product([3, 0, 5]) == 0
     wide = [np.int64(1 << 40), np.int64(1 << 40)]
     assert product(wide) == 1 << 80 and type(product(wide)) is int
+    # one pass, without warnings: iterators, factors beyond 64 bits, unsigned and narrow integers among Python's
+    assert product(iter([3, 4])) == product(np.int64(n) for n in (3, 4)) == 12
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")
+        assert product(wide) == 1 << 80 and product([np.int64(3), 1 << 70]) == 3 << 70
+        assert product(np.array([1 << 40, 1 << 40])) == 1 << 80 and product([np.int8(100), 100]) == product([np.uint64(100), np.int64(100)]) == 10000
     rng = np.random.default_rng(0)
     for _ in range(50):
         shape = [int(n) for n in rng.integers(0, 5, size=rng.integers(0, 7))]
