@@ -12,6 +12,16 @@
 #define HCK_MAX_DIMS 8
 #define HCK_BLOCK 256
 
+/* Tile that block `block` of a product with `total` tiles takes: block ids equal mod 8 run on one XCD (workgroups go to the
+ * eight round robin), and each XCD gets a contiguous band of tiles, the first total % 8 of them one tile more. */
+#ifdef __HIP__
+__host__ __device__
+#endif
+static inline uint32_t hck_band_tile(uint32_t block, uint32_t total) {
+  const uint32_t x = block & 7u, rest = total & 7u;
+  return x * (total >> 3) + (x < rest ? x : rest) + (block >> 3);
+}
+
 /* Joint broadcast descriptor for up to three operands after the host has dropped
  * size-1 axes and merged axes that are mergeable for every operand. The innermost
  * axis is split off: a thread handles `vec` consecutive inner elements, the rest of
@@ -356,7 +366,8 @@ typedef struct {
   uint64_t a_bs, b_bs, c_bs;
   uint32_t tiles_m, tiles_n;
   /* Tile order of the direct-to-LDS kernels. xcd_gn == 0: block ids equal mod 8 (one XCD)
-   * get a contiguous band of tiles. Otherwise the tile grid is cut into super-blocks of
+   * get a contiguous band of tiles (hck_band_tile), or, with xcd_sm != 0, every 8th tile (launch
+   * order). Otherwise the tile grid is cut into super-blocks of
    * (8/xcd_gn * xcd_sm) x (xcd_gn * xcd_sn) tiles, visited one after the other; inside one,
    * the 8 XCDs form an (8/xcd_gn) x xcd_gn grid and each owns xcd_sm x xcd_sn tiles. */
   uint32_t xcd_gn, xcd_sm, xcd_sn;

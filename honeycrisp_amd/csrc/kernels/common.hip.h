@@ -226,7 +226,9 @@ __device__ __forceinline__ V block_reduce(V v, Op op, V* lds /* >= 4 entries */)
 
 // Tile (tm, tn) of a GEMM block for the direct-to-LDS kernels. Block ids equal mod 8 run on one
 // XCD and share its L2: each XCD gets a compact rectangle of tiles (few distinct A and B panels)
-// inside a super-block, or, without the rectangle parameters, a contiguous band. The host only
+// inside a super-block, or, without the rectangle parameters, a contiguous band (also of a number of tiles that is no
+// multiple of 8: 4819 x 1600 x 321 in 228 tiles of 128 x 64, fp16, in launch order 19.2 us, in bands 13.8), or tiles in
+// launch order where that touches fewer panels. The host only
 // passes powers of two for xcd_gn, xcd_sm and xcd_sn, so their divisions are shifts; one real
 // division (by the number of super-blocks per row, or by tiles_n) remains.
 __device__ __forceinline__ void gemm_tile_of_block(const hck_gemm_args& p, uint32_t block, uint32_t& tm, uint32_t& tn) {
@@ -244,9 +246,7 @@ __device__ __forceinline__ void gemm_tile_of_block(const hck_gemm_args& p, uint3
     tn = (((sb_col << lg) + xn) << lsn) + ln;
     return;
   }
-  const uint32_t total = p.tiles_m * p.tiles_n;
-  uint32_t tile = block;
-  if ((total & 7u) == 0) tile = (block & 7u) * (total >> 3) + (block >> 3);
+  const uint32_t tile = p.xcd_sm != 0 ? block : hck_band_tile(block, p.tiles_m * p.tiles_n);
   tm = tile / p.tiles_n;
   tn = tile - tm * p.tiles_n;
 }

@@ -173,8 +173,7 @@ template <typename T, int ROWS, int MODE> struct KsOperand {
 
 // Workgroup -> tile: workgroups with equal number mod 8 run on one XCD; each XCD gets a contiguous band of tiles.
 __device__ __forceinline__ void ks_tile(const hck_gemm_args& p, uint32_t block, uint32_t& tm, uint32_t& tn) {
-  const uint32_t total = p.tiles_m * p.tiles_n, x = block & 7u, rest = total & 7u;
-  const uint32_t tile = x * (total >> 3) + (x < rest ? x : rest) + (block >> 3);
+  const uint32_t tile = hck_band_tile(block, p.tiles_m * p.tiles_n);
   tm = tile / p.tiles_n;
   tn = tile - tm * p.tiles_n;
 }

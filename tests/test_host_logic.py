@@ -67,6 +67,45 @@ def test_fast_division_constants_are_exact(tmp_path):
     assert " 0 wrong" in out.stdout
 
 
+BANDS = textwrap.dedent(r"""
+    #include <stdint.h>
+    #include <stdio.h>
+    #include <string.h>
+    #include "kargs.h"
+    int main(void) {
+      static unsigned char seen[5000];
+      for (uint32_t total = 1; total < 5000; total++) {
+        memset(seen, 0, sizeof(seen));
+        uint32_t end = 0, least = total, most = 0;   /* where the band of the XCD before ends */
+        for (uint32_t x = 0; x < 8 && x < total; x++) {
+          uint32_t n = 0;
+          for (uint32_t block = x; block < total; block += 8, n++) {
+            const uint32_t tile = hck_band_tile(block, total);
+            if (tile >= total || seen[tile]++ || tile != end + n) return printf("block %u of %u: tile %u\n", block, total, tile), 1;
+          }
+          end += n;
+          if (n < least) least = n;
+          if (n > most) most = n;
+        }
+        if (end != total || most - least > 1) return printf("%u tiles\n", total), 1;
+      }
+      return 0;
+    }
+""")
+
+
+@pytest.mark.skipif(shutil.which("gcc") is None, reason="needs gcc")
+def test_every_xcd_gets_a_contiguous_band_of_tiles(tmp_path):
+    """Block -> tile of the products (hck_band_tile): every tile once, the tiles of the block ids equal mod 8 side by side, and as many
+    for every XCD, also where the number of tiles is no multiple of 8."""
+    src = tmp_path / "bands.c"
+    src.write_text(BANDS)
+    exe = tmp_path / "bands"
+    subprocess.run(["gcc", "-O2", "-I", os.path.join(ROOT, "honeycrisp_amd", "csrc"), "-o", str(exe), str(src)], check=True)
+    out = subprocess.run([str(exe)], stdout=subprocess.PIPE, text=True)
+    assert out.returncode == 0, out.stdout
+
+
 def test_code_objects_hold_every_reduce_and_gemm_kernel_the_host_names():
     """The host builds kernel names from (form, op, dtype) at run time and looks them up in the
     embedded code objects; a family that was dropped from a source file would only show on a GPU.
