@@ -1,0 +1,37 @@
+"""Which kernel hc_matmul gives a product, either side of the lines of its rules, and the product's sums."""
+import numpy as np
+import pytest
+
+from honeycrisp_amd.descriptors import DType
+from honeycrisp_amd.tensor import Tensor
+from recorded_kernels import kernels_of
+
+pytestmark = pytest.mark.gpu
+
+NN, NT, TN, TT = (False, False), (False, True), (True, False), (True, True)
+
+
+def kernel_of(hip_backend, capfd, batch, m, k, n, layout=NN):
+    """Name of the one kernel that takes an fp16 product (batch 0: a single one), after its result was compared with 64-bit sums."""
+    rng = np.random.default_rng(m + k + n)
+    lead = (batch,) if batch else ()
+    a = (rng.standard_normal(lead + (m, k)) / np.sqrt(k)).astype(np.float16)
+    b = rng.standard_normal(lead + (k, n)).astype(np.float16)
+    store = lambda x, transposed: Tensor(data=np.ascontiguousarray(np.swapaxes(x, -1, -2) if transposed else x))
+    with hip_backend.use():
+        x, y = store(a, layout[0]), store(b, layout[1])
+        call = lambda: (Tensor.batchedMatmul if batch else Tensor.matmul)(x, layout[0], y, layout[1], False)
+        kernels = kernels_of(hip_backend, capfd, call)
+        got = call().numpy().astype(np.float64)
+    exact = a.astype(np.float64) @ b.astype(np.float64)
+    # K roundings of fp32 partial sums of at most the sum of magnitudes, then one to fp16
+    bound = (k + 8) * 2.0 ** -23 * (np.abs(a).astype(np.float64) @ np.abs(b).astype(np.float64)) + 2.0 ** -11 * np.abs(exact) + 2.0 ** -24
+    assert (np.abs(got - exact) <= bound).all()
+    assert len(kernels) == 1
+    return kernels[0]
+
+
+# The tiled kernels' single-slice variant takes it where an operand runs along K, unless both do and K ends within a 16-byte piece.
+@pytest.mark.parametrize("k,layout,splits", [(64, NN, False), (65, NN, True), (64, TN, True), (60, NT, True), (56, NT, False), (72, NT, True)], ids=str)
+def test_up_to_16_rows_with_a_k_of_one_slice(hip_backend, capfd, k, layout, splits):
+    assert ("_ks_" in kernel_of(hip_backend, capfd, 0, 16, k, 96, layout)) == splits
