@@ -35,3 +35,10 @@ def kernel_of(hip_backend, capfd, batch, m, k, n, layout=NN):
 @pytest.mark.parametrize("k,layout,splits", [(64, NN, False), (65, NN, True), (64, TN, True), (60, NT, True), (56, NT, False), (72, NT, True)], ids=str)
 def test_up_to_16_rows_with_a_k_of_one_slice(hip_backend, capfd, k, layout, splits):
     assert ("_ks_" in kernel_of(hip_backend, capfd, 0, 16, k, 96, layout)) == splits
+
+
+# 48, 16, 32 and 3 rows of a tile start at odd elements; an even K
+@pytest.mark.parametrize("k,n,layout,splits", [(341, 72, NT, True), (343, 72, NT, False), (4097, 72, NN, True), (513, 72, TT, False), (511, 72, TT, True),
+                                               (4097, 3, TT, True), (4098, 72, NT, True)], ids=str)
+def test_operands_along_k_whose_rows_start_at_odd_elements(hip_backend, capfd, k, n, layout, splits):
+    assert ("_ks_" in kernel_of(hip_backend, capfd, 0, 40, k, n, layout)) == splits
