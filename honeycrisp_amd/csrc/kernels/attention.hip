@@ -434,7 +434,8 @@ __device__ __forceinline__ void attention_softmax_ragged(const hck_attention_arg
 // arithmetic, about 16 instructions' time per score of which 8 are the two exponentials: 45 of the 74 us with the products
 // left out. The keys take 23 (every wave reads 32 bytes of 32 rows per load, 33 cycles of the address path; 128 KiB per
 // workgroup) and the values 12, hardly beside the softmax of the other workgroup (starting half of the workgroups later
-// changed nothing). Heads of 128 fit one workgroup per compute unit at T > 512.
+// changed nothing). Heads of 128 fit one workgroup per compute unit at T > 512, which the three launches beat (1.08 in the mean of
+// 191 shapes, up to 1.45: 7 heads of 1280 x 128 40.7 -> 59.2 us): not built for those.
 //   phase 1: wave w takes the keys 128 i + 32 w .. + 31 straight from memory into operand registers, the next ones on
 //            their way; scores to LDS, [32, T]
 //   phase 2: the row teams' chain in place; the first values are on their way into registers
@@ -770,17 +771,17 @@ template <int TMAX> __device__ __forceinline__ void attention_f32_impl(const hck
 HC_KERNEL void hc_attention_f16_t256(hck_attention_args p) { attention_impl<256, 8>(p); }
 HC_KERNEL void hc_attention_f16_t512(hck_attention_args p) { attention_impl<512, 64>(p); }
 HC_KERNEL void hc_attention_f32_t256(hck_attention_args p) { attention_f32_impl<256>(p); }
-#define DEF_ATTENTION_ROWS32(TMAX, LANES, OCC)                                                                            \
-  extern "C" __global__ __launch_bounds__(HCK_BLOCK, OCC) void hc_attention_f16_rows32_t##TMAX##_h32(hck_attention_args p) {   \
-    attention_rows32_impl<TMAX, LANES, 32>(p);                                                                            \
-  }                                                                                                                       \
-  extern "C" __global__ __launch_bounds__(HCK_BLOCK, OCC) void hc_attention_f16_rows32_t##TMAX##_h64(hck_attention_args p) {   \
-    attention_rows32_impl<TMAX, LANES, 64>(p);                                                                            \
-  }                                                                                                                       \
-  extern "C" __global__ __launch_bounds__(HCK_BLOCK, OCC) void hc_attention_f16_rows32_t##TMAX##_h128(hck_attention_args p) {  \
-    attention_rows32_impl<TMAX, LANES, 128>(p);                                                                           \
+#define DEF_ATTENTION_ROWS32(TMAX, LANES, HD, OCC)                                                                              \
+  extern "C" __global__ __launch_bounds__(HCK_BLOCK, OCC) void hc_attention_f16_rows32_t##TMAX##_h##HD(hck_attention_args p) {   \
+    attention_rows32_impl<TMAX, LANES, HD>(p);                                                                                \
   }
-DEF_ATTENTION_ROWS32(256, 8, 2)
-DEF_ATTENTION_ROWS32(512, 64, 2)
-DEF_ATTENTION_ROWS32(1024, 64, 2)
-DEF_ATTENTION_ROWS32(2048, 64, 1)
+DEF_ATTENTION_ROWS32(256, 8, 32, 2)
+DEF_ATTENTION_ROWS32(256, 8, 64, 2)
+DEF_ATTENTION_ROWS32(256, 8, 128, 2)
+DEF_ATTENTION_ROWS32(512, 64, 32, 2)
+DEF_ATTENTION_ROWS32(512, 64, 64, 2)
+DEF_ATTENTION_ROWS32(512, 64, 128, 2)
+DEF_ATTENTION_ROWS32(1024, 64, 32, 2)
+DEF_ATTENTION_ROWS32(1024, 64, 64, 2)
+DEF_ATTENTION_ROWS32(2048, 64, 32, 1)
+DEF_ATTENTION_ROWS32(2048, 64, 64, 1)

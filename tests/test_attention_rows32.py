@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 F16 = DType.float16
 # (heads, T, head width): one vector; 8 lanes per row up to 256 scores; a wave above, one to four vectors per lane
 SHAPES = [(300, 16, 32), (256, 24, 64), (130, 40, 64), (130, 64, 32), (100, 72, 128), (40, 248, 64), (32, 256, 128), (33, 264, 64),
-          (16, 512, 32), (16, 520, 128), (9, 1000, 64), (8, 1024, 64), (8, 1032, 32), (6, 1536, 64), (4, 2048, 64)]
+          (16, 512, 32), (17, 512, 128), (9, 1000, 64), (8, 1024, 64), (8, 1032, 32), (8, 1536, 64), (4, 2048, 64)]
 
 
 @pytest.mark.parametrize("heads,t,hd", SHAPES, ids=str)
@@ -64,3 +64,19 @@ def test_attention_that_leaves_compute_units_idle_stays_apart(hip_backend):
             return Tensor.batchedMatmul(p, False, v, False, False)
 
         check(hip_backend, attention, removed=2)
+
+
+# One workgroup per compute unit: heads of 128 above T = 512, and of 64 above 1024 where the rounds of blocks fill the device to less
+# than 0.75 on average (288 and 520 blocks against 588). The separate launches are faster there.
+@pytest.mark.parametrize("heads,t,hd,merged", [(16, 520, 128, False), (5, 2048, 128, False), (6, 1536, 64, False), (13, 1280, 64, False),
+                                               (16, 512, 128, True), (8, 1128, 32, True), (14, 1344, 64, True)], ids=str)
+def test_attention_with_one_workgroup_per_compute_unit(hip_backend, heads, t, hd, merged):
+    rng = np.random.default_rng(4)
+    with hip_backend.use():
+        q, k, v = (Tensor(data=rng.standard_normal((heads, t, hd)).astype(np.float32), dtype=F16) for _ in range(3))
+
+        def attention():
+            p = (Tensor.batchedMatmul(q, False, k, True, False) * 0.125).softmax()
+            return Tensor.batchedMatmul(p, False, v, False, False)
+
+        check(hip_backend, attention, removed=2 + (2 if merged else 0))
