@@ -42,3 +42,12 @@ def test_up_to_16_rows_with_a_k_of_one_slice(hip_backend, capfd, k, layout, spli
                                                (4097, 3, TT, True), (4098, 72, NT, True)], ids=str)
 def test_operands_along_k_whose_rows_start_at_odd_elements(hip_backend, capfd, k, n, layout, splits):
     assert ("_ks_" in kernel_of(hip_backend, capfd, 0, 40, k, n, layout)) == splits
+
+
+# The 16x16x32 pipeline where its 128 x 128 tile fits both extents, and where a long K's tiles are on the device at once: 176 of 256 x 128
+# and 257.
+@pytest.mark.parametrize("batch,m,k,n,mi16", [(130, 128, 1032, 127, True), (130, 65, 1032, 65, True), (130, 128, 1032, 64, False), (130, 64, 1032, 127, False),
+                                              (257, 130, 1025, 128, False), (176, 130, 1025, 128, True), (176, 130, 1025, 64, False),
+                                              (256, 130, 1023, 128, False), (130, 130, 1025, 129, True), (260, 66, 256, 72, True), (260, 66, 255, 72, False)])
+def test_pipeline_of_batches_of_few_columns(hip_backend, capfd, batch, m, k, n, mi16):
+    assert ("_mi16_" in kernel_of(hip_backend, capfd, batch, m, k, n)) == mi16
