@@ -51,3 +51,10 @@ def test_operands_along_k_whose_rows_start_at_odd_elements(hip_backend, capfd, k
                                               (256, 130, 1023, 128, False), (130, 130, 1025, 129, True), (260, 66, 256, 72, True), (260, 66, 255, 72, False)])
 def test_pipeline_of_batches_of_few_columns(hip_backend, capfd, batch, m, k, n, mi16):
     assert ("_mi16_" in kernel_of(hip_backend, capfd, batch, m, k, n)) == mi16
+
+
+# K of two to four 128-byte slices: 128 x 128 tiles, but not for slices of up to 8 tiles of 256 x 256 above K = 160
+@pytest.mark.parametrize("batch,m,k,n,tile", [(64, 168, 249, 968, "256x256"), (64, 168, 161, 968, "256x256"), (64, 168, 160, 968, "128x128"),
+                                              (36, 168, 249, 2100, "128x128")])
+def test_tiles_of_batches_with_a_short_k(hip_backend, capfd, batch, m, k, n, tile):
+    assert "_%s_" % tile in kernel_of(hip_backend, capfd, batch, m, k, n)
