@@ -4,6 +4,7 @@ Usage: python -m honeycrisp_amd.csrc.build   (or build_all() from Python)
 Outputs, all in this directory: build/*.hsaco (intermediate) and libhchip.so.
 """
 import os
+import re
 import subprocess
 import sys
 from concurrent.futures import ThreadPoolExecutor
@@ -95,6 +96,41 @@ def kernels_with_promoted_private_data(remarks, granule=8192):
     return bad
 
 
+def ks_lds_sizes(source, merged):
+    """LDS in bytes of every kernel that `source` (gemm_ks.hip) defines in the plain or the second build, by name without the _m: a partial tile of MT x (NT + 4) floats per wave,
+    and D stages (one less with both operands in them) of what goes through LDS, 64 bytes of K by the operand's rows: operands
+    contiguous along M / N, unless a lane's share of a row is 16 bytes."""
+    sizes = {}
+    for group, es, dtype, mt, nt, waves, depth in re.findall(r"^DEF_KS_(GROUP_)?TILE\((\w+), (f\d+), (\d+), (\d+), (\d+), (\d+), \d+\)", source, re.M):
+        if group and not merged:
+            continue
+        es, mt, nt, waves, depth = 2 if es == "half_t" else 4, int(mt), int(nt), int(waves), int(depth)
+        staged = lambda rows: 64 * rows if rows // 16 * es != 16 else 0
+        for a in "km":
+            for b in "kn":
+                slot = (staged(mt) if a == "m" else 0) + (staged(nt) if b == "n" else 0)
+                stages = depth - (a == "m" and b == "n")
+                for edge in ("", "_e"):
+                    sizes["hc_gemm_%s_ks_%dx%d_%s%s%s" % (dtype, mt, nt, a, b, edge)] = waves * (mt * (nt + 4) * 4 + stages * slot)
+    return sizes
+
+
+def ks_kernels_with_other_lds(remarks, sizes):
+    """What kernels_with_promoted_private_data looks for, in the kernels whose waves split K: names of those whose LDS size is not
+    the one in `sizes`, and of those that the remarks do not mention."""
+    bad, current, missing = [], None, set(sizes)
+    for line in remarks.splitlines():
+        if "Function Name:" in line:
+            current = line.split("Function Name:")[1].split()[0]
+        elif "LDS Size [bytes/block]:" in line:
+            size = int(line.split("LDS Size [bytes/block]:")[1].split()[0])
+            plain = current[:-2] if current.endswith("_m") else current
+            missing.discard(plain)
+            if size != sizes.get(plain):
+                bad.append("%s (%d bytes of LDS, not %s)" % (current, size, sizes.get(plain)))
+    return bad + ["%s (not in the remarks)" % n for n in sorted(missing)]
+
+
 def build_kernel(name, src, extra):
     out = os.path.join(BUILD_DIR, name + ".hsaco")
     # HCHIP_EXTRA_FLAGS: additional device-compile flags (kernel experiments, e.g. -DNAME=1)
@@ -105,7 +141,12 @@ def build_kernel(name, src, extra):
     if bad:
         os.remove(out)
         raise RuntimeError("%s: kernels that must not use scratch memory do: %s" % (src, ", ".join(bad)))
-    bad = kernels_with_promoted_private_data(remarks) if check and not name.startswith(("gemm_f16_fast", "gemm_ks")) else []
+    bad = []
+    if name.startswith("gemm_ks"):
+        with open(os.path.join(KERNEL_DIR, src)) as f:
+            bad = ks_kernels_with_other_lds(remarks, ks_lds_sizes(f.read(), name == "gemm_ks_m"))
+    elif check and name != "gemm_f16_fast":
+        bad = kernels_with_promoted_private_data(remarks)
     if bad:
         os.remove(out)
         raise RuntimeError("%s: private data was moved into LDS: %s" % (src, ", ".join(bad)))

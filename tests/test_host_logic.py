@@ -168,6 +168,43 @@ def test_build_refuses_register_tiled_kernels_that_use_scratch_memory():
     assert set(build.NO_SCRATCH) <= {name for name, _src, _flags in build.KERNELS}
 
 
+def test_code_objects_hold_every_kernel_whose_waves_split_k():
+    """Both builds: the plain kernels and those whose write-out applies merged operations."""
+    import itertools
+    build = os.path.join(ROOT, "honeycrisp_amd", "csrc", "build")
+    for image, suffix in (("gemm_ks", ""), ("gemm_ks_m", "_m")):
+        path = os.path.join(build, image + ".hsaco")
+        if not os.path.exists(path):
+            pytest.skip("code objects not built")
+        blob = open(path, "rb").read()
+        tiles = [("f16", "16x32"), ("f32", "16x32"), ("f32", "32x32"), ("f32", "32x64")] + ([("f16", "32x32")] if suffix else [])
+        for (dt, tile), lay, edge in itertools.product(tiles, ["kk", "kn", "mk", "mn"], ["", "_e"]):
+            name = "hc_gemm_%s_ks_%s_%s%s%s" % (dt, tile, lay, edge, suffix)
+            assert name.encode() + b"\0" in blob, name
+
+
+def test_build_compares_the_lds_of_kernels_whose_waves_split_k():
+    """Stages and partial tiles give these kernels LDS sizes of their own: one byte more is private data that the compiler moved there."""
+    from honeycrisp_amd.csrc import build
+    with open(os.path.join(build.KERNEL_DIR, "gemm_ks.hip")) as f:
+        source = f.read()
+    sizes = build.ks_lds_sizes(source, False)
+    assert len(sizes) == 4 * 4 * 2
+    second = build.ks_lds_sizes(source, True)      # with the tile of groups: two stages, of both operands one
+    assert len(second) == 5 * 4 * 2 and {n: second[n] for n in sizes} == sizes
+    assert second["hc_gemm_f16_ks_32x32_kn"] == second["hc_gemm_f16_ks_32x32_mn_e"] == 8 * 32 * 36 * 4 + 2 * 8 * 2048
+    # 8 waves: partial tiles of 16 x 36 floats, 5 stages of 64 x 32 bytes of B; 32 x 64: B's 16 bytes per lane stay in registers
+    assert sizes["hc_gemm_f16_ks_16x32_kk"] == 18432 and sizes["hc_gemm_f16_ks_16x32_kn_e"] == 18432 + 5 * 8 * 2048
+    assert sizes["hc_gemm_f32_ks_32x64_kn"] == 69632 and sizes["hc_gemm_f32_ks_32x32_mn"] == 18432 + 3 * 4 * 4096
+    remarks = lambda s: "\n".join("r: Function Name: %s [-R]\nr:     LDS Size [bytes/block]: %d [-R]" % kv for kv in s.items())
+    assert build.ks_kernels_with_other_lds(remarks(sizes), sizes) == []
+    assert build.ks_kernels_with_other_lds(remarks({n + "_m": b for n, b in second.items()}), second) == []
+    changed = dict(sizes, hc_gemm_f16_ks_16x32_mk=sizes["hc_gemm_f16_ks_16x32_mk"] + 24)
+    assert build.ks_kernels_with_other_lds(remarks(changed), sizes) == ["hc_gemm_f16_ks_16x32_mk (59416 bytes of LDS, not 59392)"]
+    del changed["hc_gemm_f16_ks_16x32_mk"]
+    assert build.ks_kernels_with_other_lds(remarks(changed), sizes) == ["hc_gemm_f16_ks_16x32_mk (not in the remarks)"]
+
+
 @pytest.mark.parametrize("rows,n,composed", [(1, 65536, False), (1, 65537, True), (31, 65536, False), (31, 131072, True), (32, 131071, True),
                                              (32, 98301, False), (32, 98304, False), (32, 131072, True), (40, 1 << 20, True), (64, 196608, False),
                                              (64, 262144, True), (64, 98305, True), (96, 524288, False), (128, 98305, True),
