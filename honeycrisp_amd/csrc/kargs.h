@@ -142,10 +142,11 @@ typedef struct {
 #define HCK_SM_MASK 2u
 #define HCK_SM_EXP 4u
 
-/* One attention head per workgroup column: out = softmax-chain(q k^T) v with 64-wide heads, fp16.
- * q, out: [T, 64] rows at row strides q_rs / o_rs; k: [T, 64] at k_rs; v: [T, 64] at v_rs (all
- * contiguous along the 64). Slice z of an operand starts at z * bs, or with bdiv != 0 at
- * (z / bdiv) * bs + (z % bdiv) * bs2 (heads that are an inner axis of [B, T, H, 64]). The chain
+/* One attention head per workgroup column: out = softmax-chain(q k^T) v, fp16 or fp32. The kernel fixes the
+ * width H of a head (32, 64 or 128) and how many query rows a workgroup takes (64 or 32).
+ * q, out: [T, H] rows at row strides q_rs / o_rs; k: [T, H] at k_rs; v: [T, H] at v_rs (all
+ * contiguous along the H). Slice z of an operand starts at z * bs, or with bdiv != 0 at
+ * (z / bdiv) * bs + (z % bdiv) * bs2 (heads that are an inner axis of [B, T, heads, H]). The chain
  * between the two products is that of hck_softmax_chain_args (flags, scale, mask, mask_rows: row
  * r of all batch * T score rows takes mask row r % mask_rows). */
 typedef struct {
@@ -154,7 +155,7 @@ typedef struct {
   const void* v;
   const void* mask;
   void* out;
-  uint32_t T;      /* queries = keys per head, a multiple of 64 */
+  uint32_t T;      /* queries = keys per head: a multiple of 64, or of 8 with 32 rows per workgroup */
   uint32_t bdiv;
   uint32_t q_rs, k_rs, v_rs, o_rs;
   uint64_t q_bs, q_bs2, k_bs, k_bs2, v_bs, v_bs2, o_bs, o_bs2;

@@ -44,7 +44,7 @@ __device__ __forceinline__ void lds_barrier() {
   asm volatile("" ::: "memory");
 }
 
-// Which head (z) and which block of 64 query rows (qb) a workgroup takes; grid.x = blocks per head, grid.y = heads.
+// Which head (z) and which block of query rows (qb; 64 rows, or 32 in attention_rows32_impl) a workgroup takes; grid.x = blocks per head, grid.y = heads.
 // Workgroups go to the eight XCDs round robin in launch order and every XCD has an L2 of its own: the blocks
 // of one head, which all read that head's keys and values, are given to workgroups 8 apart, so they run on
 // one XCD and the keys and values come from memory once. (Heads beyond the last whole group of 8: launch order.)

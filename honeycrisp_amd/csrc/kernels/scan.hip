@@ -264,7 +264,8 @@ __device__ __forceinline__ void count_before(const SortBuf<WIDE>& buf, uint32_t 
   }
 }
 
-// Merge sort of E entries per lane, E * 256 in all, of which the first `count` are wanted, then runs merged pairwise through
+// Merge sort of E entries per lane, E * BLOCK in all (E up to 16 with 256 lanes, up to 4 with 1024), of which the first `count`
+// are wanted, then runs merged pairwise through
 // LDS: a lane finds by bisection where the merge path crosses its first output and merges E entries from there, one LDS
 // read per entry. A level costs at most 13 + E dependent LDS reads (12 steps of the bisection at runs of 2048, the first entries
 // of the two runs) and two barriers, whatever the run length; a bitonic network needs log2(run) stages for the same merge

@@ -174,8 +174,10 @@ int hc_launch_host_func(hc_ctx* ctx, void (*fn)(void*), void* user);
  *      [cast ->] normalize -> [(gain + c) *, + bias] -> [cast]      one LayerNorm kernel
  *      [* s ->] [+ mask ->] logSoftmax -> [exp]                     one softmax kernel
  *      swap of two batch axes -> batchedMatmul -> swap back         read / written through strides
- *      q k^T -> that softmax kernel -> x v, 64-wide heads, T a
- *      multiple of 64 up to 512 (fp16) / 256 (fp32)                 one attention kernel
+ *      q k^T -> that softmax kernel -> x v                          one attention kernel
+ *        (64-wide heads, T a multiple of 64 up to 512 (fp16) / 256 (fp32); fp16 also T a multiple of 8 while
+ *        blocks of 32 rows number at least the compute units: heads of 32 up to T = 2048, of 128 up to 512, of 64 up
+ *        to 1024, or 2048 where the blocks fill at least 3/4 of the rounds they take)
  *      products of one shape over the same input (q, k, v)          one launch
  *      argmax | argmin over rows -> gather of those indices from
  *      the same tensor (Tensor.max / min / all / some)              one row kernel
