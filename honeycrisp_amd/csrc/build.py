@@ -101,15 +101,16 @@ def ks_lds_sizes(source, merged):
     and D stages (one less with both operands in them) of what goes through LDS, 64 bytes of K by the operand's rows: operands
     contiguous along M / N, unless a lane's share of a row is 16 bytes."""
     sizes = {}
-    for group, es, dtype, mt, nt, waves, depth in re.findall(r"^DEF_KS_(GROUP_)?TILE\((\w+), (f\d+), (\d+), (\d+), (\d+), (\d+), \d+\)", source, re.M):
+    for group, es, dtype, mt, nt, waves, depth, along_k in re.findall(
+            r"^DEF_KS_(GROUP_)?TILE(?:_M)?\((\w+), (f\d+), (\d+), (\d+), (\d+), (\d+), \d+(?:, (\d+), \d+)?\)", source, re.M):
         if group and not merged:
             continue
-        es, mt, nt, waves, depth = 2 if es == "half_t" else 4, int(mt), int(nt), int(waves), int(depth)
+        es, mt, nt, waves = 2 if es == "half_t" else 4, int(mt), int(nt), int(waves)
         staged = lambda rows: 64 * rows if rows // 16 * es != 16 else 0
         for a in "km":
             for b in "kn":
                 slot = (staged(mt) if a == "m" else 0) + (staged(nt) if b == "n" else 0)
-                stages = depth - (a == "m" and b == "n")
+                stages = int(along_k if merged and a == "k" and along_k else depth) - (a == "m" and b == "n")
                 for edge in ("", "_e"):
                     sizes["hc_gemm_%s_ks_%dx%d_%s%s%s" % (dtype, mt, nt, a, b, edge)] = waves * (mt * (nt + 4) * 4 + stages * slot)
     return sizes

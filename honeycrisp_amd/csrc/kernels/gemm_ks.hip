@@ -412,15 +412,29 @@ __device__ __forceinline__ void gemm_ks_impl(const hck_gemm_args& p, char* const
     KS_BODY(T, MT, NT, W, KS_DEPTH(D, AM, BMODE), AM, BMODE, true)                                                                     \
   }
 // (OCC: wavefronts per SIMD that the registers have to leave room for)
+#define DEF_KS_LAYOUTS(T, TN, MT, NT, W, D, OCC, AN, AM)     \
+  DEF_KS(T, TN, MT, NT, W, D, OCC, AN, AM, k, KS_K)          \
+  DEF_KS(T, TN, MT, NT, W, D, OCC, AN, AM, n, KS_MN)
 #define DEF_KS_TILE(T, TN, MT, NT, W, D, OCC)                \
-  DEF_KS(T, TN, MT, NT, W, D, OCC, k, KS_K, k, KS_K)         \
-  DEF_KS(T, TN, MT, NT, W, D, OCC, k, KS_K, n, KS_MN)        \
-  DEF_KS(T, TN, MT, NT, W, D, OCC, m, KS_MN, k, KS_K)        \
-  DEF_KS(T, TN, MT, NT, W, D, OCC, m, KS_MN, n, KS_MN)
+  DEF_KS_LAYOUTS(T, TN, MT, NT, W, D, OCC, k, KS_K)          \
+  DEF_KS_LAYOUTS(T, TN, MT, NT, W, D, OCC, m, KS_MN)
+// In the second build DM stages and room for OCCM wavefronts, where A is contiguous along K: a group of such products has up to four
+// times the workgroups of one product, so that a compute unit has several to run, and with two stages two of them run
+// side by side and hide each other's start and write-out (four stages: one, the registers). Groups of two to four 32 x 64 products
+// 0.77 to 1.0 of the time on four stages, 0.87 in the mean of 20 with A along K, single ones with a row added 0.92 to 1.0; 32 x 32 0.88 to
+// 1.01, 0.96 of 40: 3 x 925 x 328 x 280 16.0 -> 13.1 us, 2 x 119 x 1176 x 4024 39.2 -> 31.5, 4 x 47 x 552 x 3728 21.1 -> 19.9.
+// With A along M (1.0, up to 1.07) its LDS leaves room for one workgroup anyway.
+#ifdef HC_GEMM_MERGED
+#define DEF_KS_TILE_M(T, TN, MT, NT, W, D, OCC, DM, OCCM)    \
+  DEF_KS_LAYOUTS(T, TN, MT, NT, W, DM, OCCM, k, KS_K)        \
+  DEF_KS_LAYOUTS(T, TN, MT, NT, W, D, OCC, m, KS_MN)
+#else
+#define DEF_KS_TILE_M(T, TN, MT, NT, W, D, OCC, DM, OCCM) DEF_KS_TILE(T, TN, MT, NT, W, D, OCC)
+#endif
 DEF_KS_TILE(half_t, f16, 16, 32, 8, 5, 2)
 DEF_KS_TILE(float, f32, 16, 32, 8, 5, 2)
-DEF_KS_TILE(float, f32, 32, 32, 4, 4, 2)
-DEF_KS_TILE(float, f32, 32, 64, 8, 4, 2)
+DEF_KS_TILE_M(float, f32, 32, 32, 4, 4, 2, 2, 4)
+DEF_KS_TILE_M(float, f32, 32, 64, 8, 4, 2, 2, 4)
 // Only for groups of products, which the second build runs: on 16 x 32 tiles a group of three has three times as many workgroups, of
 // which a compute unit holds one (five stages), and runs them in rounds. This tile gives the same sums, twice the outputs per fetched
 // column of B, and its two stages leave room for two workgroups. 3 products of 35 x 512 x 2176 with a bias 14.7 -> 9.7 us (four stages:
