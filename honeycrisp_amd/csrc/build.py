@@ -101,14 +101,14 @@ def ks_lds_sizes(source, merged):
     and D stages (one less with both operands in them) of what goes through LDS, 64 bytes of K by the operand's rows: operands
     contiguous along M / N, unless a lane's share of a row is 16 bytes."""
     sizes = {}
-    for group, es, dtype, mt, nt, waves, depth, along_k in re.findall(
-            r"^DEF_KS_(GROUP_)?TILE(?:_M)?\((\w+), (f\d+), (\d+), (\d+), (\d+), (\d+), \d+(?:, (\d+), \d+)?\)", source, re.M):
+    for group, layouts, es, dtype, mt, nt, waves, depth, along_k in re.findall(
+            r"^DEF_KS_(GROUP_)?(TILE|TILE_M|KK)\((\w+), (f\d+), (\d+), (\d+), (\d+), (\d+), \d+(?:, (\d+), \d+)?\)", source, re.M):
         if group and not merged:
             continue
         es, mt, nt, waves = 2 if es == "half_t" else 4, int(mt), int(nt), int(waves)
         staged = lambda rows: 64 * rows if rows // 16 * es != 16 else 0
-        for a in "km":
-            for b in "kn":
+        for a in "k" if layouts == "KK" else "km":
+            for b in "k" if layouts == "KK" else "kn":
                 slot = (staged(mt) if a == "m" else 0) + (staged(nt) if b == "n" else 0)
                 stages = int(along_k if merged and a == "k" and along_k else depth) - (a == "m" and b == "n")
                 for edge in ("", "_e"):

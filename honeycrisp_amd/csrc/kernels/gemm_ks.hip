@@ -441,7 +441,13 @@ DEF_KS_TILE_M(float, f32, 32, 64, 8, 4, 2, 2, 4)
 // 11.8), of 16 x 3008 x 3904 25.0 -> 22.3.
 #ifdef HC_GEMM_MERGED
 #define DEF_KS_GROUP_TILE DEF_KS_TILE
+#define DEF_KS_GROUP_KK(T, TN, MT, NT, W, D, OCC) DEF_KS(T, TN, MT, NT, W, D, OCC, k, KS_K, k, KS_K)
 #else
 #define DEF_KS_GROUP_TILE(...)
+#define DEF_KS_GROUP_KK(...)
 #endif
 DEF_KS_GROUP_TILE(half_t, f16, 32, 32, 8, 2, 4)
+// Likewise for fp32 groups with both operands along K, whose loads of 16 rows' 64 bytes each bound the 32 x 64 tile: a third fewer per output.
+// A workgroup fills a compute unit's LDS, so only where the group is one round of them (use_group_tile_kernel). Against 32 x 64:
+// 2 x 238 x 3656 x 1968 102.5 -> 75.4 us, 3 x 43 x 2144 x 4264 51.9 -> 39.6; other layouts and more tiles gain nothing (0.97 to 1.18 in the mean).
+DEF_KS_GROUP_KK(float, f32, 64, 64, 8, 2, 2)

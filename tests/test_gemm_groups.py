@@ -44,3 +44,23 @@ def test_groups_take_a_larger_tile(hip_backend, capfd, dtype, tile, layout):
                 name = "hc_gemm_%s_ks_%s_%s%s_m" % (SHORT[dtype], tile if larger else "16x32", modes, edge)
                 assert kernels_of(hip_backend, capfd, program).count(name) == 1
                 check(hip_backend, program, removed=members * merged + members - 1)
+
+
+# 344 and 172 tiles of 64 x 64, a K either side of the line and one that ends within a block; B along N
+@pytest.mark.parametrize("K,members,tb,tile", [(448, 2, True, "64x64_kk"), (456, 2, True, "64x64_kk_e"), (440, 2, True, "32x64_kk_e"), (456, 4, True, "32x64_kk_e"),
+                                               (448, 2, False, "32x64_kn")], ids=str)
+def test_groups_along_k_take_tiles_of_64_by_64(hip_backend, capfd, K, members, tb, tile):
+    M, N = 104, 2696
+    rng = np.random.default_rng(8)
+    t = lambda *shape: Tensor(data=rng.standard_normal(shape).astype(np.float32))
+    with hip_backend.use():
+        x, ws = t(M, K), [t(N, K) if tb else t(K, N) for _ in range(members)]
+        rows, res = [t(N) for _ in range(members)], t(M, N)
+
+        def group(member):
+            outs = [member(Tensor.matmul(x, False, ws[i], tb, False), i) for i in range(members)]
+            return functools.reduce(lambda p, q: p * q, outs)
+
+        for program, merged in ((lambda: group(lambda h, i: h), 0), (lambda: group(lambda h, i: (h + rows[i]).gelu()), 2), (lambda: group(lambda h, i: res + h), 1)):
+            assert kernels_of(hip_backend, capfd, program).count("hc_gemm_f32_ks_%s_m" % tile) == 1
+            check(hip_backend, program, removed=members * merged + members - 1)

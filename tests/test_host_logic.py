@@ -193,7 +193,8 @@ def test_build_compares_the_lds_of_kernels_whose_waves_split_k():
     second = build.ks_lds_sizes(source, True)      # with the tile of groups: two stages, of both operands one
     # ... and with two stages instead of four in two more tiles, where A runs along K (one of them has B in LDS)
     fewer = {"hc_gemm_f32_ks_32x32_kn" + edge: 18432 + 2 * 4 * 2048 for edge in ("", "_e")}
-    assert len(second) == 5 * 4 * 2 and {n: second[n] for n in sizes} == dict(sizes, **fewer)
+    assert len(second) == 5 * 4 * 2 + 2 and {n: second[n] for n in sizes} == dict(sizes, **fewer)
+    assert second["hc_gemm_f32_ks_64x64_kk"] == 8 * 64 * 68 * 4      # (one layout)
     assert second["hc_gemm_f16_ks_32x32_kn"] == second["hc_gemm_f16_ks_32x32_mn_e"] == 8 * 32 * 36 * 4 + 2 * 8 * 2048
     # 8 waves: partial tiles of 16 x 36 floats, 5 stages of 64 x 32 bytes of B; 32 x 64: B's 16 bytes per lane stay in registers
     assert sizes["hc_gemm_f16_ks_16x32_kk"] == 18432 and sizes["hc_gemm_f16_ks_16x32_kn_e"] == 18432 + 5 * 8 * 2048
