@@ -282,8 +282,12 @@ typedef struct {
   uint32_t n_src, n_dst;
   uint32_t row_vecs;       /* 16-byte vectors per row */
   uint32_t total_src;      /* outer * n_src */
+  uint32_t n_buckets;      /* outer * n_dst */
+  uint32_t list_rows;      /* hc_scatter_rows_lists: destination rows of a workgroup, at most HCK_SCATTER_LIST_ROWS */
+  int64_t* starts_out;     /* hc_scatter_rows_lists: `starts`, to be written */
   hck_bcast idx;           /* operand 0 = index offset for a flat source row, vec = 1 */
 } hck_scatter_rows_args;
+#define HCK_SCATTER_LIST_ROWS 1024
 
 /* Element gather: general index map over the flat output index. */
 typedef struct {

@@ -148,6 +148,92 @@ HC_KERNEL void hc_scatter_rows_fill(hck_scatter_rows_args p) {
   p.list[p.starts[bucket] + (int64_t)slot] = r;
 }
 
+// Passes 1 and 2 and the scan between them in one launch (up to the host's number of source rows): every workgroup owns `list_rows`
+// consecutive destination rows and reads all indices, so that it finds where its slices of `list` begin without a word from the others. It is
+// bound by those reads, 8 bytes per source row and workgroup from L2, and for few rows by its launch and three barriers. The whole scatter of rows of
+// 1 KiB, in us, with counters cleared, counted, scanned (two launches) and filled instead / now: 256 rows into 8192 20.2 / 9.6, 2048 into
+// 8192 21.9 / 11.2, 65536 into 32000 53.9 / 42.9 (eight loads in flight; one at a time 50.3), 786432 into 4000 231 / 229. Row numbers wait in LDS for the
+// scan; a workgroup with more than SCATTER_HELD_ROWS of them reads the indices again instead.
+constexpr uint32_t SCATTER_LISTS_BLOCK = 1024, SCATTER_HELD_ROWS = 8192;
+extern "C" __global__ __launch_bounds__(SCATTER_LISTS_BLOCK) void hc_scatter_rows_lists(hck_scatter_rows_args p) {
+  __shared__ uint32_t count[HCK_SCATTER_LIST_ROWS], held[SCATTER_HELD_ROWS], sums[SCATTER_LISTS_BLOCK / 64 + 1], n_held;
+  __shared__ uint16_t held_row[SCATTER_HELD_ROWS];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint64_t first = (uint64_t)blockIdx.x * p.list_rows, rows = p.n_buckets - first < p.list_rows ? p.n_buckets - first : p.list_rows;
+  if (tid < HCK_SCATTER_LIST_ROWS) count[tid] = 0;
+  if (tid == 0) n_held = 0;
+  __syncthreads();
+
+  uint32_t before = 0;   // source rows of the destinations in front of this workgroup's
+  auto visit = [&](auto&& f) {
+    const bool dense = p.idx.n_outer == 0 && p.idx.inner_stride[0] == 1 && p.n_src == p.total_src;   // (wave-uniform)
+    if (dense) {
+      constexpr uint32_t STEP = SCATTER_LISTS_BLOCK * 2;   // 16 bytes per lane, eight loads in flight
+      uint32_t r = tid * 2;
+      for (; r + 7 * STEP + 1 < p.total_src; r += 8 * STEP) {
+        int64_t id[8][2];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; u++) load_vec_loose<int64_t, 2>(p.indices + r + u * STEP, id[u]);
+#pragma unroll
+        for (uint32_t u = 0; u < 8; u++) f(r + u * STEP, (uint64_t)id[u][0]), f(r + u * STEP + 1, (uint64_t)id[u][1]);
+      }
+      for (; r + 1 < p.total_src; r += STEP) {
+        int64_t id[2];
+        load_vec_loose<int64_t, 2>(p.indices + r, id);
+        f(r, (uint64_t)id[0]), f(r + 1, (uint64_t)id[1]);
+      }
+      if (r < p.total_src) f(r, (uint64_t)p.indices[r]);
+    } else {
+      for (uint32_t r = tid; r < p.total_src; r += SCATTER_LISTS_BLOCK) {
+        uint32_t off[1];
+        size_t unused;
+        bcast_offsets<1, 1>(p.idx, r, off, unused);
+        f(r, (uint64_t)(r / p.n_src) * p.n_dst + (uint64_t)p.indices[off[0]]);
+      }
+    }
+  };
+  visit([&](uint32_t r, uint64_t bucket) {
+    if (bucket < first) before++;
+    const uint64_t mine = bucket - first;
+    if (mine < rows) {
+      atomicAdd(&count[mine], 1u);
+      const uint32_t slot = atomicAdd(&n_held, 1u);
+      if (slot < SCATTER_HELD_ROWS) held[slot] = r, held_row[slot] = (uint16_t)mine;
+    }
+  });
+  before = wave_reduce(before, SumOp{});
+  if (lane == 0) sums[wave] = before;
+  __syncthreads();
+  uint32_t base = 0;
+  for (uint32_t w = 0; w < SCATTER_LISTS_BLOCK / 64; w++) base += sums[w];
+  // exclusive scan of the counts, a row per thread
+  const uint32_t mine = tid < rows ? count[tid] : 0;
+  uint32_t up = mine;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t v = __shfl_up(up, o, 64);
+    if (lane >= (uint32_t)o) up += v;
+  }
+  __syncthreads();
+  if (lane == 63) sums[wave] = up;
+  __syncthreads();
+  for (uint32_t w = 0; w < wave; w++) base += sums[w];
+  const uint32_t start = base + up - mine;
+  if (tid < rows) {
+    p.counts[first + tid] = mine;
+    p.starts_out[first + tid] = start;
+    count[tid] = start;
+  }
+  __syncthreads();
+  if (n_held <= SCATTER_HELD_ROWS) {
+    for (uint32_t t = tid; t < n_held; t += SCATTER_LISTS_BLOCK) p.list[atomicAdd(&count[held_row[t]], 1u)] = held[t];
+  } else {
+    visit([&](uint32_t r, uint64_t bucket) {
+      if (bucket - first < rows) p.list[atomicAdd(&count[bucket - first], 1u)] = r;
+    });
+  }
+}
+
 // Ascending sort of n distinct values by the whole workgroup: a bitonic network whose
 // comparators all point the same way (each merge starts with a mirrored stage), so positions
 // past n behave as +infinity and n need not be a power of two. Works on LDS or global memory.
