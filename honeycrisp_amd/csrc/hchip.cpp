@@ -2220,9 +2220,12 @@ extern "C" int hc_argsort(hc_ctx* ctx, int dtype, const void* in, void* out, int
   k.inner = (uint32_t)inner;
   k.reverse = descending != 0;
   char name[64];
-  const bool wide = wide_sort(ctx, (uint64_t)outer * (uint64_t)inner, (uint64_t)reduce);
-  snprintf(name, sizeof(name), "hc_argsort%s_%s", wide ? "_wide" : "", dtype_name(dtype));
-  return launch(ctx, name, (uint64_t)outer * (uint64_t)inner, 1, &k, sizeof(k), wide ? 1024 : HCK_BLOCK);
+  const uint64_t lines = (uint64_t)outer * (uint64_t)inner;
+  const bool wide = wide_sort(ctx, lines, (uint64_t)reduce);
+  // (the radix sort, 32-bit keys only: wide blocks, and those of 256 lanes with more than half of an entry per lane)
+  const bool radix = !wide && dtype != HC_I64 && reduce > 128 && reduce <= 512 && lines <= (uint64_t)ctx->props.multiProcessorCount;
+  snprintf(name, sizeof(name), "hc_argsort%s_%s", wide ? "_wide" : radix ? "_radix" : "", dtype_name(dtype));
+  return launch(ctx, name, lines, 1, &k, sizeof(k), wide ? 1024 : HCK_BLOCK);
 }
 
 // Whether the rows go to the logSoftmax kernels whose blocks hold 8 vectors of 16 bytes per lane: rows of whole vectors,

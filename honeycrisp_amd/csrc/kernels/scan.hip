@@ -209,10 +209,10 @@ __device__ __forceinline__ uint64_t sort_key(float x) {
 __device__ __forceinline__ uint64_t sort_key(int64_t x) { return (uint64_t)x ^ 0x8000000000000000ull; }
 
 constexpr int ARGSORT_MAX = 4096;
-// Lanes of a sorting block while there are no more blocks than compute units. What bounds a block alone is the chain of dependent
-// LDS reads: 26 per level and 8 levels with 16 entries per lane, 13 per level and 10 levels with 4. us, 256 lanes / 1024: 8 lines of
-// 600 fp32 11.1 / 9.9, of 1025 15.4 / 12.8, of 4096 24.8 / 19.8 (int64 34.9 / 25.7), of 50257 47.7 / 42.0; 256 lines of 4096 26.6 / 21.6,
-// but 512 33.0 / 33.4 and 1024 45.2 / 58.7, where blocks share a unit; 512 entries and fewer 7.6 / 8.2.
+// Lanes of a sorting block while there are no more blocks than compute units. What bounds a block alone that merges (int64; 32-bit keys have the
+// radix sort there) is the chain of dependent LDS reads: 26 per level and 8 levels with 16 entries per lane, 13 per level and 10 levels with 4. us,
+// 256 lanes / 1024: 8 lines of 4096 int64 34.9 / 25.7, and of fp32, merged, 256 lines of 4096 26.6 / 21.6, but 512 33.0 / 33.4 and 1024
+// 45.2 / 58.7, where blocks share a unit; 512 entries and fewer 7.6 / 8.2.
 constexpr uint32_t SORT_WIDE_BLOCK = 1024;
 
 // What the block sort orders. Keys of 32 significant bits (floats, halfs) travel with their
@@ -377,6 +377,118 @@ template <bool WIDE, uint32_t BLOCK> __device__ __forceinline__ void sort_lds(co
   if (e == 4) merge_sort_lds<WIDE, 4, BLOCK>(buf, count);
   else if (e == 2) merge_sort_lds<WIDE, 2, BLOCK>(buf, count);
   else merge_sort_lds<WIDE, 1, BLOCK>(buf, count);
+}
+
+// ---- Lines and chunks of 32-bit keys, blocks alone on their compute unit: radix sort of up to four entries per lane.
+// A pass of 8 bits: a wave finds, entry by entry, the lanes with the same digit (a ballot per bit), which gives an entry its place among
+// its wave's; the block sums up the counts of digits and waves; the entries move through LDS. Four passes for fp32, three for fp16 whatever the
+// length, where merging takes ten levels of 13 dependent LDS reads. With four entries bound by the vector ALU (45 operations per entry and pass),
+// with one by the latencies of four barriers. us, merged / now: 256 lines of 4096 fp32 21.6 / 17.4, fp16 21.9 / 13.4, of 1500 15.0 / 10.7, 8 of
+// 1000 10.4 / 7.7, of 50257 (with the merging of 13 runs) 42.7 / 39.0, 256 of 300 (256 lanes) 7.5 / 6.6, of 128 4.9 / 5.2. Blocks that share
+// a unit keep merging (1024 lines of 4096 44.8 / 60.4, of 512 11.9 / 12.7).
+
+// Inclusive sum over the lanes of a wave: six DPP additions, no LDS.
+__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 (rows of 16 lanes)
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
+template <uint32_t BLOCK> struct RadixLds {
+  static constexpr uint32_t WAVES = BLOCK / 64, PITCH = 257;   // (counters of a digit in different banks)
+  static constexpr uint32_t ENTRIES = BLOCK == SORT_WIDE_BLOCK ? ARGSORT_MAX : 2 * BLOCK;
+  uint32_t keys[ENTRIES], counts[WAVES * PITCH], sums[WAVES];
+  uint16_t idxs[ENTRIES];
+};
+
+// key[e], idx[e]: entry (E wave + e) 64 + lane; afterwards the entry at that place in ascending order, equal keys in the order they had.
+// FIRST: the lowest bit that differs between keys.
+template <uint32_t BLOCK, int E, int FIRST> __device__ __forceinline__ void radix_sort(RadixLds<BLOCK>& lds, uint32_t (&key)[E], uint32_t (&idx)[E]) {
+  constexpr uint32_t WAVES = RadixLds<BLOCK>::WAVES, PITCH = RadixLds<BLOCK>::PITCH, OWN = WAVES * 256 / BLOCK;
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  volatile uint32_t* mine = lds.counts + wave * PITCH;   // (volatile: a wave's LDS accesses are in order, and stay in the program's)
+#pragma unroll
+  for (int shift = FIRST; shift < 32; shift += 8) {
+#pragma unroll
+    for (int x = 0; x < 4; x++) mine[lane + 64 * x] = 0;
+    uint32_t place[E];
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+      const uint32_t d = (key[e] >> shift) & 255;
+      uint32_t low = ~0u, high = ~0u;   // the lanes whose entry has the same digit
+#pragma unroll
+      for (int bit = shift; bit < shift + 8 && bit < 32; bit++) {
+        const uint32_t one = (uint32_t)__builtin_amdgcn_sbfe((int)key[e], bit, 1);   // 0 or all ones
+        const uint64_t ones = __ballot(one != 0);
+        low &= ~((uint32_t)ones ^ one);
+        high &= ~((uint32_t)(ones >> 32) ^ one);
+      }
+      const uint32_t before = __builtin_amdgcn_mbcnt_hi(high, __builtin_amdgcn_mbcnt_lo(low, 0)), seen = mine[d];
+      place[e] = seen + before;
+      if (before == 0) mine[d] = seen + __popc(low) + __popc(high);
+    }
+    __syncthreads();
+    // exclusive sums in the order of digits, a digit's waves one after the other
+    const uint32_t d = tid * OWN / WAVES, w0 = tid * OWN % WAVES;
+    uint32_t c[OWN], sum = 0;
+#pragma unroll
+    for (uint32_t x = 0; x < OWN; x++) c[x] = lds.counts[(w0 + x) * PITCH + d], sum += c[x];
+    const uint32_t up = wave_scan_u32(sum);
+    if (lane == 63) lds.sums[wave] = up;
+    __syncthreads();
+    uint32_t base = up - sum;
+#pragma unroll
+    for (uint32_t w = 0; w < WAVES; w++) base += w < wave ? lds.sums[w] : 0;
+#pragma unroll
+    for (uint32_t x = 0; x < OWN; x++) {
+      lds.counts[(w0 + x) * PITCH + d] = base;
+      base += c[x];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+      const uint32_t to = place[e] + mine[(key[e] >> shift) & 255];
+      lds.keys[to] = key[e];
+      lds.idxs[to] = (uint16_t)idx[e];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+      const uint32_t at = (E * wave + e) * 64 + lane;
+      key[e] = lds.keys[at];
+      idx[e] = lds.idxs[at];
+    }
+  }
+}
+
+// The `count` elements in[t * stride], sorted: f(place, key, t).
+template <typename T, uint32_t BLOCK, int E, typename F>
+__device__ __forceinline__ void radix_sort_line(RadixLds<BLOCK>& lds, const T* in, size_t stride, uint32_t count, uint32_t flip, F&& f) {
+  uint32_t key[E], idx[E];
+  const uint32_t first = threadIdx.x / 64 * (64 * E) + threadIdx.x % 64;
+#pragma unroll
+  for (int e = 0; e < E; e++) {
+    const uint32_t t = first + 64 * e;
+    idx[e] = t;
+    key[e] = t < count ? (uint32_t)sort_key(to_arith(in[(size_t)t * stride])) ^ flip : 0xffffffffu;   // (sorts behind every real entry)
+  }
+  radix_sort<BLOCK, E, sizeof(T) == 2 ? 13 : 0>(lds, key, idx);   // (a half as a float: 13 bits of the mantissa are clear)
+#pragma unroll
+  for (int e = 0; e < E; e++)
+    if (first + 64 * e < count) f(first + 64 * e, key[e], idx[e]);
+}
+template <typename T, uint32_t BLOCK, typename F>
+__device__ __forceinline__ void radix_sort_line(RadixLds<BLOCK>& lds, const T* in, size_t stride, uint32_t count, uint32_t flip, F&& f) {
+  const uint32_t e = sort_entries<BLOCK>(count);
+  if constexpr (BLOCK == SORT_WIDE_BLOCK) {
+    if (e == 4) return radix_sort_line<T, BLOCK, 4>(lds, in, stride, count, flip, f);
+  }
+  if (e == 2) radix_sort_line<T, BLOCK, 2>(lds, in, stride, count, flip, f);
+  else radix_sort_line<T, BLOCK, 1>(lds, in, stride, count, flip, f);
 }
 
 // descending order = ascending order of the inverted key
@@ -548,13 +660,37 @@ DEF_RANK(2)
 DEF_RANK(4)
 DEF_RANK(8)
 
-#define DEF_ARGSORT(T, TN, K)                                                                                                   \
+template <typename T, uint32_t BLOCK> __device__ __forceinline__ void argsort_radix_impl(const hck_scan_args& p) {
+  __shared__ RadixLds<BLOCK> lds;
+  const uint32_t i = blockIdx.x / p.inner, j = blockIdx.x - i * p.inner;
+  const size_t base = (size_t)i * p.reduce * p.inner + j;
+  int64_t* out = (int64_t*)p.out + base;
+  radix_sort_line<T, BLOCK>(lds, (const T*)p.in + base, p.inner, p.reduce, (uint32_t)key_flip<float>(p.reverse),
+                            [&](uint32_t place, uint32_t, uint32_t t) { out[(size_t)place * p.inner] = (int64_t)t; });
+}
+template <typename T, uint32_t BLOCK> __device__ __forceinline__ void argsort_chunks_radix_impl(const hck_sort_args& p) {
+  __shared__ RadixLds<BLOCK> lds;
+  const uint32_t chunks = (p.reduce + ARGSORT_MAX - 1) / ARGSORT_MAX;
+  uint32_t line, chunk;
+  line_on_xcd(blockIdx.x, chunks, p.outer * p.inner, line, chunk);
+  const uint32_t i = line / p.inner, j = line - i * p.inner, first = chunk * ARGSORT_MAX;
+  const uint32_t count = p.reduce - first < ARGSORT_MAX ? p.reduce - first : ARGSORT_MAX;
+  const size_t run = (size_t)line * p.reduce + first;
+  radix_sort_line<T, BLOCK>(lds, (const T*)p.in + ((size_t)i * p.reduce + first) * p.inner + j, p.inner, count, (uint32_t)key_flip<float>(p.descending),
+                            [&](uint32_t place, uint32_t key, uint32_t t) {
+                              ((uint32_t*)p.keys_out)[run + place] = key;
+                              p.idx_out[run + place] = first + t;
+                            });
+}
+
+#define DEF_ARGSORT(T, TN, K, WIDE_CHUNKS, WIDE_LINE)                                                                             \
   HC_KERNEL void hc_argsort_chunks_##TN(hck_sort_args p) { argsort_chunks_impl<T, K, HCK_BLOCK>(p); }                           \
   HC_KERNEL void hc_argsort_##TN(hck_scan_args p) { argsort_impl<T, HCK_BLOCK>(p); }                                            \
-  extern "C" __global__ __launch_bounds__(SORT_WIDE_BLOCK) void hc_argsort_chunks_wide_##TN(hck_sort_args p) {                  \
-    argsort_chunks_impl<T, K, SORT_WIDE_BLOCK>(p);                                                                              \
-  }                                                                                                                             \
-  extern "C" __global__ __launch_bounds__(SORT_WIDE_BLOCK) void hc_argsort_wide_##TN(hck_scan_args p) { argsort_impl<T, SORT_WIDE_BLOCK>(p); }
-DEF_ARGSORT(float, f32, uint32_t)
-DEF_ARGSORT(half_t, f16, uint32_t)
-DEF_ARGSORT(int64_t, i64, uint64_t)
+  extern "C" __global__ __launch_bounds__(SORT_WIDE_BLOCK) void hc_argsort_chunks_wide_##TN(hck_sort_args p) { WIDE_CHUNKS(p); } \
+  extern "C" __global__ __launch_bounds__(SORT_WIDE_BLOCK) void hc_argsort_wide_##TN(hck_scan_args p) { WIDE_LINE(p); }
+#define DEF_ARGSORT_RADIX(T, TN)                                                                                                  \
+  DEF_ARGSORT(T, TN, uint32_t, (argsort_chunks_radix_impl<T, SORT_WIDE_BLOCK>), (argsort_radix_impl<T, SORT_WIDE_BLOCK>))         \
+  HC_KERNEL void hc_argsort_radix_##TN(hck_scan_args p) { argsort_radix_impl<T, HCK_BLOCK>(p); }
+DEF_ARGSORT_RADIX(float, f32)
+DEF_ARGSORT_RADIX(half_t, f16)
+DEF_ARGSORT(int64_t, i64, uint64_t, (argsort_chunks_impl<int64_t, uint64_t, SORT_WIDE_BLOCK>), (argsort_impl<int64_t, SORT_WIDE_BLOCK>))
