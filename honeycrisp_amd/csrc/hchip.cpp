@@ -2126,6 +2126,20 @@ extern "C" int hc_cumulative(hc_ctx* ctx, int op, int dtype, const void* in, voi
     }
   }
   char name[64];
+  // A workgroup per row, one launch (cumulative_rowblock_impl). us, a wave per row or segments of one / a workgroup per row: fp32 [8, 600] 3.9 / 3.0,
+  // [8, 4096] 8.1 / 3.1, [8, 20000] 9.1 / 5.0, [8, 50257] 9.3 / 8.4, [256, 50257] 50 / 25, [4096, 8192] 86 / 49, [16384, 600] 22 / 17. Not rows of up to 256
+  // elements, one tile of a wave ([4096, 100] 3.6 / 4.7), nor many of up to 512 (fp16 [16384, 300] 11.1 / 13.5); and not a few rows so long that one
+  // unit each takes longer than all units and a second launch: [8, 60000] 9.2 / 9.4, [8, 100000] 9.6 / 14.1, fp16 [8, 45000] 9.5 / 9.1 and [8, 60000]
+  // 9.6 / 11.2, int64 [8, 20000] 8.9 / 7.3 and [8, 30000] 9.1 / 9.6. With a row for every fourth unit (int64: second) the totals' pass over the data
+  // costs more at any length: [64, 80000] 21 / 14, [128, 200000] 97 / 54, int64 [64, 60000] 22.1 / 21.5 and [64, 100000] 33 / 48.
+  const uint64_t longest = dtype == HC_F32 ? 57344 : dtype == HC_F16 ? 49152 : 24576;
+  if (inner == 1 && reduce > 256 && (reduce >= 512 || outer <= 2048) &&
+      ((uint64_t)reduce <= longest || (uint64_t)outer >= cus / (dtype == HC_I64 ? 2 : 4))) {
+    // (1024 lanes while a unit has no more than one row of more than a quarter of a tile: [8, 4096] 3.9 / 3.1, [512, 2000] 3.9 / 4.1)
+    const bool wide = reduce > 1024 && (uint64_t)outer < 2 * cus;
+    snprintf(name, sizeof(name), "hc_cumulative_%s_rowblock%s_%s", opn, wide ? "_wide" : "", tn);
+    return launch(ctx, name, (uint64_t)outer, 1, &k, sizeof(k), wide ? 1024 : HCK_BLOCK);
+  }
   const uint64_t units = (uint64_t)outer * segs * (uint64_t)inner;  // waves (rows) or columns (cols)
   const uint64_t blocks = inner == 1 && !lane_rows ? ceil_div(units, HCK_BLOCK / 64) : ceil_div(units / (colsv ? vec : 1), HCK_BLOCK);
   Scratch scratch(ctx);

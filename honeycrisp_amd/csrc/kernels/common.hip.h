@@ -77,6 +77,16 @@ template <typename T, int N> __device__ __forceinline__ void load_vec_loose(cons
   for (int i = 0; i < N; i++) dst[i] = t.v[i];
 }
 
+template <typename T, int N> __device__ __forceinline__ void store_vec_loose(T* dst, const T (&src)[N]) {
+  struct __attribute__((packed, aligned(sizeof(T)))) Loose {
+    Vec<T, N> v;
+  };
+  Vec<T, N> t;
+#pragma unroll
+  for (int i = 0; i < N; i++) t.v[i] = src[i];
+  reinterpret_cast<Loose*>(dst)->v = t;
+}
+
 // The same with the stride known at compile time: S = 1 one 16-byte load, S = 0 one element
 // repeated, S < 0 decided at run time. Kernels branch once on the (wave-uniform) strides of
 // all their operands and run a body whose loads are unconditional, so they issue back to back;

@@ -1,12 +1,12 @@
 // Running sums / products and argsort along the middle axis of an [outer, reduce, inner] view.
 //
 // cumulativeSum / cumulativeProd (BackendCPU.swift:922-998): out[k] = x[0] (op) ... (op) x[k]
-// (or up to x[k-1] when exclusive), optionally from the far end. Rows (inner == 1): one wave
-// per row walks it in tiles of 64 x 4 elements (in-lane scan, wave scan of the lane totals
-// with shuffles, running carry); floats are combined in tree order, so they differ from the
+// (or up to x[k-1] when exclusive), optionally from the far end. Rows (inner == 1): a workgroup per row, or, for
+// short ones, one wave that walks it in tiles of 64 x 4 elements (in-lane scan, wave scan of the lane totals
+// by DPP, running carry); floats are combined in tree order, so they differ from the
 // sequential CPU loop by rounding only; int64 is exact. Columns (inner > 1): one lane per
 // column, sequential along the axis, lanes coalesced along inner. When there are too few lines
-// to fill the chip, the axis is cut into segments: totals per segment, a small scan of the
+// to fill the chip (rows: and they are long), the axis is cut into segments: totals per segment, a small scan of the
 // totals, then the segments are scanned starting from what precedes them.
 //
 // argsort (BackendCPU.swift:888-920): one block per (outer, inner) pair merge-sorts (key, index)
@@ -24,19 +24,49 @@ template <int OP, typename C> __device__ __forceinline__ C scan_combine(C a, C b
   return OP == SCAN_SUM ? a + b : a * b;
 }
 
+// v of another lane by DPP (`identity` where there is none), a cross-lane move of the vector ALU: no LDS, unlike a shuffle.
+template <int CTRL, int ROWS, typename C> __device__ __forceinline__ C lane_move(C v, C identity) {
+  if constexpr (sizeof(C) == 8) {
+    const uint64_t x = (uint64_t)v, i = (uint64_t)identity;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp((int)i, (int)x, CTRL, ROWS, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp((int)(i >> 32), (int)(x >> 32), CTRL, ROWS, 0xf, false);
+    return (C)((uint64_t)hi << 32 | lo);
+  } else {
+    return __builtin_bit_cast(C, __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, identity), __builtin_bit_cast(int, v), CTRL, ROWS, 0xf, false));
+  }
+}
+// Inclusive scan over the lanes of a wave: within rows of 16 lanes, then from row to row.
+template <int OP, typename C> __device__ __forceinline__ C wave_scan(C v) {
+  constexpr C id = OP == SCAN_SUM ? (C)0 : (C)1;
+  v = scan_combine<OP, C>(lane_move<0x111, 0xf>(v, id), v);   // row_shr:1, 2, 4, 8
+  v = scan_combine<OP, C>(lane_move<0x112, 0xf>(v, id), v);
+  v = scan_combine<OP, C>(lane_move<0x114, 0xf>(v, id), v);
+  v = scan_combine<OP, C>(lane_move<0x118, 0xf>(v, id), v);
+  v = scan_combine<OP, C>(lane_move<0x142, 0xa>(v, id), v);   // row_bcast:15 into rows 1 and 3
+  v = scan_combine<OP, C>(lane_move<0x143, 0xc>(v, id), v);   // row_bcast:31 into rows 2 and 3
+  return v;
+}
+// What is in the lanes below: the inclusive scan of the lane before (wave_shr:1).
+template <int OP, typename C> __device__ __forceinline__ C wave_before(C incl) { return lane_move<0x138, 0xf>(incl, OP == SCAN_SUM ? (C)0 : (C)1); }
+
+// v of lane `l` (the same in every lane)
+template <typename C> __device__ __forceinline__ C lane_value(C v, uint32_t l) {
+  if constexpr (sizeof(C) == 8) {
+    const uint64_t x = (uint64_t)v;
+    return (C)((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32 | (uint32_t)__builtin_amdgcn_readlane((int)x, l));
+  } else {
+    return __builtin_bit_cast(C, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), l));
+  }
+}
+
 // What precedes segment `seg` of a row, from the totals of all of them, in the order of cumulative_carry_impl (same bits).
 // A row of up to 256 segments does with this, four rounds at most in every wave, and saves the launch between
-// the totals and the scan (2.8 us for [8, 50257] fp32; softmax, argsort, gather and running sum: 89.1 -> 87.5 us).
+// the totals and the scan (2.8 us for [8, 50257] fp32 cut into segments).
 template <typename C, int OP>
 __device__ __forceinline__ C carry_before(const C* totals, uint32_t segs, uint32_t seg, uint32_t lane) {
   C run = scan_identity<OP, C>();
   for (uint32_t s0 = 0;; s0 += 64) {
-    C incl = s0 + lane < segs ? totals[s0 + lane] : scan_identity<OP, C>();
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const C up = __shfl_up(incl, d, 64);
-      if ((int)lane >= d) incl = scan_combine<OP, C>(up, incl);
-    }
+    const C incl = wave_scan<OP, C>(s0 + lane < segs ? totals[s0 + lane] : scan_identity<OP, C>());
     if (seg < s0 + 64) {   // (the same in every lane)
       const C before = __shfl(incl, (int)((seg - s0 - 1) & 63), 64);
       return scan_combine<OP, C>(run, seg == s0 ? scan_identity<OP, C>() : before);
@@ -79,15 +109,8 @@ template <typename T, int OP, int PHASE> __device__ __forceinline__ void cumulat
       continue;
     }
     // inclusive scan of the lane totals across the wave
-    C incl = run;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const C up = __shfl_up(incl, d, 64);
-      if (lane >= (uint32_t)d) incl = scan_combine<OP, C>(up, incl);
-    }
-    C before = __shfl_up(incl, 1, 64);  // everything in lanes below this one
-    if (lane == 0) before = scan_identity<OP, C>();
-    C acc = scan_combine<OP, C>(carry, before);
+    const C incl = wave_scan<OP, C>(run);
+    C acc = scan_combine<OP, C>(carry, wave_before<OP, C>(incl));
 #pragma unroll
     for (int e = 0; e < E; e++) {
       const uint32_t t = base + lane * E + e;
@@ -101,6 +124,89 @@ template <typename T, int OP, int PHASE> __device__ __forceinline__ void cumulat
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) carry = scan_combine<OP, C>(carry, __shfl_down(carry, d, 64));
     if (lane == 0) ((C*)p.carry)[unit] = carry;
+  }
+}
+
+// A workgroup per row, one launch (the host's rule and figures: hc_cumulative). BLOCK lanes take tiles of 4 elements each, GROUP tiles at a time: all
+// loads of a group are out before the first is waited for, and its waves' totals meet in LDS once. Bound by the vector ALU of the row's one
+// unit, about 3.5 us per 32768 fp32. What it depends on is that lanes exchange by DPP: with shuffles, which go through LDS, rows of 4096 took 5.8 us
+// on 256 lanes and 7.3 on 1024 (now 3.9 and 3.1), and with every lane reading all 16 totals of a tile [8, 50257] 10.1 (8.4).
+template <typename T, int OP, uint32_t BLOCK> __device__ __forceinline__ void cumulative_rowblock_impl(const hck_scan_args& p) {
+  typedef typename Arith<T>::type C;
+  constexpr uint32_t E = 4, GROUP = sizeof(C) == 8 ? 4 : 8, WAVES = BLOCK / 64;
+  __shared__ C totals[2][GROUP][WAVES];
+  const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = p.reduce;
+  const T* in = (const T*)p.in + (size_t)blockIdx.x * n;
+  T* out = (T*)p.out + (size_t)blockIdx.x * n;
+  C carry = scan_identity<OP, C>();
+  uint32_t half = 0;   // (totals of neighbouring groups in turn: one barrier per group)
+  for (uint32_t first = 0; first < n; first += GROUP * BLOCK * E, half ^= 1) {
+    // x[g]: logical positions t .. t + 3 (in scan order) of tile g; the element sits at n-1-t when reversed
+    T x[GROUP][E];
+    const uint32_t tiles = (n - first + BLOCK * E - 1) / (BLOCK * E);
+#pragma unroll
+    for (uint32_t g = 0; g < GROUP; g++) {
+      if (g >= tiles) break;
+      const uint32_t t = first + (g * BLOCK + threadIdx.x) * E;
+      if (t + E <= n) {
+        load_vec_loose<T, E>(in + (p.reverse ? n - E - t : t), x[g]);
+      } else {
+#pragma unroll
+        for (uint32_t e = 0; e < E; e++) x[g][p.reverse ? E - 1 - e : e] = t + e < n ? in[p.reverse ? n - 1 - t - e : t + e] : (T)scan_identity<OP, C>();
+      }
+    }
+    C before[GROUP];   // everything in the wave's lanes below this one
+#pragma unroll
+    for (uint32_t g = 0; g < GROUP; g++) {
+      if (g >= tiles) break;
+      if (p.reverse) {
+        const T x0 = x[g][0], x1 = x[g][1];
+        x[g][0] = x[g][3], x[g][1] = x[g][2], x[g][2] = x1, x[g][3] = x0;
+      }
+      C incl = scan_identity<OP, C>();
+#pragma unroll
+      for (uint32_t e = 0; e < E; e++) incl = scan_combine<OP, C>(incl, to_arith(x[g][e]));
+      incl = wave_scan<OP, C>(incl);
+      before[g] = wave_before<OP, C>(incl);
+      if (lane == 63) totals[half][g][wave] = incl;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t g = 0; g < GROUP; g++) {
+      if (g >= tiles) break;
+      const uint32_t t = first + (g * BLOCK + threadIdx.x) * E;
+      // (the waves' totals in a row of 16 lanes, scanned)
+      static_assert(WAVES == 16 || WAVES == 4, "a power of two of at most 16");
+      C total = totals[half][g][lane % WAVES];
+      total = scan_combine<OP, C>(lane_move<0x111, 0xf>(total, scan_identity<OP, C>()), total);
+      total = scan_combine<OP, C>(lane_move<0x112, 0xf>(total, scan_identity<OP, C>()), total);
+      if constexpr (WAVES > 4) {
+        total = scan_combine<OP, C>(lane_move<0x114, 0xf>(total, scan_identity<OP, C>()), total);
+        total = scan_combine<OP, C>(lane_move<0x118, 0xf>(total, scan_identity<OP, C>()), total);
+      }
+      const C all = lane_value(total, WAVES - 1), lower = wave == 0 ? scan_identity<OP, C>() : lane_value(total, wave - 1);
+      C acc = scan_combine<OP, C>(carry, scan_combine<OP, C>(lower, before[g]));
+      carry = scan_combine<OP, C>(carry, all);
+      if (t >= n) continue;
+      T o[E];
+#pragma unroll
+      for (uint32_t e = 0; e < E; e++) {
+        const C next = scan_combine<OP, C>(acc, to_arith(x[g][e]));
+        o[e] = from_arith<T>(p.exclusive ? acc : next);
+        acc = next;
+      }
+      if (t + E <= n) {
+        if (p.reverse) {
+          const T o0 = o[0], o1 = o[1];
+          o[0] = o[3], o[1] = o[2], o[2] = o1, o[3] = o0;
+        }
+        store_vec_loose<T, E>(out + (p.reverse ? n - E - t : t), o);
+      } else {
+#pragma unroll
+        for (uint32_t e = 0; e + 1 < E; e++)
+          if (t + e < n) out[p.reverse ? n - 1 - t - e : t + e] = o[e];
+      }
+    }
   }
 }
 
@@ -156,15 +262,8 @@ template <typename C, int OP> __device__ __forceinline__ void cumulative_carry_i
   for (uint32_t s0 = 0; s0 < p.segs; s0 += 64) {
     const uint32_t s = s0 + lane;
     const bool ok = s < p.segs;
-    C incl = ok ? c[(size_t)s * p.inner] : scan_identity<OP, C>();
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const C up = __shfl_up(incl, d, 64);
-      if ((int)lane >= d) incl = scan_combine<OP, C>(up, incl);
-    }
-    C before = __shfl_up(incl, 1, 64);
-    if (lane == 0) before = scan_identity<OP, C>();
-    if (ok) c[(size_t)s * p.inner] = scan_combine<OP, C>(run, before);
+    const C incl = wave_scan<OP, C>(ok ? c[(size_t)s * p.inner] : scan_identity<OP, C>());
+    if (ok) c[(size_t)s * p.inner] = scan_combine<OP, C>(run, wave_before<OP, C>(incl));
     run = scan_combine<OP, C>(run, __shfl(incl, 63, 64));
   }
 }
@@ -190,6 +289,17 @@ template <typename C, int OP> __device__ __forceinline__ void cumulative_carry_i
   HC_KERNEL void hc_cumulative_prod_rows_totals_##TN(hck_scan_args p) { cumulative_rows_impl<T, SCAN_PROD, 1>(p); } \
   HC_KERNEL void hc_cumulative_sum_cols_totals_##TN(hck_scan_args p) { cumulative_cols_impl<T, SCAN_SUM, 1, 1>(p); }   \
   HC_KERNEL void hc_cumulative_prod_cols_totals_##TN(hck_scan_args p) { cumulative_cols_impl<T, SCAN_PROD, 1, 1>(p); }
+#define DEF_CUMULATIVE_ROWBLOCK(TN, T, NAME, OP)                                                                                   \
+  HC_KERNEL void hc_cumulative_##NAME##_rowblock_##TN(hck_scan_args p) { cumulative_rowblock_impl<T, OP, HCK_BLOCK>(p); }           \
+  extern "C" __global__ __launch_bounds__(1024) void hc_cumulative_##NAME##_rowblock_wide_##TN(hck_scan_args p) {                   \
+    cumulative_rowblock_impl<T, OP, 1024>(p);                                                                                      \
+  }
+DEF_CUMULATIVE_ROWBLOCK(f32, float, sum, SCAN_SUM)
+DEF_CUMULATIVE_ROWBLOCK(f32, float, prod, SCAN_PROD)
+DEF_CUMULATIVE_ROWBLOCK(f16, half_t, sum, SCAN_SUM)
+DEF_CUMULATIVE_ROWBLOCK(f16, half_t, prod, SCAN_PROD)
+DEF_CUMULATIVE_ROWBLOCK(i64, int64_t, sum, SCAN_SUM)
+DEF_CUMULATIVE_ROWBLOCK(i64, int64_t, prod, SCAN_PROD)
 DEF_CUMULATIVE(f32, float)
 DEF_CUMULATIVE(f16, half_t)
 DEF_CUMULATIVE(i64, int64_t)
@@ -387,17 +497,6 @@ template <bool WIDE, uint32_t BLOCK> __device__ __forceinline__ void sort_lds(co
 // 1000 10.4 / 7.7, of 50257 (with the merging of 13 runs) 42.7 / 39.0, 256 of 300 (256 lanes) 7.5 / 6.6, of 128 4.9 / 5.2. Blocks that share
 // a unit keep merging (1024 lines of 4096 44.8 / 60.4, of 512 11.9 / 12.7).
 
-// Inclusive sum over the lanes of a wave: six DPP additions, no LDS.
-__device__ __forceinline__ uint32_t wave_scan_u32(uint32_t v) {
-  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);   // row_shr:1, 2, 4, 8 (rows of 16 lanes)
-  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
-  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);   // row_bcast:15 into rows 1 and 3
-  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);   // row_bcast:31 into rows 2 and 3
-  return v;
-}
-
 template <uint32_t BLOCK> struct RadixLds {
   static constexpr uint32_t WAVES = BLOCK / 64, PITCH = 257;   // (counters of a digit in different banks)
   static constexpr uint32_t ENTRIES = BLOCK == SORT_WIDE_BLOCK ? ARGSORT_MAX : 2 * BLOCK;
@@ -437,7 +536,7 @@ template <uint32_t BLOCK, int E, int FIRST> __device__ __forceinline__ void radi
     uint32_t c[OWN], sum = 0;
 #pragma unroll
     for (uint32_t x = 0; x < OWN; x++) c[x] = lds.counts[(w0 + x) * PITCH + d], sum += c[x];
-    const uint32_t up = wave_scan_u32(sum);
+    const uint32_t up = wave_scan<SCAN_SUM, uint32_t>(sum);
     if (lane == 63) lds.sums[wave] = up;
     __syncthreads();
     uint32_t base = up - sum;
