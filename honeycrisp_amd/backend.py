@@ -20,16 +20,25 @@ from typing import List, Optional, Sequence, Union
 import numpy as np
 
 from . import _lib
+try:
+    from . import _native
+except ImportError:     # not built: HIPBackend says so, everything else of this module works
+    _native = None
 from .descriptors import (BackendError, BitwiseOp, BroadcastData, BroadcastStrides, ComparisonOp, DType,
                           ElemwiseOp, NumericBinaryOp, ReduceDims, ReduceOp, RepeatDims,
                           ScatterGatherIndices, product)
+
+
+class _Uses(threading.local):
+    """Each thread's stack of Backend.use(); None before its first."""
+    stack = None
 
 
 class Backend:
     """Abstract op set (Backend.swift:170-815)."""
 
     _default: Optional["Backend"] = None
-    _tls = threading.local()
+    _tls = _Uses()
 
     # -- Backend.defaultBackend / current / use (Backend.swift:44-88)
     @classmethod
@@ -38,7 +47,7 @@ class Backend:
 
     @classmethod
     def current(cls) -> "Backend":
-        stack = getattr(Backend._tls, "stack", None)
+        stack = Backend._tls.stack
         if stack:
             return stack[-1]
         if Backend._default is None:
@@ -50,7 +59,7 @@ class Backend:
             self.backend = backend
 
         def __enter__(self):
-            if not hasattr(Backend._tls, "stack"):
+            if Backend._tls.stack is None:
                 Backend._tls.stack = []
             Backend._tls.stack.append(self.backend)
             return self.backend
@@ -240,13 +249,11 @@ def powf(x, y) -> np.float32:
     return np.float32(_libm.powf(float(x), float(y)))
 
 
-class HIPData:
-    """Device buffer backing a tensor: this backend's `Tensor.Data` (Tensor.swift:69-85)."""
+class HIPData(_native.Data if _native else object):
+    """Device buffer backing a tensor: this backend's `Tensor.Data` (Tensor.swift:69-85). HIPData(backend, ptr, byteCount): the
+    base class has the three and gives the buffer back with the object."""
 
-    def __init__(self, backend: "HIPBackend", ptr: int, byteCount: int):
-        self.backend = backend
-        self.ptr = ptr
-        self.byteCount = byteCount
+    permutation = None
 
     def wait(self):
         self.backend.sync()
@@ -267,12 +274,6 @@ class HIPData:
         if self.byteCount:
             self.backend._check(self.backend._lib.hc_memcpy_h2d(
                 self.backend._ctx, c_void_p(self.ptr), host.ctypes.data_as(c_void_p), self.byteCount))
-
-    def __del__(self):
-        backend, ptr = self.backend, self.ptr
-        self.ptr = None
-        if ptr and backend is not None and backend._ctx:
-            backend._lib.hc_free(backend._ctx, ptr)
 
 
 class PermutationData(HIPData):
@@ -366,15 +367,18 @@ class HIPBackend(Backend):
     """MI355X backend: one device, one in-order stream, kernels from libhchip.so."""
 
     def __init__(self, device: int = 0):
-        self._ctx = None
+        self._ctx = self._native = None
         self._capturing = False
         self._perm_cache, self._perm_cache_bytes = {}, 0
+        if _native is None:
+            raise ImportError("honeycrisp_amd/_native.so is missing: build it with `python -m honeycrisp_amd.csrc.build`")
         self._lib = _lib.load()
         ctx = c_void_p()
         status = self._lib.hc_init(device, byref(ctx))
         if status != _lib.HC_OK:
             self._raise(status)
         self._ctx = ctx
+        self._native = _native.Context(_lib.LIB_PATH, ctx.value, HIPData)
         # hc_set_batching's current values (HCHIP_BATCHING in the environment gives a context its first)
         env = (os.environ.get("HCHIP_BATCHING") or "0").split(",")
         self._batching = (int(env[0]), int(env[1]) if len(env) > 1 else 0)
@@ -382,6 +386,7 @@ class HIPBackend(Backend):
     def close(self):
         if self._ctx:
             self._perm_cache.clear()
+            self._native.close()
             self._lib.hc_shutdown(self._ctx)
             self._ctx = None
 
@@ -484,12 +489,7 @@ class HIPBackend(Backend):
     # -- storage (DataAllocator, Backend.swift:894-896)
 
     def allocate(self, byteCount: int) -> HIPData:
-        byteCount = int(byteCount)
-        ptr = c_void_p()
-        status = self._lib.hc_malloc(self._ctx, byteCount if byteCount > 0 else 0, byref(ptr))
-        if status != _lib.HC_OK:
-            self._raise(status)
-        return HIPData(self, ptr.value, byteCount)
+        return self._native.alloc(self, int(byteCount))
 
     def upload(self, host: np.ndarray) -> HIPData:
         host = np.ascontiguousarray(host)
@@ -530,52 +530,27 @@ class HIPBackend(Backend):
         return self.upload(convert_host_array(arr.reshape(-1), dtype))
 
     def constant(self, value, count: int, dtype: DType) -> HIPData:
-        out = self.allocate(count * dtype.byteSize)
         vf, vi = self._scalar(value, dtype)
-        if dtype != DType.int64:
-            vf = c_float(float(np.float32(value)))
-        self._check(self._lib.hc_fill(self._ctx, dtype, vf, vi, out.ptr, count))
-        return out
+        return self._native.fill(self, dtype, vf, vi, count)
 
     def broadcast(self, a: BroadcastData, dtype: DType) -> HIPData:
-        out = self.allocate(product(a.strides.shape) * dtype.byteSize)
-        ad = self._dev(a.data)
-        s = self._s(a.strides)
-        self._check(self._lib.hc_broadcast(self._ctx, dtype, ad.ptr, s, out.ptr))
-        return out
+        return self._native.broadcast(self, dtype, a.data, a.strides)
 
     def binaryOp(self, a, b, op: NumericBinaryOp, dtype: DType, count: Optional[int] = None) -> HIPData:
         if isinstance(a, BroadcastData) and isinstance(b, BroadcastData):
-            out = self.allocate(product(a.strides.shape) * dtype.byteSize)
-            ad, bd = self._dev(a.data), self._dev(b.data)
-            sa, sb = self._s(a.strides), self._s(b.strides)
-            self._check(self._lib.hc_binary_op(self._ctx, op, dtype, ad.ptr, sa,
-                                               bd.ptr, sb, out.ptr))
-            return out
+            return self._native.binary(self, op, dtype, a.data, a.strides, b.data, b.strides)
         if count is None:
             raise TypeError("binaryOp with a scalar needs count")
         scalar_first = isinstance(a, (int, float, np.floating, np.integer))
         tensor, scalar = (b, a) if scalar_first else (a, b)
-        out = self.allocate(count * dtype.byteSize)
-        td = self._dev(tensor)
         sf, si = self._scalar(scalar, dtype)
-        self._check(self._lib.hc_binary_op_scalar(self._ctx, op, dtype, td.ptr, sf, si,
-                                                  int(scalar_first), out.ptr, count))
-        return out
-
-    def _fused(self, fn, x, y, z, dtype):
-        out = self.allocate(product(x.strides.shape) * dtype.byteSize)
-        xd, yd, zd = self._dev(x.data), self._dev(y.data), self._dev(z.data)
-        sx, sy, sz = self._s(x.strides), self._s(y.strides), self._s(z.strides)
-        self._check(fn(self._ctx, dtype, xd.ptr, sx, yd.ptr, sy,
-                       zd.ptr, sz, out.ptr))
-        return out
+        return self._native.binary_scalar(self, op, dtype, tensor, sf, si, scalar_first, count)
 
     def mulAdd(self, input: BroadcastData, coeff: BroadcastData, bias: BroadcastData, dtype: DType):
-        return self._fused(self._lib.hc_mul_add, input, coeff, bias, dtype)
+        return self._native.mul_add(self, dtype, input.data, input.strides, coeff.data, coeff.strides, bias.data, bias.strides)
 
     def addMul(self, input: BroadcastData, bias: BroadcastData, coeff: BroadcastData, dtype: DType):
-        return self._fused(self._lib.hc_add_mul, input, bias, coeff, dtype)
+        return self._native.add_mul(self, dtype, input.data, input.strides, bias.data, bias.strides, coeff.data, coeff.strides)
 
     def when(self, mask: BroadcastData, a, b, dtype: DType):
         """a / b: BroadcastData, or ("scalar", value, shape) like Backend.TensorOrScalar
@@ -586,7 +561,8 @@ class HIPBackend(Backend):
                 return x
             _, value, shape = x
             return BroadcastData(BroadcastStrides(shape, [0] * len(shape)), self.constant(value, 1, dtype))
-        return self._fused(self._lib.hc_when, mask, branch(a), branch(b), dtype)
+        a, b = branch(a), branch(b)
+        return self._native.when(self, dtype, mask.data, mask.strides, a.data, a.strides, b.data, b.strides)
 
     def compare(self, a, b, op: ComparisonOp, dtype: DType, count: Optional[int] = None) -> HIPData:
         if isinstance(a, BroadcastData) and isinstance(b, BroadcastData):
@@ -608,57 +584,29 @@ class HIPBackend(Backend):
         return out
 
     def cast(self, a, count: int, inType: DType, outType: DType) -> HIPData:
-        out = self.allocate(count * outType.byteSize)
-        ad = self._dev(a)
-        self._check(self._lib.hc_cast(self._ctx, ad.ptr, inType, out.ptr,
-                                      outType, count))
-        return out
+        return self._native.cast(self, a, count, inType, outType)
 
     def pow(self, a, b: Scalar, scale: Scalar, scales, count: int, dtype: DType) -> HIPData:
-        out = self.allocate(count * dtype.byteSize)
-        ad = self._dev(a)
-        sd = self._dev(scales) if scales is not None else None
         bf, bi = self._scalar(b, dtype)
         scf, sci = self._scalar(scale, dtype)
-        self._check(self._lib.hc_pow(self._ctx, dtype, ad.ptr, bf, scf, bi, sci,
-                                     sd.ptr if sd else None, out.ptr, count))
-        return out
+        return self._native.pow(self, dtype, a, bf, scf, bi, sci, scales, count)
 
     def elemwise(self, a, op: ElemwiseOp, scales, count: int, dtype: DType) -> HIPData:
-        out = self.allocate(count * dtype.byteSize)
-        ad = self._dev(a)
-        sd = self._dev(scales) if scales is not None else None
-        self._check(self._lib.hc_elemwise(self._ctx, op, dtype, ad.ptr,
-                                          sd.ptr if sd else None, out.ptr, count))
-        return out
+        return self._native.elemwise(self, op, dtype, a, scales, count)
 
     def reduce(self, a, op: ReduceOp, dims: ReduceDims, dtype: DType) -> HIPData:
         outType = DType.int64 if op.isIntOut else dtype
-        out = self.allocate(dims.outCount * outType.byteSize)
-        ad = self._dev(a)
-        self._check(self._lib.hc_reduce(self._ctx, op, dtype, ad.ptr, out.ptr,
-                                        dims.outerCount, dims.reduceCount, dims.innerCount))
-        return out
+        return self._native.reduce(self, op, dtype, outType, a, dims.outerCount, dims.reduceCount, dims.innerCount)
 
     def logSoftmax(self, a, dims: ReduceDims, dtype: DType) -> HIPData:
-        out = self.allocate(dims.inCount * dtype.byteSize)
-        ad = self._dev(a)
-        self._check(self._lib.hc_log_softmax(self._ctx, dtype, ad.ptr, out.ptr,
-                                             dims.outerCount, dims.reduceCount, dims.innerCount))
-        return out
+        return self._native.log_softmax(self, dtype, a, dims.outerCount, dims.reduceCount, dims.innerCount)
 
     def normalize(self, input, dims: ReduceDims, eps: Scalar, dtype: DType) -> HIPData:
         """Fused override of the base-class composition (same arithmetic, one kernel for
         innerCount == 1)."""
-        out = self.allocate(dims.inCount * dtype.byteSize)
-        ad = self._dev(input)
-        self._check(self._lib.hc_normalize(self._ctx, dtype, ad.ptr, out.ptr,
-                                           dims.outerCount, dims.reduceCount, dims.innerCount,
-                                           c_float(float(np.float32(eps)))))
-        return out
+        return self._native.normalize(self, dtype, input, dims.outerCount, dims.reduceCount, dims.innerCount, eps)
 
     def gather(self, a, s: ScatterGatherIndices, dtype: DType) -> HIPData:
-        out = self.allocate(s.gatherOutCount * dtype.byteSize)
         # The gather of t / swap / move / PermuteAxes: its index vector came from axisPermutation
         # and runs along the gathered axis only. One direct copy moves the same bytes without
         # reading 8 bytes of index per element.
@@ -667,6 +615,7 @@ class HIPBackend(Backend):
         if (meta is not None and st_.shape[s.axis] == s.middleCount == product(meta[1])
                 and all(stride == (1 if ax == s.axis else 0) or size == 1
                         for ax, (stride, size) in enumerate(zip(st_.strides, st_.shape)))):
+            out = self.allocate(s.gatherOutCount * dtype.byteSize)
             perm, shape = list(meta[0]), list(meta[1])
             if s.outerCount > 1:
                 perm, shape = [0] + [p + 1 for p in perm], [s.outerCount] + shape
@@ -676,12 +625,7 @@ class HIPBackend(Backend):
                                                  (c_int64 * max(n, 1))(*perm), (c_int64 * max(n, 1))(*shape), n,
                                                  s.innerCount, out.ptr))
                 return out
-        ad, idx = self._dev(a), self._dev(s.indices.data)
-        st = self._s(s.indices.strides)
-        self._check(self._lib.hc_gather(self._ctx, dtype, ad.ptr, idx.ptr, st,
-                                        out.ptr, s.outerCount, s.middleCount, s.outCount,
-                                        s.innerCount))
-        return out
+        return self._native.gather(self, dtype, a, s.indices.data, st_, s.outerCount, s.middleCount, s.outCount, s.innerCount)
 
     def bitwiseOp(self, a, b, op: BitwiseOp, dtype: DType, count: Optional[int] = None) -> HIPData:
         def operand(x, other):
@@ -705,13 +649,8 @@ class HIPBackend(Backend):
         return out
 
     def scatter(self, a, s: ScatterGatherIndices, dtype: DType) -> HIPData:
-        out = self.allocate(s.gatherInCount * dtype.byteSize)
-        ad, idx = self._dev(a), self._dev(s.indices.data)
-        st = self._s(s.indices.strides)
-        self._check(self._lib.hc_scatter(self._ctx, dtype, ad.ptr, idx.ptr, st,
-                                         out.ptr, s.outerCount, s.middleCount, s.outCount,
-                                         s.innerCount, int(bool(s.indicesAreUnique))))
-        return out
+        return self._native.scatter(self, dtype, a, s.indices.data, s.indices.strides, s.outerCount, s.middleCount, s.outCount, s.innerCount,
+                                    bool(s.indicesAreUnique))
 
     @staticmethod
     def _fewLongRows(dims: ReduceDims, dtype: DType) -> bool:
@@ -741,20 +680,10 @@ class HIPBackend(Backend):
         return out
 
     def logSoftmaxGrad(self, a, outGrad, dims: ReduceDims, dtype: DType) -> HIPData:
-        out = self.allocate(dims.inCount * dtype.byteSize)
-        ad, gd = self._dev(a), self._dev(outGrad)
-        self._check(self._lib.hc_log_softmax_grad(self._ctx, dtype, ad.ptr, gd.ptr,
-                                                  out.ptr, dims.outerCount, dims.reduceCount,
-                                                  dims.innerCount))
-        return out
+        return self._native.log_softmax_grad(self, dtype, a, outGrad, dims.outerCount, dims.reduceCount, dims.innerCount)
 
     def _cumulative(self, op: int, a, dims: ReduceDims, exclusive: bool, reverse: bool, dtype: DType) -> HIPData:
-        out = self.allocate(dims.inCount * dtype.byteSize)
-        ad = self._dev(a)
-        self._check(self._lib.hc_cumulative(self._ctx, op, int(dtype), ad.ptr, out.ptr,
-                                            dims.outerCount, dims.reduceCount, dims.innerCount, int(bool(exclusive)),
-                                            int(bool(reverse))))
-        return out
+        return self._native.cumulative(self, op, dtype, a, dims.outerCount, dims.reduceCount, dims.innerCount, bool(exclusive), bool(reverse))
 
     def cumulativeSum(self, a, dims: ReduceDims, exclusive: bool, reverse: bool, dtype: DType) -> HIPData:
         return self._cumulative(0, a, dims, exclusive, reverse, dtype)
@@ -764,11 +693,7 @@ class HIPBackend(Backend):
 
     def argsort(self, a, dims: ReduceDims, descending: bool, stable: bool, dtype: DType) -> HIPData:
         """Always stable, which `stable=False` permits (Backend.swift:535-545)."""
-        out = self.allocate(dims.inCount * 8)
-        ad = self._dev(a)
-        self._check(self._lib.hc_argsort(self._ctx, dtype, ad.ptr, out.ptr, dims.outerCount,
-                                         dims.reduceCount, dims.innerCount, int(bool(descending))))
-        return out
+        return self._native.argsort(self, dtype, a, dims.outerCount, dims.reduceCount, dims.innerCount, bool(descending))
 
     def clamp(self, a: BroadcastData, min, max, dtype: DType) -> HIPData:
         """min / max: None, BroadcastData, or ("scalar", value, shape) (Backend.TensorOrScalar)."""
@@ -793,11 +718,7 @@ class HIPBackend(Backend):
     def adamW(self, param, grad, moment1, moment2, beta1, beta2, eps, weightDecay, lr, step, count,
               dtype: DType):
         """One fused kernel, bit-identical to the base-class composition (Backend.adamW)."""
-        outs = [self.allocate(count * dtype.byteSize) for _ in range(3)]
-        ins = [self._dev(x) for x in (param, grad, moment1, moment2)]
-        self._check(self._lib.hc_adamw(
-            self._ctx, dtype, *[x.ptr for x in ins], beta1, beta2, eps, weightDecay, lr, step, count, *[o.ptr for o in outs]))
-        return tuple(outs)
+        return self._native.adamw(self, dtype, param, grad, moment1, moment2, beta1, beta2, eps, weightDecay, lr, step, count)
 
     def matmul(self, a, transA: bool, b, transB: bool, transOut: bool, rows: int, inner: int, cols: int,
                dtype: DType) -> HIPData:
@@ -805,12 +726,7 @@ class HIPBackend(Backend):
 
     def batchedMatmul(self, matrixCount: int, a, transA: bool, b, transB: bool, transOut: bool, rows: int,
                       inner: int, cols: int, dtype: DType) -> HIPData:
-        out = self.allocate(matrixCount * rows * cols * dtype.byteSize)
-        ad, bd = self._dev(a), self._dev(b)
-        self._check(self._lib.hc_matmul(self._ctx, dtype, matrixCount, ad.ptr, int(transA),
-                                        bd.ptr, int(transB), int(transOut), rows, inner, cols,
-                                        out.ptr))
-        return out
+        return self._native.matmul(self, dtype, matrixCount, a, transA, b, transB, transOut, rows, inner, cols)
 
     def triangular(self, a, batch: int, rows: int, cols: int, upper: bool, offset: int, dtype: DType):
         out = self.allocate(batch * rows * cols * dtype.byteSize)

@@ -7,6 +7,7 @@ import os
 import re
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
@@ -178,6 +179,11 @@ def build_all(verbose=True):
     ])
     if verbose:
         print("built", os.path.relpath(LIB_PATH, HERE), os.path.getsize(LIB_PATH), "bytes")
+    native = os.path.join(os.path.dirname(HERE), "_native.so")
+    _run(["gcc", "-O2", "-std=gnu11", "-fPIC", "-shared", "-Wall", "-I" + sysconfig.get_path("include"), os.path.join(HERE, "native.c"),
+          "-o", native, "-ldl"])
+    if verbose:
+        print("built", os.path.relpath(native, HERE), os.path.getsize(native), "bytes")
     if LIB_PATH == os.path.join(HERE, "libhchip.so"):
         # C++ host mirror + HCMatrixBench (links the library just built, and the Linux stand-in for
         # Accelerate that its CPU leg calls the way the reference's CPUBackend calls Accelerate)

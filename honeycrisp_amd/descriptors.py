@@ -173,9 +173,13 @@ class BroadcastStrides:
     def expanding(shape: Sequence[int], newShape: Sequence[int]) -> "BroadcastStrides":
         """Dense data of `shape` seen as `newShape` (Broadcast.swift:148-170). A program's calls repeat a few pairs of
         shapes, so what follows from a pair is kept (by value, 4096 pairs); the object and its lists are the caller's own."""
+        return BroadcastStrides.fromExpansion(expansion(tuple(shape), tuple(newShape)))
+
+    @staticmethod
+    def fromExpansion(found) -> "BroadcastStrides":
         made = BroadcastStrides.__new__(BroadcastStrides)
-        newShape, strides, made.dataCount, made.isNoOp = _expanded(tuple(shape), tuple(newShape))
-        made.shape, made.strides = list(newShape), list(strides)
+        shape, strides, made.dataCount, made.isNoOp = found
+        made.shape, made.strides = list(shape), list(strides)
         return made
 
     def __call__(self, i: int) -> int:
@@ -193,7 +197,8 @@ class BroadcastStrides:
 
 
 @functools.lru_cache(maxsize=4096)
-def _expanded(shape, newShape):
+def expansion(shape, newShape):
+    """What BroadcastStrides.expanding finds for two tuples."""
     assert len(newShape) >= len(shape), "cannot broadcast %s to shorter shape %s" % (list(shape), list(newShape))
     extra = len(newShape) - len(shape)
     strides = [0] * extra

@@ -11,6 +11,7 @@ ReduceRepeat.swift:67-331, ScatterGather.swift:51-110, Index.swift:36-410,
 Broadcast.swift:115-245, Elemwise.swift:187-322, Softmax.swift, FusedOps.swift,
 Comparison.swift, When.swift, ConcatSplit.swift.
 """
+import functools
 from typing import List, Optional, Sequence
 
 import numpy as np
@@ -18,7 +19,7 @@ import numpy as np
 from .backend import Backend, convert_host_array
 from .descriptors import (BitwiseOp, BroadcastData, BroadcastStrides, ComparisonOp, DType, ElemwiseOp,
                           NumericBinaryOp, ReduceDims, ReduceOp, RepeatDims, ScatterGatherIndices,
-                          product, stridesForShape)
+                          expansion, product, stridesForShape)
 
 _SCALARS = (int, float, np.floating, np.integer)
 
@@ -203,6 +204,19 @@ def _index_list(items, inShape) -> TensorIndexResult:
 
 # ---------------------------------------------------------------- Tensor
 
+@functools.lru_cache(maxsize=4096)
+def _reduceDims(shape, axis) -> ReduceDims:
+    """`shape` seen from its axis `axis`. A program's calls repeat a few pairs, and a ReduceDims is never written: kept by value."""
+    return ReduceDims(product(shape[:axis]), int(shape[axis]), product(shape[axis + 1:]))
+
+
+@functools.lru_cache(maxsize=4096)
+def _broadcasts(shapes):
+    """The shape that `shapes` broadcast to, and how each gets there; kept by value like _reduceDims."""
+    newShape = tuple(int(n) for n in Tensor.broadcastShape(shapes))
+    return newShape, [expansion(shape, newShape) for shape in shapes]
+
+
 class Tensor:
     def __init__(self, data=None, shape=None, dtype=None, reverse=False, dataHandle=None):
         """Tensor(data:shape:dtype:) uploads host values through `Backend.collection`
@@ -346,8 +360,8 @@ class Tensor:
 
     @staticmethod
     def lazyBroadcast(ts: Sequence["Tensor"]):
-        newShape = Tensor.broadcastShape([t.shape for t in ts])
-        return newShape, [t.expandStrides(newShape) for t in ts]
+        newShape, expansions = _broadcasts(tuple([tuple(t.shape) for t in ts]))
+        return list(newShape), [BroadcastStrides.fromExpansion(e) for e in expansions]
 
     def expand(self, shape) -> "Tensor":
         shape = shape.shape if isinstance(shape, Tensor) else list(shape)
@@ -547,7 +561,7 @@ class Tensor:
             return ReduceDims(1, product(self.shape), 1)
         axis = self.positiveAxis(axis)
         assert 0 <= axis < len(self.shape), "axis %d out of bounds for shape %s" % (axis, self.shape)
-        return ReduceDims(product(self.shape[:axis]), self.shape[axis], product(self.shape[axis + 1:]))
+        return _reduceDims(tuple(self.shape), axis)
 
     def reduce(self, op: ReduceOp, axis=None, keepdims=False) -> "Tensor":
         axis = self.positiveAxis(axis)
@@ -706,8 +720,7 @@ class Tensor:
     def logSoftmax(self, axis=-1) -> "Tensor":
         posAxis = self.positiveAxis(axis)
         assert 0 <= posAxis < len(self.shape)
-        dims = ReduceDims(product(self.shape[:posAxis]), self.shape[posAxis], product(self.shape[posAxis + 1:]))
-        return self._new(Backend.current().logSoftmax(self.data, dims, self.dtype))
+        return self._new(Backend.current().logSoftmax(self.data, _reduceDims(tuple(self.shape), posAxis), self.dtype))
 
     def softmax(self, axis=-1) -> "Tensor":
         # Softmax.swift:64-66 ignores `axis` and always normalises the last axis.
