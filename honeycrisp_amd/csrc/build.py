@@ -31,6 +31,8 @@ KERNELS = [
     ("gemm_dma", "gemm_dma.hip", ["-ffp-contract=off"]),
     ("gemm_dma2", "gemm_dma2.hip", ["-ffp-contract=off"]),
     ("gemm_mi16", "gemm_mi16.hip", ["-ffp-contract=off"]),
+    # a third build of this source: tiles over a part of K, and their sum
+    ("gemm_parts", "gemm_dma2.hip", ["-ffp-contract=off", "-DHC_GEMM_PARTS=1"]),
     ("gemm_ks", "gemm_ks.hip", ["-ffp-contract=off"]),
     # the same four sources once more: kernels named *_m whose write-out applies the operations a
     # recording merged into the product (the plain kernels above contain none of that code)
@@ -61,7 +63,7 @@ def _run(cmd):
 # sit at the 256-VGPR limit; the edge kernels' write-out needs a few registers more): up to 96 bytes
 # per lane in the plain kernels, up to 128 in the kernels with merged epilogues.
 NO_SCRATCH = {"gemm_dma": 96, "gemm_dma2": 96, "gemm_mi16": 96, "gemm_f16_fast": 16,
-              "gemm_ks": 0, "gemm_ks_m": 0,
+              "gemm_ks": 0, "gemm_ks_m": 0, "gemm_parts": 0,
               "gemm_dma_m": 128, "gemm_dma2_m_f16": 128, "gemm_dma2_m_f32": 128, "gemm_mi16_m": 128}
 
 

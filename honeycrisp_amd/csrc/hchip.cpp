@@ -35,6 +35,7 @@ extern const unsigned char hc_image_gemm_f16_fast[], hc_image_gemm_f16_fast_end[
 extern const unsigned char hc_image_gemm_dma[], hc_image_gemm_dma_end[];
 extern const unsigned char hc_image_gemm_dma2[], hc_image_gemm_dma2_end[];
 extern const unsigned char hc_image_gemm_mi16[], hc_image_gemm_mi16_end[];
+extern const unsigned char hc_image_gemm_parts[], hc_image_gemm_parts_end[];
 extern const unsigned char hc_image_gemm_ks[], hc_image_gemm_ks_end[];
 extern const unsigned char hc_image_gemm_dma_m[], hc_image_gemm_dma_m_end[];
 extern const unsigned char hc_image_gemm_dma2_m_f16[], hc_image_gemm_dma2_m_f16_end[];
@@ -333,6 +334,7 @@ extern "C" int hc_init(int device, hc_ctx** out) {
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma, hc_image_gemm_dma_end, "gemm_dma");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma2, hc_image_gemm_dma2_end, "gemm_dma2");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_mi16, hc_image_gemm_mi16_end, "gemm_mi16");
+  if (s == HC_OK) s = load_image(ctx, hc_image_gemm_parts, hc_image_gemm_parts_end, "gemm_parts");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_ks, hc_image_gemm_ks_end, "gemm_ks");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma_m, hc_image_gemm_dma_m_end, "gemm_dma_m");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma2_m_f16, hc_image_gemm_dma2_m_f16_end, "gemm_dma2_m_f16");

@@ -401,6 +401,19 @@ typedef struct {
   void* g_c[4];
   const void* g_ep[3][4];
 } hck_gemm_args;
+
+/* A product in parts of K: part i (blockIdx.y) covers k = i * kchunk .. (kchunk a multiple of 64; a_bs, b_bs: what lies between
+ * two parts' first elements), c: fp32 partial sums [parts][M][N], N a multiple of 4. */
+typedef struct {
+  hck_gemm_args g;
+  uint32_t kchunk;
+} hck_gemm_part_args;
+/* ... and their sum: c[row * c_rs + col], col < N, from sums [parts][M][ld] */
+typedef struct {
+  const void* sums;
+  void* c;
+  uint32_t M, N, ld, c_rs, parts;
+} hck_gemm_part_sum_args;
 #define HCK_GEMM_GROUP 4
 
 #define HCK_EP_NONE 0

@@ -234,15 +234,17 @@ template <typename T, int ROWS, int MODE> struct DmaOperand {
 // (waits, barrier, scalar bookkeeping: the four-stage pipeline of 64-byte slices spends about 275
 // cycles per slice on a 64 x 64 tile, of which the MFMAs are 128), so the slices should be long,
 // and with one workgroup per compute unit only a deep ring keeps enough loads in flight.
-template <typename T, int BM, int BN, int MODE_A, int MODE_B, bool EDGE, bool ONE = false, bool RING4 = false>
+// kchunk (the third build, see the kernels at the end): the workgroup multiplies the kchunk values of K from blockIdx.y * kchunk on and
+// stores TO = float; 0: all of K.
+template <typename T, int BM, int BN, int MODE_A, int MODE_B, bool EDGE, bool ONE = false, bool RING4 = false, typename TO = T>
 __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds0, char* lds1, char* lds2 = nullptr,
-                                               char* lds3 = nullptr) {
+                                               char* lds3 = nullptr, const uint32_t kchunk = 0) {
   static_assert(!(ONE && RING4), "one slice needs no ring");
   constexpr int MT = BM / 64, NT = BN / 64;
   constexpr int SLOTS = MT * NT;
   typedef DmaOperand<T, BM, MODE_A> OpA;
   typedef DmaOperand<T, BN, MODE_B> OpB;
-  constexpr bool F32 = sizeof(T) == 4;
+  constexpr bool F32 = sizeof(T) == 4, F32_OUT = sizeof(TO) == 4;
   constexpr uint32_t BK = 128 / sizeof(T);  // K-slice of one stage
   constexpr int READS = OpA::READS + OpB::READS;
   constexpr int NDMA = OpA::NI + OpB::NI;  // per wave and K-step
@@ -276,8 +278,9 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
 #else
   const T* A = (const T*)p.a + batch * p.a_bs;
   const T* B = (const T*)p.b + batch * p.b_bs;
-  T* C = (T*)p.c + batch * p.c_bs;
+  TO* C = (TO*)p.c + batch * p.c_bs;
 #endif
+  const uint32_t K = kchunk == 0 ? p.K : min(p.K - batch * kchunk, kchunk);
 
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
@@ -295,7 +298,7 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
   OpB ob;
   oa.init(p.a_rs, p.a_cs, m0, wm, EDGE ? p.a_lim : 0);
   ob.init(p.b_cs, p.b_rs, n0, wn, EDGE ? p.b_lim : 0);
-  const uint32_t kend = EDGE ? p.K : 0;
+  const uint32_t kend = EDGE ? K : 0;
 
   struct Frags {
     Chunk a[MT];
@@ -346,11 +349,11 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
   // units of the first window part (sub-step 3): [0, U0)
   constexpr int U0 = (SLOTS * NDMA + W - 1) / W < NDMA ? (SLOTS * NDMA + W - 1) / W : NDMA;
 
-  const uint32_t nk = (p.K + BK - 1) / BK;
+  const uint32_t nk = (K + BK - 1) / BK;
   auto kclamp = [&](uint32_t j) { return (j < nk ? j : nk - 1) * BK; };  // steps past the end repeat the last one
   // (edge kernels) K is not a whole number of 16-byte pieces: the last slice of a K-contiguous
   // operand is cleaned up after it has landed
-  const bool ktail = EDGE && p.K % (16 / sizeof(T)) != 0;
+  const bool ktail = EDGE && K % (16 / sizeof(T)) != 0;
   auto zero_tail = [&](char* stage, uint32_t k0) {
     oa.zero_k_tail(stage, k0, kend);
     ob.zero_k_tail(stage + A_BYTES, k0, kend);
@@ -497,7 +500,7 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
   lds_barrier();
   constexpr uint32_t MINE = ONE ? (BM + BN) * 32 : (BM + BN) * 64;  // bytes of LDS per wave for the write-out
   char* mine = ONE ? lds0 + wave * MINE : (wave < 2 ? lds0 : lds1) + (wave & 1) * MINE;
-  constexpr uint32_t ES = sizeof(T), WN = BN / 2, RB = WN * ES, UNITS = RB / 16;
+  constexpr uint32_t ES = sizeof(TO), WN = BN / 2, RB = WN * ES, UNITS = RB / 16;
   constexpr uint32_t SLAB = 32 * RB, NSLAB = MINE / SLAB;
   static_assert(NSLAB >= 1 && (32 * UNITS) % 64 == 0, "a slab must fit half a stage");
   // (the swizzle stays inside aligned groups of USWZ + 1 units, a divisor of UNITS)
@@ -540,7 +543,7 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
       for (int j = 0; j < NT; j++) {
 #pragma unroll
         for (int g = 0; g < 4; g++) {
-          if constexpr (F32) {
+          if constexpr (F32_OUT) {
             floatx4 h;
 #pragma unroll
             for (int e = 0; e < 4; e++) h[e] = acc[i][j][4 * g + e];
@@ -560,7 +563,7 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
           const uint32_t piece = it * 64 + lane, r = piece / UNITS, u = piece % UNITS;
           const Chunk v = *reinterpret_cast<const Chunk*>(slab + r * RB + ((u ^ unit_swz(r)) * 16));
           const uint32_t row = m0 + wm + i * 32 + r, col = n0 + wn + u * (16 / ES);
-          gemm_store_piece<T, Chunk, EDGE, gemm_loose_stores<EDGE, BM, BN>()>(C + (size_t)row * p.c_rs + col, row, col, p.M, p.N, v, slab + r * RB + ((u ^ unit_swz(r)) * 16));
+          gemm_store_piece<TO, Chunk, EDGE, gemm_loose_stores<EDGE, BM, BN>()>(C + (size_t)row * p.c_rs + col, row, col, p.M, p.N, v, slab + r * RB + ((u ^ unit_swz(r)) * 16));
         }
       }
 #ifdef HC_GEMM_MERGED
@@ -640,6 +643,61 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
     __shared__ __attribute__((aligned(1024))) char lds3[(BM + BN) * 128];                             \
     gemm_dma2_impl<T, BM, BN, AM, BMODE, true, false, true>(p, lds0, lds1, lds2, lds3);               \
   }
+#ifdef HC_GEMM_PARTS
+// Products of few tiles over a long K: as many workgroups as compute units, each a tile over a part of K (blockIdx.y) into fp32 partial
+// sums, which a second launch adds up, parts in order. 64 x 64 tiles fetch whole cache lines, so that a part of K takes little
+// longer than its bytes need.
+#define DEF_PART(T, TN, AN, AM, BNAME, BMODE, E, SUFFIX)                                               \
+  extern "C" __global__ __launch_bounds__(256) void hc_gemm_##TN##_part_64x64_##AN##BNAME##SUFFIX(hck_gemm_part_args p) { \
+    __shared__ __attribute__((aligned(1024))) char lds0[128 * 128];                                   \
+    __shared__ __attribute__((aligned(1024))) char lds1[128 * 128];                                   \
+    __shared__ __attribute__((aligned(1024))) char lds2[128 * 128];                                   \
+    __shared__ __attribute__((aligned(1024))) char lds3[128 * 128];                                   \
+    gemm_dma2_impl<T, 64, 64, AM, BMODE, E, false, true, float>(p.g, lds0, lds1, lds2, lds3, p.kchunk); \
+  }
+#define DEF_PART_LAYOUT(T, TN, AN, AM, BNAME, BMODE) \
+  DEF_PART(T, TN, AN, AM, BNAME, BMODE, false, )     \
+  DEF_PART(T, TN, AN, AM, BNAME, BMODE, true, _e)
+#define DEF_PARTS(T, TN)                          \
+  DEF_PART_LAYOUT(T, TN, k, DMA_K, k, DMA_K)      \
+  DEF_PART_LAYOUT(T, TN, k, DMA_K, n, DMA_MN)     \
+  DEF_PART_LAYOUT(T, TN, m, DMA_MN, k, DMA_K)     \
+  DEF_PART_LAYOUT(T, TN, m, DMA_MN, n, DMA_MN)
+DEF_PARTS(half_t, f16)
+DEF_PARTS(float, f32)
+
+// A lane adds up four neighbouring outputs (a row of partial sums is a whole number of those), loads of four parts at a time on their way.
+template <typename T> __device__ __forceinline__ void gemm_part_sum_impl(const hck_gemm_part_sum_args& p) {
+  const uint32_t per_row = p.ld / 4, q = blockIdx.x * HCK_BLOCK + threadIdx.x;
+  if (q >= p.M * per_row) return;
+  const uint32_t row = q / per_row, col = (q - row * per_row) * 4;
+  const size_t part = (size_t)p.M * per_row;
+  const floatx4* src = (const floatx4*)p.sums + q;
+  floatx4 s = src[0];
+  uint32_t i = 1;
+  for (; i + 4 <= p.parts; i += 4) {
+    floatx4 v[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) v[u] = src[(i + u) * part];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++) s += v[u];
+  }
+  for (; i < p.parts; i++) s += src[i * part];
+  T y[4];
+#pragma unroll
+  for (int x = 0; x < 4; x++) y[x] = narrow<T>(s[x]);
+  T* dst = (T*)p.c + (size_t)row * p.c_rs + col;
+  if (col + 4 <= p.N) {
+    store_vec_loose<T, 4>(dst, y);
+  } else {
+#pragma unroll
+    for (uint32_t x = 0; x < 3; x++)
+      if (col + x < p.N) dst[x] = y[x];
+  }
+}
+extern "C" __global__ __launch_bounds__(HCK_BLOCK) void hc_gemm_part_sum_f16(hck_gemm_part_sum_args p) { gemm_part_sum_impl<half_t>(p); }
+extern "C" __global__ __launch_bounds__(HCK_BLOCK) void hc_gemm_part_sum_f32(hck_gemm_part_sum_args p) { gemm_part_sum_impl<float>(p); }
+#else
 #define DEF_DMA_RING4_TILE(T, TN, BM, BN)                                                             \
   DEF_DMA_RING4(T, TN, BM, BN, k, DMA_K, k, DMA_K)                                                    \
   DEF_DMA_RING4(T, TN, BM, BN, k, DMA_K, n, DMA_MN)                                                   \
@@ -687,3 +745,4 @@ DEF_DMA_TILE(float, f32, 256, 192)
 DEF_DMA_TILE(float, f32, 192, 256)
 DEF_DMA_TILE(float, f32, 192, 192)
 #endif
+#endif   // HC_GEMM_PARTS

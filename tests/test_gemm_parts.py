@@ -1,0 +1,62 @@
+"""Products of few tiles over a long K, computed in parts of K that are added up: the ends of tiles, parts and rows, every layout."""
+import numpy as np
+import pytest
+
+from honeycrisp_amd.descriptors import DType
+from honeycrisp_amd.tensor import Tensor
+
+pytestmark = pytest.mark.gpu
+
+# (m, k, n): one tile and the most parts; parts that end inside a 64 of K, with it, and one element after; whole and ragged tiles; rows that
+# are no multiple of 16 bytes or of 4 elements; the fewest outputs; the most tiles there are (128 on a device of 256 compute units) and one more
+SHAPES = [(64, 3072, 64), (64, 3136, 32), (5, 3073, 411), (5, 4097, 411), (65, 3137, 63), (16, 3200, 4096), (200, 4099, 130), (512, 3136, 1024),
+          (127, 8191, 33), (300, 5000, 256), (40, 3330, 1001), (520, 3200, 1024)]
+
+
+@pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
+@pytest.mark.parametrize("m,k,n", SHAPES, ids=str)
+def test_against_float64(hip_backend, dtype, m, k, n):
+    rng = np.random.default_rng(m * k + n)
+    with hip_backend.use():
+        for ta in (False, True):
+            for tb in (False, True):
+                for to in (False, True):
+                    a = (rng.standard_normal((k, m) if ta else (m, k)) / np.sqrt(k)).astype(dtype.numpy)
+                    b = rng.standard_normal((n, k) if tb else (k, n)).astype(dtype.numpy)
+                    x, y = Tensor(data=a, dtype=dtype), Tensor(data=b, dtype=dtype)
+                    a, b = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)
+                    want, size = a @ b, np.abs(a) @ np.abs(b)
+                    if to:
+                        want, size = want.T, size.T
+                    got = Tensor.matmul(x, ta, y, tb, to).numpy().astype(np.float64)
+                    # k additions in fp32, each off by half a last place of a partial sum, and one rounding to the result's type
+                    bound = k * 2.0 ** -24 * size + (2.0 ** -11 * np.abs(want) + 2.0 ** -24 if dtype == DType.float16 else 0)
+                    assert np.all(np.abs(got - want) <= bound), (ta, tb, to, np.max(np.abs(got - want) / size))
+
+
+def test_a_recording_returns_the_bits_of_the_call(hip_backend):
+    rng = np.random.default_rng(7)
+    with hip_backend.use():
+        x = Tensor(data=rng.standard_normal((48, 4100)).astype(np.float32), dtype=DType.float16)
+        w = Tensor(data=(rng.standard_normal((4100, 300)) / 64).astype(np.float32), dtype=DType.float16)
+        bias = Tensor(data=rng.standard_normal(300).astype(np.float32), dtype=DType.float16)
+        f = lambda: (Tensor.matmul(x, False, w, False, False) + bias).gelu()
+        want = f().numpy()
+        with hip_backend.capture() as recording:
+            out = f()
+        for _ in range(3):
+            recording.graph.launch()
+            np.testing.assert_array_equal(out.numpy().view(np.uint16), want.view(np.uint16))
+        with hip_backend.batching():
+            got = f()
+        np.testing.assert_array_equal(got.numpy().view(np.uint16), want.view(np.uint16))
+
+
+@pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
+def test_an_infinity_or_a_nan_stays_in_its_row_and_column(hip_backend, dtype):
+    m, k, n = 70, 3100, 66
+    a, b = np.ones((m, k), np.float32), np.ones((k, n), np.float32)
+    a[3, 3099], a[69, 0], b[1024, 65] = np.inf, np.nan, -np.inf
+    with hip_backend.use(), np.errstate(invalid="ignore"):
+        got = Tensor.matmul(Tensor(data=a, dtype=dtype), False, Tensor(data=b, dtype=dtype), False, False).numpy()
+        np.testing.assert_array_equal(got, (a.astype(np.float64) @ b.astype(np.float64)).astype(dtype.numpy))
