@@ -414,6 +414,16 @@ typedef struct {
   void* c;
   uint32_t M, N, ld, c_rs, parts;
 } hck_gemm_part_sum_args;
+
+/* Two matrices of 2-byte elements copied to rows of whole cache lines: out[r * ld + c] = in[r * cols + c], zeros from cols on;
+ * ld a multiple of 64. Workgroups below `split` copy the first. */
+typedef struct {
+  const void* in[2];
+  void* out[2];
+  uint32_t rows[2];
+  uint32_t cols, ld, split;
+} hck_copy_lines_args;
+#define HCK_COPY_LINES 4   /* pieces of 16 bytes per lane */
 #define HCK_GEMM_GROUP 4
 
 #define HCK_EP_NONE 0

@@ -9,7 +9,7 @@ pytestmark = pytest.mark.gpu
 
 # (m, k, n): one tile and the most parts; parts that end inside a 64 of K, with it, and one element after; whole and ragged tiles; rows that
 # are no multiple of 16 bytes or of 4 elements; the fewest outputs; the most tiles there are (128 on a device of 256 compute units) and one more
-SHAPES = [(64, 3072, 64), (64, 3136, 32), (5, 3073, 411), (5, 4097, 411), (65, 3137, 63), (16, 3200, 4096), (200, 4099, 130), (512, 3136, 1024),
+SHAPES = [(64, 3072, 64), (64, 3136, 80), (9, 3073, 461), (5, 4097, 821), (65, 3137, 63), (16, 3200, 4096), (200, 4099, 130), (512, 3136, 1024),
           (127, 8191, 33), (300, 5000, 256), (40, 3330, 1001), (520, 3200, 1024)]
 
 
