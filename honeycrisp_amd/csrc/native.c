@@ -158,9 +158,6 @@ static Call begin(Context* c, PyObject* const* a, Py_ssize_t n, Py_ssize_t want)
   if (n != want) {
     PyErr_Format(PyExc_TypeError, "%zd arguments instead of %zd", n, want);
     call.failed = 1;
-  } else if (!c->ctx) {
-    PyErr_SetString(PyExc_RuntimeError, "the backend is closed");
-    call.failed = 1;
   }
   return call;
 }
@@ -270,7 +267,7 @@ static PyObject* end(Call* call, PyObject* result) {
   return result;
 }
 
-/* n buffers of `bytes` into out[], then `expr`; the results, or the backend's exception */
+/* n buffers of `bytes` into out[], then `expr`; the results, or the backend's exception (also once it is closed: hc_malloc refuses a null context) */
 #define RUN(n, bytes, expr)                                                            \
   hc_ctx* const ctx = c->ctx;                                                          \
   void* out[n] = {NULL};                                                               \

@@ -17,7 +17,7 @@ TYPED = r"""
 #include <stdlib.h>
 #include "hchip.h"
 int live, calls, fail; long long seen[16]; hc_strides shape;
-int hc_malloc(hc_ctx* c, size_t n, void** p) { if (fail == 2 && live) return HC_ERR_ALLOC; *p = malloc(1); live++; return 0; }
+int hc_malloc(hc_ctx* c, size_t n, void** p) { if (!c) return HC_ERR_INVALID; if (fail == 2 && live) return HC_ERR_ALLOC; *p = malloc(1); live++; return 0; }
 int hc_free(hc_ctx* c, void* p) { free(p); live--; return 0; }
 int hc_binary_op(hc_ctx* c, int op, int t, const void* a, const hc_strides* sa, const void* b, const hc_strides* sb, void* o) {
   seen[0] = op; seen[1] = t; seen[2] = (long long)a; seen[3] = (long long)b; shape = *sa; calls++; return fail ? HC_ERR_UNSUPPORTED : 0; }
@@ -139,8 +139,9 @@ def test_other_data_goes_through_the_backend(lib, fake):
 def test_after_close_nothing_is_called_or_given_back(lib, fake):
     x = fake.made(8)
     fake._native.close()
-    with pytest.raises(RuntimeError):
+    with pytest.raises(Refused) as e:
         fake.made(8)
+    assert e.value.args[0] == 1
     del x
     assert value(lib, "live") == 1
 
