@@ -22,9 +22,10 @@ __device__ __forceinline__ float sigmoid_hw(float x) {
   const float inside = __builtin_amdgcn_rcpf(1.0f + exp_hw(-x));
   return x < -20.0f ? 0.0f : (x > 20.0f ? 1.0f : inside);
 }
-// GELU for results that are rounded to fp16: (1 + tanh u) / 2 is 1 / (1 + exp(-2u)), so a value is f * rcp(1 + exp2(z)) with z a cubic of f:
-// seven instructions, two of them quarter rate, with no subtraction next to 1 and nothing to select (exp2 gives 0 or infinity past its range, and
-// rcp(infinity) is 0). With the tanh written out it was 22: a 2048 x 512 x 2048 product with bias and GELU merged 12.1 us, 10.9 now (without the GELU 9.9); 4 M
+// GELU for results that are rounded to fp16: (1 + tanh u) / 2 is 1 / (1 + exp(-2u)) = s, so a value is f * s with s = rcp(1 + exp2(z)) and z a cubic
+// of f: nine instructions, two of them quarter rate, and nothing to select (exp2 gives 0 or infinity past its range, and
+// rcp(infinity) is 0). Two of the nine take s to s - 1/2 and back: half of the reference's tanh u = 2 s - 1 and 1 + tanh u, rounded where it rounds
+// them, so that values far below 0 lose the digits there that they lose in the reference. With the tanh written out it was 22: a 2048 x 512 x 2048 product with bias and GELU merged 12.1 us, 10.9 now (without the GELU 9.9); 4 M
 // values 6.1 -> 5.2. -2 u log2(e): the constants of the reference's formula, multiplied out.
 __device__ __forceinline__ float gelu_exponent(float f) { return f * fmaf(f * f, -0.102943237f, -2.30220820f); }
 
@@ -40,7 +41,7 @@ __device__ __forceinline__ float cube(float f) {
 // ElemwiseOp.geluApprox (Elemwise.swift:109-111) on a value of tensor type T held as float; the
 // caller multiplies by the scale (1 without scales) and rounds to T, as the element-wise kernel does.
 template <bool HALF> __device__ __forceinline__ float gelu_approx(float f) {
-  if (HALF) return f * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gelu_exponent(f)));
+  if (HALF) return f * (0.5f + (__builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(gelu_exponent(f))) - 0.5f));
   return 0.5f * f * (1.0f + safe_tanh(0.797884561f * (f + 0.044715f * cube(f))));
 }
 
