@@ -25,8 +25,8 @@ __device__ __forceinline__ float sigmoid_hw(float x) {
 // GELU for results that are rounded to fp16: (1 + tanh u) / 2 is 1 / (1 + exp(-2u)) = s, so a value is f * s with s = rcp(1 + exp2(z)) and z a cubic
 // of f: nine instructions, two of them quarter rate, and nothing to select (exp2 gives 0 or infinity past its range, and
 // rcp(infinity) is 0). Two of the nine take s to s - 1/2 and back: half of the reference's tanh u = 2 s - 1 and 1 + tanh u, rounded where it rounds
-// them, so that values far below 0 lose the digits there that they lose in the reference. With the tanh written out it was 22: a 2048 x 512 x 2048 product with bias and GELU merged 12.1 us, 10.9 now (without the GELU 9.9); 4 M
-// values 6.1 -> 5.2. -2 u log2(e): the constants of the reference's formula, multiplied out.
+// them, so that values far below 0 lose the digits there that they lose in the reference. With the tanh written out it was 22: a 2048 x 512 x 2048 product with bias and GELU merged 12.3 us, 11.2 now (without the GELU 9.9); 4 M
+// values 6.1 -> 5.3. -2 u log2(e): the constants of the reference's formula, multiplied out.
 __device__ __forceinline__ float gelu_exponent(float f) { return f * fmaf(f * f, -0.102943237f, -2.30220820f); }
 
 // powf(f, 3.0f) of the reference formula: the cube formed in double and rounded once is the
