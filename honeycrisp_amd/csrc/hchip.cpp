@@ -2588,7 +2588,12 @@ extern "C" int hc_gather(hc_ctx* ctx, int dtype, const void* in, const void* ind
   return launch(ctx, name, ceil_div(total, HCK_BLOCK), 1, &k, sizeof(k));
 }
 
-static const uint64_t SCATTER_LISTS_ROWS = 786432;   // (the largest number timed: 0.95 to 0.99 of the time of the five launches there; 65536 rows into 32000 0.80, 256 into 8192 0.48)
+// Source rows of which one launch makes the lists of a scatter. Dense indices, of which a lane has sixteen on their way: the largest number timed, 0.95 to 0.99 of
+// the time of the five launches there; 65536 rows into 32000 0.80, 256 into 8192 0.48.
+static const uint64_t SCATTER_LISTS_ROWS = 786432;
+// Several outer slices or indices read through strides, one at a time and with a division each: 66 shapes of 4096 to 24576 rows 0.40 to 0.89 of the time of
+// the five launches, 28 of 32768 and 33000 0.54 to 1.01, 65536 (64 x 1024 into 512) 1.14, 524288 (64 x 8192 into 512) 1.79.
+static const uint64_t SCATTER_LISTS_STRIDED_ROWS = 24576;
 
 extern "C" int hc_scatter(hc_ctx* ctx, int dtype, const void* in, const void* indices,
                           const hc_strides* idx_strides, void* out, int64_t outer, int64_t middle,
@@ -2638,15 +2643,21 @@ extern "C" int hc_scatter(hc_ctx* ctx, int dtype, const void* in, const void* in
       const uint64_t n_buckets = (uint64_t)outer * (uint64_t)middle, n_rows = (uint64_t)outer * (uint64_t)out_count;
       Scratch scratch(ctx);
       void *counters = nullptr, *starts = nullptr, *list = nullptr;
+      hck_scatter_rows_args k;
+      memset(&k, 0, sizeof(k));
+      int vec;
+      uint64_t rows;
+      const hc_strides* ops[] = {&row_strides};
+      const void* ptrs[] = {indices};
+      HC_TRY(make_bcast(1, ops, ptrs, out, 1, &k.idx, &vec, &rows));
       // One launch for the lists where its reading of every index by every workgroup is cheaper than the launches of the other way
       // (hc_scatter_rows_lists).
+      const bool dense = outer == 1 && k.idx.n_outer == 0 && k.idx.inner_stride[0] == 1;   // (as the kernel has it)
       const uint32_t list_rows = (uint32_t)std::max<uint64_t>(32, ceil_div(n_buckets, (uint64_t)ctx->props.multiProcessorCount));
-      const bool one_launch = n_rows <= SCATTER_LISTS_ROWS && list_rows <= HCK_SCATTER_LIST_ROWS;
+      const bool one_launch = n_rows <= (dense ? SCATTER_LISTS_ROWS : SCATTER_LISTS_STRIDED_ROWS) && list_rows <= HCK_SCATTER_LIST_ROWS;
       HC_TRY(scratch.get((one_launch ? 1 : 2) * n_buckets * sizeof(int64_t), &counters));  // counts, then cursors
       HC_TRY(scratch.get(n_buckets * sizeof(int64_t), &starts));
       HC_TRY(scratch.get(n_rows * sizeof(uint32_t), &list));
-      hck_scatter_rows_args k;
-      memset(&k, 0, sizeof(k));
       k.in = in;
       k.indices = (const int64_t*)indices;
       k.out = out;
@@ -2661,11 +2672,6 @@ extern "C" int hc_scatter(hc_ctx* ctx, int dtype, const void* in, const void* in
       k.n_buckets = (uint32_t)n_buckets;
       k.list_rows = list_rows;
       k.starts_out = (int64_t*)starts;
-      int vec;
-      uint64_t rows;
-      const hc_strides* ops[] = {&row_strides};
-      const void* ptrs[] = {indices};
-      HC_TRY(make_bcast(1, ops, ptrs, out, 1, &k.idx, &vec, &rows));
       if (one_launch) {
         HC_TRY(launch(ctx, "hc_scatter_rows_lists", ceil_div(n_buckets, list_rows), 1, &k, sizeof(k), 1024));
       } else {

@@ -150,7 +150,7 @@ HC_KERNEL void hc_scatter_rows_fill(hck_scatter_rows_args p) {
 
 // Passes 1 and 2 and the scan between them in one launch (up to the host's number of source rows): every workgroup owns `list_rows`
 // consecutive destination rows and reads all indices, so that it finds where its slices of `list` begin without a word from the others. It is
-// bound by those reads, 8 bytes per source row and workgroup from L2, and for few rows by its launch and three barriers. The whole scatter of rows of
+// bound by those reads, 8 bytes per source row and workgroup from L2, and for few rows by its launch and five barriers. The whole scatter of rows of
 // 1 KiB, in us, with counters cleared, counted, scanned (two launches) and filled instead / now: 256 rows into 8192 20.2 / 9.6, 2048 into
 // 8192 21.9 / 11.2, 65536 into 32000 53.9 / 42.9 (eight loads in flight; one at a time 50.3), 786432 into 4000 231 / 229. Row numbers wait in LDS for the
 // scan; a workgroup with more than SCATTER_HELD_ROWS of them reads the indices again instead.

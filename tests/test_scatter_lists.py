@@ -3,6 +3,7 @@ past its number of destinations. Whole numbers: every sum is exact."""
 import numpy as np
 import pytest
 
+from honeycrisp_amd.descriptors import BroadcastData, BroadcastStrides, DType, ScatterGatherIndices
 from honeycrisp_amd.tensor import Tensor
 from recorded_kernels import kernels_of
 
@@ -30,15 +31,35 @@ def test_scatter_of_rows(hip_backend, capfd, n, rows):
     assert not got.any()
 
 
-@pytest.mark.parametrize("outer,n,rows", [(3, 1000, 50), (70, 40, 300)])
-def test_scatter_along_an_inner_axis(hip_backend, outer, n, rows):
+# (up to 24576 rows here, whose indices are read one at a time: both sides of that)
+@pytest.mark.parametrize("outer,n,rows", [(3, 1000, 50), (70, 40, 300), (24, 1024, 40), (24, 1025, 40)])
+def test_scatter_along_an_inner_axis(hip_backend, capfd, outer, n, rows):
     """Destinations of several outer slices, indices of one slice for all of them and of their own."""
     rng = np.random.default_rng(outer)
     x = rng.integers(-2, 3, size=(outer, n, 256)).astype(np.float32)
     for shape in ((1, n, 1), (outer, n, 1)):
         ids = rng.integers(0, rows, size=shape)
         with hip_backend.use():
-            got = Tensor(data=x).scatter(1, rows, Tensor(data=ids)).numpy()
+            sources, index = Tensor(data=x), Tensor(data=ids)
+            kernels = kernels_of(hip_backend, capfd, lambda: sources.scatter(1, rows, index))
+            got = sources.scatter(1, rows, index).numpy()
+        assert ("hc_scatter_rows_lists" in kernels) == (outer * n <= 24576) != ("hc_scatter_rows_count" in kernels)
         want = np.zeros((outer, rows, 256), np.float32)
         np.add.at(want, (np.arange(outer)[:, None], np.broadcast_to(ids, (outer, n, 1))[..., 0]), x)
         assert np.array_equal(got, want)
+
+
+@pytest.mark.parametrize("n", [24576, 24577])
+def test_indices_read_through_strides(hip_backend, capfd, n):
+    """One slice, one index for all rows: not the dense reading, and its limit."""
+    x = np.ones((n, 256), np.float32)
+    with hip_backend.use():
+        sources = Tensor(data=x)
+        index_data, strides = Tensor(data=np.array([3])).data, BroadcastStrides([n, 256], [0, 0])
+        call = lambda: hip_backend.scatter(sources.data, ScatterGatherIndices([5, 256], 0, BroadcastData(strides, index_data)), DType.float32)
+        kernels = kernels_of(hip_backend, capfd, call)
+        got = Tensor(dataHandle=call(), shape=[5, 256], dtype=DType.float32).numpy()
+    assert ("hc_scatter_rows_lists" in kernels) == (n <= 24576) != ("hc_scatter_rows_count" in kernels)
+    want = np.zeros((5, 256), np.float32)
+    want[3] = n
+    np.testing.assert_array_equal(got, want)
