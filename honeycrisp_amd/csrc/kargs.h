@@ -408,11 +408,12 @@ typedef struct {
   hck_gemm_args g;
   uint32_t kchunk;
 } hck_gemm_part_args;
-/* ... and their sum: c[row * c_rs + col], col < N, from sums [parts][M][ld] */
+/* ... and their sum: the whole product's g.c[row * g.c_rs + col], col < g.N, from sums [parts][g.M][ld]; kernels ending in _m then
+ * apply g.ep_*. (g first: what merges operations into a product finds it in the same place as in a launch of one.) */
 typedef struct {
+  hck_gemm_args g;
   const void* sums;
-  void* c;
-  uint32_t M, N, ld, c_rs, parts;
+  uint32_t ld, parts;
 } hck_gemm_part_sum_args;
 
 /* Two matrices of 2-byte elements copied to rows of whole cache lines: out[r * ld + c] = in[r * cols + c], zeros from cols on;

@@ -294,8 +294,8 @@ __device__ __forceinline__ void gemm_block_and_batch(uint32_t& block, uint32_t& 
 #define HC_GEMM_IS_MERGED 0
 #endif
 
-// The operations are applied to 16-byte pieces of finished outputs of type T (already rounded to
-// T), in order, each in float with one rounding to T: bit for bit what the separate broadcast-add /
+// The operations are applied to pieces of finished outputs of type T (already rounded to
+// T; 16 bytes, 8 where fp16 partial sums are added up), in order, each in float with one rounding to T: bit for bit what the separate broadcast-add /
 // element-wise kernels would have produced. A lane's pieces all lie in the same columns, so the row
 // operands (a bias) are fetched once per kernel; the matrix operand (at most one of the three
 // operations) is fetched for a few pieces at a time, all loads in flight before the first use.
@@ -364,14 +364,14 @@ template <typename T> __device__ __forceinline__ void gemm_zero_piece_tail(char*
   }
 }
 
-template <typename T, typename Chunk16>
-__device__ __forceinline__ Chunk16 gemm_epilogue_row_piece(uint32_t kind, const void* ptr, uint32_t col, bool col_ok) {
-  constexpr int V = 16 / sizeof(T);
-  static_assert(sizeof(Chunk16) == 16, "a 16-byte piece");
-  Chunk16 out = Chunk16{};
+template <typename T, typename Piece>
+__device__ __forceinline__ Piece gemm_epilogue_row_piece(uint32_t kind, const void* ptr, uint32_t col, bool col_ok) {
+  constexpr int V = sizeof(Piece) / sizeof(T);
+  static_assert(V % 4 == 0, "four outputs of an fp32 row at a time");
+  Piece out = Piece{};
   if (!col_ok) return out;
   if (kind == HCK_EP_ADD_ROW) {
-    out = *reinterpret_cast<const Chunk16*>((const T*)ptr + col);
+    out = *reinterpret_cast<const Piece*>((const T*)ptr + col);
   } else if (kind == HCK_EP_ADD_ROW_F32) {
     const float* src = (const float*)ptr + col;
     T y[V];
@@ -380,20 +380,20 @@ __device__ __forceinline__ Chunk16 gemm_epilogue_row_piece(uint32_t kind, const 
       const float4 w = *reinterpret_cast<const float4*>(src + e);
       y[e] = narrow<T>(w.x), y[e + 1] = narrow<T>(w.y), y[e + 2] = narrow<T>(w.z), y[e + 3] = narrow<T>(w.w);
     }
-    __builtin_memcpy(&out, y, 16);
+    __builtin_memcpy(&out, y, sizeof(out));
   }
   return out;
 }
 
 // the matrix operand's piece for the output piece at (row, col); one of the stages has one
-template <typename T, typename Chunk16>
-__device__ __forceinline__ Chunk16 gemm_epilogue_matrix_piece(const hck_gemm_args& p, const void* p0, const void* p1,
+template <typename T, typename Piece>
+__device__ __forceinline__ Piece gemm_epilogue_matrix_piece(const hck_gemm_args& p, const void* p0, const void* p1,
                                                               const void* p2, uint32_t row, uint32_t col) {
   // (stage picked with scalar selects, then a single load: no register is written twice)
   const bool s0 = p.ep_kind[0] == HCK_EP_ADD_MATRIX, s1 = p.ep_kind[1] == HCK_EP_ADD_MATRIX;
   const void* base = s0 ? p0 : s1 ? p1 : p2;
   const uint32_t ld = s0 ? p.ep_ld[0] : s1 ? p.ep_ld[1] : p.ep_ld[2];
-  return *reinterpret_cast<const Chunk16*>((const T*)base + (size_t)row * ld + col);
+  return *reinterpret_cast<const Piece*>((const T*)base + (size_t)row * ld + col);
 }
 
 // r0, r1, r2: the row operands of the three stages (gemm_epilogue_row_piece; passed as three values
@@ -402,17 +402,17 @@ __device__ __forceinline__ Chunk16 gemm_epilogue_matrix_piece(const hck_gemm_arg
 // activation: the host puts GELU only at the end of a list, and never together with a matrix
 // operand. (A loop over the stages with the operation picked inside cost 7 us on a 256 x 256 tile
 // for a single bias addition; this form costs 1 us.)
-template <typename T, typename Chunk16, bool MATRIX, bool GELU>
-__device__ __forceinline__ Chunk16 gemm_epilogue_apply(const hck_gemm_args& p, Chunk16 v, Chunk16 r0, Chunk16 r1, Chunk16 r2,
-                                                       Chunk16 matrix_piece) {
-  constexpr int V = 16 / sizeof(T);
+template <typename T, typename Piece, bool MATRIX, bool GELU>
+__device__ __forceinline__ Piece gemm_epilogue_apply(const hck_gemm_args& p, Piece v, Piece r0, Piece r1, Piece r2,
+                                                       Piece matrix_piece) {
+  constexpr int V = sizeof(Piece) / sizeof(T);
   T x[V];
-  __builtin_memcpy(x, &v, 16);
+  __builtin_memcpy(x, &v, sizeof(v));
   const uint32_t k0 = p.ep_kind[0], k1 = p.ep_kind[1], k2 = p.ep_kind[2];
-  auto add = [&](uint32_t kind, Chunk16 row) {
-    const Chunk16 w = MATRIX && kind == HCK_EP_ADD_MATRIX ? matrix_piece : row;
+  auto add = [&](uint32_t kind, Piece row) {
+    const Piece w = MATRIX && kind == HCK_EP_ADD_MATRIX ? matrix_piece : row;
     T y[V];
-    __builtin_memcpy(y, &w, 16);
+    __builtin_memcpy(y, &w, sizeof(w));
 #pragma unroll
     for (int e = 0; e < V; e++) x[e] = narrow<T>((float)x[e] + (float)y[e]);
   };
@@ -424,8 +424,8 @@ __device__ __forceinline__ Chunk16 gemm_epilogue_apply(const hck_gemm_args& p, C
 #pragma unroll
     for (int e = 0; e < V; e++) x[e] = narrow<T>(gelu_approx<sizeof(T) == 2>((float)x[e]) * 1.0f);
   }
-  Chunk16 out;
-  __builtin_memcpy(&out, x, 16);
+  Piece out;
+  __builtin_memcpy(&out, x, sizeof(out));
   return out;
 }
 

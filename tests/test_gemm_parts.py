@@ -4,6 +4,7 @@ import pytest
 
 from honeycrisp_amd.descriptors import DType
 from honeycrisp_amd.tensor import Tensor
+from recorded_kernels import kernels_of
 
 pytestmark = pytest.mark.gpu
 
@@ -34,22 +35,51 @@ def test_against_float64(hip_backend, dtype, m, k, n):
                     assert np.all(np.abs(got - want) <= bound), (ta, tb, to, np.max(np.abs(got - want) / size))
 
 
+def same_bits(hip, fn):
+    """fn() call by call, recorded (three replays) and batched."""
+    bits = lambda t: t.numpy().view(np.uint8)
+    want = [bits(t) for t in fn()]
+    with hip.capture() as recording:
+        outs = fn()
+    for _ in range(3):
+        recording.graph.launch()
+        assert all(np.array_equal(bits(t), w) for t, w in zip(outs, want))
+    recording.graph.destroy()
+    with hip.batching():
+        outs = fn()
+    assert all(np.array_equal(bits(t), w) for t, w in zip(outs, want))
+
+
 def test_a_recording_returns_the_bits_of_the_call(hip_backend):
     rng = np.random.default_rng(7)
     with hip_backend.use():
         x = Tensor(data=rng.standard_normal((48, 4100)).astype(np.float32), dtype=DType.float16)
         w = Tensor(data=(rng.standard_normal((4100, 300)) / 64).astype(np.float32), dtype=DType.float16)
         bias = Tensor(data=rng.standard_normal(300).astype(np.float32), dtype=DType.float16)
-        f = lambda: (Tensor.matmul(x, False, w, False, False) + bias).gelu()
-        want = f().numpy()
-        with hip_backend.capture() as recording:
-            out = f()
-        for _ in range(3):
-            recording.graph.launch()
-            np.testing.assert_array_equal(out.numpy().view(np.uint16), want.view(np.uint16))
-        with hip_backend.batching():
-            got = f()
-        np.testing.assert_array_equal(got.numpy().view(np.uint16), want.view(np.uint16))
+        same_bits(hip_backend, lambda: [(Tensor.matmul(x, False, w, False, False) + bias).gelu()])
+
+
+# (whole and ragged tiles, a last part shorter than the others)
+@pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
+@pytest.mark.parametrize("m,k,n", [(64, 3072, 768), (16, 4096, 1024), (13, 3208, 824)], ids=str)
+def test_what_follows_is_merged_into_the_sum(hip_backend, capfd, dtype, m, k, n):
+    rng = np.random.default_rng(m)
+    tensor = lambda *shape, to=dtype: Tensor(data=rng.standard_normal(shape).astype(np.float32), dtype=to)
+    with hip_backend.use():
+        x, w, row, row2, rest = tensor(m, k), tensor(k, n), tensor(n), tensor(n), tensor(m, n)
+        row32 = tensor(n, to=DType.float32)
+        product = lambda: Tensor.matmul(x, False, w, False, False)
+        for fn in (lambda: product() + row, lambda: (row + product()).gelu(), lambda: (product() + row) + rest, lambda: rest + product(),
+                   lambda: ((product() + row) + rest) + row2, lambda: ((product() + row) + row2).gelu(), lambda: product().gelu(),
+                   lambda: product() + row32.cast(dtype)):
+            names = kernels_of(hip_backend, capfd, fn)
+            assert len(names) == 2 and "_part_64x64_kn" in names[0] and names[1] == "hc_gemm_part_sum_%s_m" % names[0].split("_")[2], names
+            same_bits(hip_backend, lambda: [fn()])
+        # a result that the caller keeps is stored
+        kept = []
+        names = kernels_of(hip_backend, capfd, lambda: (kept.append(product()), kept[-1] + row))
+        assert names[1] == "hc_gemm_part_sum_%s" % names[0].split("_")[2] and len(names) == 3
+        del kept[:]
 
 
 @pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
