@@ -39,6 +39,8 @@ KERNELS = [
     ("gemm_dma_m", "gemm_dma.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1"]),
     ("gemm_dma2_m_f16", "gemm_dma2.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1", "-DHC_GEMM_ONLY=16"]),
     ("gemm_dma2_m_f32", "gemm_dma2.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1", "-DHC_GEMM_ONLY=32"]),
+    # ... and the kernels of it that take the parts of the third build one after the other
+    ("gemm_chains", "gemm_dma2.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1", "-DHC_GEMM_CHAINS=1"]),
     ("gemm_mi16_m", "gemm_mi16.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1"]),
     ("gemm_ks_m", "gemm_ks.hip", ["-ffp-contract=off", "-DHC_GEMM_MERGED=1"]),
 ]
@@ -63,7 +65,7 @@ def _run(cmd):
 # sit at the 256-VGPR limit; the edge kernels' write-out needs a few registers more): up to 96 bytes
 # per lane in the plain kernels, up to 128 in the kernels with merged epilogues.
 NO_SCRATCH = {"gemm_dma": 96, "gemm_dma2": 96, "gemm_mi16": 96, "gemm_f16_fast": 16,
-              "gemm_ks": 0, "gemm_ks_m": 0, "gemm_parts": 0,
+              "gemm_ks": 0, "gemm_ks_m": 0, "gemm_parts": 0, "gemm_chains": 0,
               "gemm_dma_m": 128, "gemm_dma2_m_f16": 128, "gemm_dma2_m_f32": 128, "gemm_mi16_m": 128}
 
 

@@ -24,6 +24,7 @@
     EMBED hc_image_gemm_dma2, "gemm_dma2.hsaco"
     EMBED hc_image_gemm_mi16, "gemm_mi16.hsaco"
     EMBED hc_image_gemm_parts, "gemm_parts.hsaco"
+    EMBED hc_image_gemm_chains, "gemm_chains.hsaco"
     EMBED hc_image_gemm_ks, "gemm_ks.hsaco"
     EMBED hc_image_gemm_dma_m, "gemm_dma_m.hsaco"
     EMBED hc_image_gemm_dma2_m_f16, "gemm_dma2_m_f16.hsaco"

@@ -36,6 +36,7 @@ extern const unsigned char hc_image_gemm_dma[], hc_image_gemm_dma_end[];
 extern const unsigned char hc_image_gemm_dma2[], hc_image_gemm_dma2_end[];
 extern const unsigned char hc_image_gemm_mi16[], hc_image_gemm_mi16_end[];
 extern const unsigned char hc_image_gemm_parts[], hc_image_gemm_parts_end[];
+extern const unsigned char hc_image_gemm_chains[], hc_image_gemm_chains_end[];
 extern const unsigned char hc_image_gemm_ks[], hc_image_gemm_ks_end[];
 extern const unsigned char hc_image_gemm_dma_m[], hc_image_gemm_dma_m_end[];
 extern const unsigned char hc_image_gemm_dma2_m_f16[], hc_image_gemm_dma2_m_f16_end[];
@@ -106,6 +107,7 @@ struct hc_pending {
   int op = 0;
   int lanes = 0;
   void* out = nullptr;
+  const void* sums = nullptr;          // the partial sums that the two launches of a product in parts of K share
   bool dropped = false;                // merged into another entry
   bool merged = false;                 // the rewrite's own launch: stands where the last entry of its chain stood
 };
@@ -335,6 +337,7 @@ extern "C" int hc_init(int device, hc_ctx** out) {
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma2, hc_image_gemm_dma2_end, "gemm_dma2");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_mi16, hc_image_gemm_mi16_end, "gemm_mi16");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_parts, hc_image_gemm_parts_end, "gemm_parts");
+  if (s == HC_OK) s = load_image(ctx, hc_image_gemm_chains, hc_image_gemm_chains_end, "gemm_chains");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_ks, hc_image_gemm_ks_end, "gemm_ks");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma_m, hc_image_gemm_dma_m_end, "gemm_dma_m");
   if (s == HC_OK) s = load_image(ctx, hc_image_gemm_dma2_m_f16, hc_image_gemm_dma2_m_f16_end, "gemm_dma2_m_f16");
@@ -1140,6 +1143,7 @@ struct OpNote {
   std::vector<const void*> reads, writes;
   hc_pending::Tag tag = hc_pending::NONE;
   hc_pending meta;    // tag fields for the next launch only (consumed by it)
+  const void* sums = nullptr;   // (hc_pending::sums, of every launch)
   OpNote* outer;
   static thread_local OpNote* current;
   OpNote(std::initializer_list<const void*> r, std::initializer_list<const void*> w) : reads(r), writes(w), outer(current) {
@@ -1178,6 +1182,7 @@ static void record_launch_locked(hc_ctx* ctx, const std::string& name, hipFuncti
     e.known = true;
     e.reads = n->reads;
     e.writes = n->writes;
+    e.sums = n->sums;
     if (n->tag != hc_pending::NONE) {   // the tag describes exactly one launch: the next one
       e.tag = n->tag;
       e.dtype = n->meta.dtype;

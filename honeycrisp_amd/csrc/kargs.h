@@ -403,10 +403,10 @@ typedef struct {
 } hck_gemm_args;
 
 /* A product in parts of K: part i (blockIdx.y) covers k = i * kchunk .. (kchunk a multiple of 64; a_bs, b_bs: what lies between
- * two parts' first elements), c: fp32 partial sums [parts][M][N], N a multiple of 4. */
+ * two parts' first elements), c: fp32 partial sums [parts][M][N], N a multiple of 4. A group of products: blockIdx.y = member * parts + i. */
 typedef struct {
   hck_gemm_args g;
-  uint32_t kchunk;
+  uint32_t kchunk, parts;
 } hck_gemm_part_args;
 /* ... and their sum: the whole product's g.c[row * g.c_rs + col], col < g.N, from sums [parts][g.M][ld]; kernels ending in _m then
  * apply g.ep_*. (g first: what merges operations into a product finds it in the same place as in a launch of one.) */
@@ -414,6 +414,7 @@ typedef struct {
   hck_gemm_args g;
   const void* sums;
   uint32_t ld, parts;
+  const void* g_sums[4];   /* a group of products: blockIdx.y picks the member's sums, g.g_c and g.g_ep */
 } hck_gemm_part_sum_args;
 
 /* Two matrices of 2-byte elements copied to rows of whole cache lines: out[r * ld + c] = in[r * cols + c], zeros from cols on;

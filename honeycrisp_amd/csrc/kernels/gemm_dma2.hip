@@ -234,11 +234,12 @@ template <typename T, int ROWS, int MODE> struct DmaOperand {
 // (waits, barrier, scalar bookkeeping: the four-stage pipeline of 64-byte slices spends about 275
 // cycles per slice on a 64 x 64 tile, of which the MFMAs are 128), so the slices should be long,
 // and with one workgroup per compute unit only a deep ring keeps enough loads in flight.
-// kchunk (the third build, see the kernels at the end): the workgroup multiplies the kchunk values of K from blockIdx.y * kchunk on and
-// stores TO = float; 0: all of K.
-template <typename T, int BM, int BN, int MODE_A, int MODE_B, bool EDGE, bool ONE = false, bool RING4 = false, typename TO = T>
+// kchunk (the third build, see the kernels at the end): the workgroup multiplies the kchunk values of K from i * kchunk on, i = blockIdx.y or, of a
+// group, blockIdx.y % parts, and stores TO = float; 0: all of K. CHAIN: the workgroup takes one part after the other and adds them up like the launch
+// that follows the parts, in the same order: the same bits.
+template <typename T, int BM, int BN, int MODE_A, int MODE_B, bool EDGE, bool ONE = false, bool RING4 = false, typename TO = T, bool GROUP = false, bool CHAIN = false>
 __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds0, char* lds1, char* lds2 = nullptr,
-                                               char* lds3 = nullptr, const uint32_t kchunk = 0) {
+                                               char* lds3 = nullptr, const uint32_t kchunk = 0, const uint32_t parts = 1) {
   static_assert(!(ONE && RING4), "one slice needs no ring");
   constexpr int MT = BM / 64, NT = BN / 64;
   constexpr int SLOTS = MT * NT;
@@ -275,12 +276,19 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
   const void* const ep_p0 = gemm_epilogue_operand(p, 0, batch);
   const void* const ep_p1 = gemm_epilogue_operand(p, 1, batch);
   const void* const ep_p2 = gemm_epilogue_operand(p, 2, batch);
+  const uint32_t K = p.K;
+#elif defined(HC_GEMM_PARTS)
+  const uint32_t member = GROUP ? batch / parts : 0, part = batch - member * parts;
+  const T* A = (const T*)p.a + part * p.a_bs;
+  const T* B = (const T*)(GROUP ? gemm_table_entry(p.g_b, member) : p.b) + part * p.b_bs;
+  TO* C = (TO*)(GROUP ? gemm_table_entry(p.g_c, member) : p.c) + part * p.c_bs;
+  const uint32_t K = min(p.K - part * kchunk, kchunk);
 #else
   const T* A = (const T*)p.a + batch * p.a_bs;
   const T* B = (const T*)p.b + batch * p.b_bs;
   TO* C = (TO*)p.c + batch * p.c_bs;
+  const uint32_t K = p.K;
 #endif
-  const uint32_t K = kchunk == 0 ? p.K : min(p.K - batch * kchunk, kchunk);
 
   const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const uint32_t wm = (wave >> 1) * (BM / 2), wn = (wave & 1) * (BN / 2);
@@ -379,6 +387,23 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
     }
   };
 
+  floatx16 sum[MT][NT];   // (CHAIN) the parts so far
+  uint32_t steps_left = kchunk / BK;
+  bool first_part = true;
+  auto end_part = [&] {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int jj = 0; jj < NT; jj++)
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+          sum[i][jj][v] = first_part ? acc[i][jj][v] : sum[i][jj][v] + acc[i][jj][v];
+          acc[i][jj][v] = 0.0f;
+        }
+    first_part = false;
+    steps_left = kchunk / BK;
+  };
+
   // K-step j out of `cur`; `nxt` receives the rest of K-step j+1, then `cur` the start of j+2
   auto step = [&](auto tail, char* cur, char* nxt, uint32_t j) {
     __builtin_amdgcn_sched_barrier(0);
@@ -392,6 +417,9 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
     lds_barrier();  // ... and everybody's; nobody reads cur any more
     __builtin_amdgcn_sched_barrier(0);
     substep(tail, f1, f0, nxt, 0, 0, cur, kclamp(j + 2));
+    if constexpr (CHAIN) {
+      if (--steps_left == 0 || j + 1 == nk) end_part();
+    }
   };
 
   // Ring of four: K-step j out of `cur`; `nxt` holds K-step j+1 once the wait passes; the stage
@@ -412,6 +440,9 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
     lds_barrier();  // ... and everybody's; nobody reads cur any more
     __builtin_amdgcn_sched_barrier(0);
     substep(tail, f1, f0, nxt, 0, -1, nullptr, 0);
+    if constexpr (CHAIN) {
+      if (--steps_left == 0 || j + 1 == nk) end_part();
+    }
   };
 
   if constexpr (RING4) {
@@ -487,6 +518,12 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
       step(Tail{}, lds1, lds0, j + 1);
     }
     if (j < nk) step(Tail{}, lds0, lds1, j);
+  }
+  if constexpr (CHAIN) {
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+#pragma unroll
+      for (int jj = 0; jj < NT; jj++) acc[i][jj] = sum[i][jj];
   }
   wait_dma<0>();  // no LDS write of this workgroup may be in flight when it ends
 
@@ -647,13 +684,20 @@ __device__ __forceinline__ void gemm_dma2_impl(const hck_gemm_args& p, char* lds
 // Products of few tiles over a long K: as many workgroups as compute units, each a tile over a part of K (blockIdx.y) into fp32 partial
 // sums, which a second launch adds up, parts in order. 64 x 64 tiles fetch whole cache lines, so that a part of K takes little
 // longer than its bytes need.
-#define DEF_PART(T, TN, AN, AM, BNAME, BMODE, E, SUFFIX)                                               \
+// Groups (_g) in kernels of their own: what tells a member from its part costs 0.35 us where it is not wanted, and two stages leave room for
+// the workgroups of all members side by side.
+#define DEF_PART(T, TN, AN, AM, BNAME, BMODE, E, SUFFIX)                                              \
   extern "C" __global__ __launch_bounds__(256) void hc_gemm_##TN##_part_64x64_##AN##BNAME##SUFFIX(hck_gemm_part_args p) { \
     __shared__ __attribute__((aligned(1024))) char lds0[128 * 128];                                   \
     __shared__ __attribute__((aligned(1024))) char lds1[128 * 128];                                   \
     __shared__ __attribute__((aligned(1024))) char lds2[128 * 128];                                   \
     __shared__ __attribute__((aligned(1024))) char lds3[128 * 128];                                   \
-    gemm_dma2_impl<T, 64, 64, AM, BMODE, E, false, true, float>(p.g, lds0, lds1, lds2, lds3, p.kchunk); \
+    gemm_dma2_impl<T, 64, 64, AM, BMODE, E, false, true, float>(p.g, lds0, lds1, lds2, lds3, p.kchunk, p.parts); \
+  }                                                                                                   \
+  extern "C" __global__ __launch_bounds__(256) void hc_gemm_##TN##_part_64x64_##AN##BNAME##SUFFIX##_g(hck_gemm_part_args p) { \
+    __shared__ __attribute__((aligned(1024))) char lds0[128 * 128];                                   \
+    __shared__ __attribute__((aligned(1024))) char lds1[128 * 128];                                   \
+    gemm_dma2_impl<T, 64, 64, AM, BMODE, E, false, false, float, true>(p.g, lds0, lds1, nullptr, nullptr, p.kchunk, p.parts); \
   }
 #define DEF_PART_LAYOUT(T, TN, AN, AM, BNAME, BMODE) \
   DEF_PART(T, TN, AN, AM, BNAME, BMODE, false, )     \
@@ -667,9 +711,9 @@ DEF_PARTS(half_t, f16)
 DEF_PARTS(float, f32)
 
 // A lane adds up four neighbouring outputs (a row of partial sums is a whole number of those), loads of four parts at a time on their way.
-template <typename T> __device__ __forceinline__ void gemm_part_sum(const hck_gemm_part_sum_args& p, uint32_t q, T (&y)[4]) {
+template <typename T> __device__ __forceinline__ void gemm_part_sum(const hck_gemm_part_sum_args& p, const void* sums, uint32_t q, T (&y)[4]) {
   const size_t part = (size_t)p.g.M * (p.ld / 4);
-  const floatx4* src = (const floatx4*)p.sums + q;
+  const floatx4* src = (const floatx4*)sums + q;
   floatx4 s = src[0];
   uint32_t i = 1;
   for (; i + 4 <= p.parts; i += 4) {
@@ -688,7 +732,7 @@ template <typename T> __device__ __forceinline__ void gemm_part_sum_impl(const h
   if (q >= p.g.M * per_row) return;
   const uint32_t row = q / per_row, col = (q - row * per_row) * 4;
   T y[4];
-  gemm_part_sum<T>(p, q, y);
+  gemm_part_sum<T>(p, p.sums, q, y);
   T* dst = (T*)p.g.c + (size_t)row * p.g.c_rs + col;
   if (col + 4 <= p.g.N) {
     store_vec_loose<T, 4>(dst, y);
@@ -701,7 +745,7 @@ template <typename T> __device__ __forceinline__ void gemm_part_sum_impl(const h
 extern "C" __global__ __launch_bounds__(HCK_BLOCK) void hc_gemm_part_sum_f16(hck_gemm_part_sum_args p) { gemm_part_sum_impl<half_t>(p); }
 extern "C" __global__ __launch_bounds__(HCK_BLOCK) void hc_gemm_part_sum_f32(hck_gemm_part_sum_args p) { gemm_part_sum_impl<float>(p); }
 
-// The same with what a recording merged into the product (only with rows of C of whole 16-byte pieces): one of three bodies per
+// The same with what a recording merged into the product, and for a group of products (only with rows of C of whole 16-byte pieces): one of three bodies per
 // launch like the tiled kernels' write-out, the operands' loads in front of those of the partial sums. Product, bias and residual, fp16, us,
 // one launch without parts / parts with the operations launched apart / this: 16 x 3072 x 768 11.5 / 12.7 / 8.9, 512 x 4096 x 1024
 // 18.6 / 22.1 / 17.6.
@@ -710,16 +754,19 @@ template <typename T, bool MATRIX, bool GELU> __device__ __forceinline__ void ge
   const uint32_t per_row = p.ld / 4, q = blockIdx.x * HCK_BLOCK + threadIdx.x;
   if (q >= p.g.M * per_row) return;
   const uint32_t row = q / per_row, col = (q - row * per_row) * 4;
-  const void *p0 = gemm_epilogue_operand(p.g, 0, 0), *p1 = gemm_epilogue_operand(p.g, 1, 0), *p2 = gemm_epilogue_operand(p.g, 2, 0);
+  const uint32_t member = blockIdx.y;
+  const bool grouped = p.g.group != 0;
+  const void *p0 = gemm_epilogue_operand(p.g, 0, member), *p1 = gemm_epilogue_operand(p.g, 1, member), *p2 = gemm_epilogue_operand(p.g, 2, member);
+  T* c = (T*)(grouped ? gemm_table_entry(p.g.g_c, member) : p.g.c);
   const Piece r0 = gemm_epilogue_row_piece<T, Piece>(p.g.ep_kind[0], p0, col, true), r1 = gemm_epilogue_row_piece<T, Piece>(p.g.ep_kind[1], p1, col, true),
               r2 = gemm_epilogue_row_piece<T, Piece>(p.g.ep_kind[2], p2, col, true);
   Piece m = Piece{};
   if (MATRIX) m = gemm_epilogue_matrix_piece<T, Piece>(p.g, p0, p1, p2, row, col);
   T y[4];
-  gemm_part_sum<T>(p, q, y);
+  gemm_part_sum<T>(p, grouped ? gemm_table_entry(p.g_sums, member) : p.sums, q, y);
   Piece v;
   __builtin_memcpy(&v, y, sizeof(v));
-  *reinterpret_cast<Piece*>((T*)p.g.c + (size_t)row * p.g.c_rs + col) = gemm_epilogue_apply<T, Piece, MATRIX, GELU>(p.g, v, r0, r1, r2, m);
+  *reinterpret_cast<Piece*>(c + (size_t)row * p.g.c_rs + col) = gemm_epilogue_apply<T, Piece, MATRIX, GELU>(p.g, v, r0, r1, r2, m);
 }
 template <typename T> __device__ __forceinline__ void gemm_part_sum_merged(const hck_gemm_part_sum_args& p) {
   const uint32_t k0 = p.g.ep_kind[0], k1 = p.g.ep_kind[1], k2 = p.g.ep_kind[2];
@@ -729,6 +776,24 @@ template <typename T> __device__ __forceinline__ void gemm_part_sum_merged(const
 }
 extern "C" __global__ __launch_bounds__(HCK_BLOCK) void hc_gemm_part_sum_f16_m(hck_gemm_part_sum_args p) { gemm_part_sum_merged<half_t>(p); }
 extern "C" __global__ __launch_bounds__(HCK_BLOCK) void hc_gemm_part_sum_f32_m(hck_gemm_part_sum_args p) { gemm_part_sum_merged<float>(p); }
+#elif defined(HC_GEMM_CHAINS)
+// Groups of fp16 products in parts of K whose tiles keep most of the device busy by themselves (the host's rule and figures: fuse_product_groups). Built with
+// what the second build has: the write-out takes what a recording merged.
+#define DEF_CHAIN(AN, AM, BNAME, BMODE, E, SUFFIX)                                                    \
+  extern "C" __global__ __launch_bounds__(256) void hc_gemm_f16_chain_64x64_##AN##BNAME##SUFFIX##_m(hck_gemm_part_args p) { \
+    __shared__ __attribute__((aligned(1024))) char lds0[128 * 128];                                   \
+    __shared__ __attribute__((aligned(1024))) char lds1[128 * 128];                                   \
+    __shared__ __attribute__((aligned(1024))) char lds2[128 * 128];                                   \
+    __shared__ __attribute__((aligned(1024))) char lds3[128 * 128];                                   \
+    gemm_dma2_impl<half_t, 64, 64, AM, BMODE, E, false, true, half_t, false, true>(p.g, lds0, lds1, lds2, lds3, p.kchunk); \
+  }
+#define DEF_CHAIN_LAYOUT(AN, AM, BNAME, BMODE) \
+  DEF_CHAIN(AN, AM, BNAME, BMODE, false, )     \
+  DEF_CHAIN(AN, AM, BNAME, BMODE, true, _e)
+DEF_CHAIN_LAYOUT(k, DMA_K, k, DMA_K)
+DEF_CHAIN_LAYOUT(k, DMA_K, n, DMA_MN)
+DEF_CHAIN_LAYOUT(m, DMA_MN, k, DMA_K)
+DEF_CHAIN_LAYOUT(m, DMA_MN, n, DMA_MN)
 #else
 #define DEF_DMA_RING4_TILE(T, TN, BM, BN)                                                             \
   DEF_DMA_RING4(T, TN, BM, BN, k, DMA_K, k, DMA_K)                                                    \
@@ -777,4 +842,4 @@ DEF_DMA_TILE(float, f32, 256, 192)
 DEF_DMA_TILE(float, f32, 192, 256)
 DEF_DMA_TILE(float, f32, 192, 192)
 #endif
-#endif   // HC_GEMM_PARTS
+#endif   // HC_GEMM_PARTS, HC_GEMM_CHAINS

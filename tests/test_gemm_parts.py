@@ -82,6 +82,53 @@ def test_what_follows_is_merged_into_the_sum(hip_backend, capfd, dtype, m, k, n)
         del kept[:]
 
 
+# (groups of two to four, and one more than a launch takes; at most as many parts of one tile, and few parts of many; fp16 above and at 128 tiles)
+@pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
+@pytest.mark.parametrize("m,k,n,count", [(64, 3072, 768, 3), (16, 4096, 1024, 2), (13, 3208, 824, 5), (64, 4160, 64, 4), (300, 3072, 768, 3), (300, 3080, 840, 2), (64, 3072, 4096, 2),
+                                       (512, 5064, 1024, 4)], ids=str)
+def test_products_over_one_input_share_their_launches(hip_backend, capfd, dtype, m, k, n, count):
+    rng = np.random.default_rng(m)
+    tensor = lambda *shape: Tensor(data=rng.standard_normal(shape).astype(np.float32), dtype=dtype)
+    with hip_backend.use():
+        x, ws, rows = tensor(m, k), [tensor(k, n) for _ in range(count)], [tensor(n) for _ in range(count)]
+        if "hc_gemm_part_sum_%s" % {DType.float16: "f16", DType.float32: "f32"}[dtype] not in kernels_of(
+                hip_backend, capfd, lambda: Tensor.matmul(x, False, ws[0], False, False)):
+            assert dtype == DType.float32 and m * n > 200000      # (longer chains than those of a workgroup's waves)
+            return
+        chain = dtype == DType.float16 and 2 * count * -(-m // 64) * -(-n // 64) > 256
+        for fn in (lambda: [Tensor.matmul(x, False, w, False, False) for w in ws],
+                   lambda: [Tensor.matmul(x, False, w, False, False) + row for w, row in zip(ws, rows)]):
+            names = kernels_of(hip_backend, capfd, fn)
+            assert len(names) == (1 if chain else 2 if count <= 4 else 4) and ("_chain_" in names[0]) == chain, names
+            same_bits(hip_backend, fn)
+
+        def used_between():
+            first = Tensor.matmul(x, False, ws[0], False, False)
+            return [first.exp(), Tensor.matmul(x, False, ws[1], False, False), first]
+
+        assert len(kernels_of(hip_backend, capfd, used_between)) == 5
+        same_bits(hip_backend, used_between)
+
+
+@pytest.mark.parametrize("m,k,n", [(64, 3072, 768), (300, 3072, 768)], ids=str)
+@pytest.mark.parametrize("which", [0, 1])
+def test_an_operand_may_change_behind_its_product(hip_backend, m, k, n, which):
+    """The parts are moved next to those of the other member, or next to their sum, only as far as what they read stays as it was."""
+    rng = np.random.default_rng(m)
+    tensor = lambda *shape: Tensor(data=rng.standard_normal(shape).astype(np.float32), dtype=DType.float16)
+    with hip_backend.use():
+        x, ws, row = tensor(m, k), [tensor(k, n) for _ in range(2)], tensor(n)
+        fill = lambda w, v: hip_backend._check(hip_backend._lib.hc_fill(hip_backend._ctx, DType.float16, v, 0, w.data.ptr, k * n))
+
+        def program():
+            fill(ws[0], 0.25), fill(ws[1], 0.5)
+            products = [Tensor.matmul(x, False, w, False, False) for w in ws]
+            fill(ws[which], 2.0)
+            return [y + row for y in products]
+
+        same_bits(hip_backend, program)
+
+
 @pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
 def test_an_infinity_or_a_nan_stays_in_its_row_and_column(hip_backend, dtype):
     m, k, n = 70, 3100, 66
