@@ -129,6 +129,23 @@ def test_an_operand_may_change_behind_its_product(hip_backend, m, k, n, which):
         same_bits(hip_backend, program)
 
 
+@pytest.mark.parametrize("m,k,n", [(64, 3072, 768), (300, 3072, 768)], ids=str)
+def test_sums_in_another_order_than_their_parts(hip_backend, capfd, m, k, n):
+    """The second product's bias comes last, and what the third multiplies with is made between the two."""
+    rng = np.random.default_rng(m)
+    tensor = lambda *shape: Tensor(data=rng.standard_normal(shape).astype(np.float32), dtype=DType.float16)
+    with hip_backend.use():
+        x, ws, row = tensor(m, k), [tensor(k, n) for _ in range(3)], tensor(n)
+
+        def program():
+            a, b = (Tensor.matmul(x, False, w, False, False) for w in ws[:2])
+            c = Tensor.matmul(x, False, ws[2] * ws[0], False, False)
+            return [t + row for t in (a, c, b)]
+
+        assert len(kernels_of(hip_backend, capfd, program)) == (2 if m == 300 else 3)
+        same_bits(hip_backend, program)
+
+
 @pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
 def test_an_infinity_or_a_nan_stays_in_its_row_and_column(hip_backend, dtype):
     m, k, n = 70, 3100, 66
