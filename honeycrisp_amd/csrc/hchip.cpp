@@ -14,6 +14,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <cmath>
+#include <deque>
 #include <map>
 #include <unordered_set>
 #include <mutex>
@@ -116,6 +117,8 @@ struct hc_graph {
   hipGraph_t graph = nullptr;
   hipGraphExec_t exec = nullptr;
   std::unordered_map<size_t, std::vector<void*>> parked;
+  // while it is recorded, and its list will be rewritten: blocks that calls had for launches of their own only, by bucket size, oldest first (Scratch::own)
+  std::unordered_map<size_t, std::deque<void*>> spare;
   // HCHIP_GRAPH_AS_LAUNCHES=1 at hc_capture_end: the rewritten list, replayed launch by launch
   // instead of through hipGraphLaunch (for kernel traces: the tracer of this ROCm release aborts
   // inside hipGraphLaunch)
@@ -994,6 +997,13 @@ static int end_capture(hc_ctx* ctx, hc_graph** out) {
 static int end_capture_locked(hc_ctx* ctx, hc_graph** out) {
   hc_graph* g = ctx->capturing;
   int emitted = HC_OK;
+  for (auto& kv : g->spare)   // (from here on the recording's blocks like all others)
+    for (void* p : kv.second) {
+      ctx->live.erase(p);
+      ctx->bytes_in_use -= kv.first;
+      g->parked[kv.first].push_back(p);
+    }
+  g->spare.clear();
   if (ctx->lazy) {
     ctx->lazy = false;
     if (out) {
@@ -1841,13 +1851,14 @@ extern "C" int hc_fill(hc_ctx* ctx, int dtype, float vf, int64_t vi, void* out, 
 // from that range instead, 256-byte aligned, and nothing is allocated or freed.
 struct Scratch {
   hc_ctx* ctx;
-  std::vector<void*> ptrs;
+  std::vector<void*> ptrs, owned;
   char* arena = nullptr;
   size_t arena_bytes = 0, arena_used = 0;
   explicit Scratch(hc_ctx* c) : ctx(c) {}
   Scratch(hc_ctx* c, void* base, size_t bytes) : ctx(c), arena((char*)base), arena_bytes(bytes) {}
   ~Scratch() {
     for (void* p : ptrs) (void)hc_free(ctx, p);
+    for (void* p : owned) give_back(p);
   }
   bool fixed() const { return arena != nullptr; }
   int get(size_t bytes, void** out) {
@@ -1864,6 +1875,35 @@ struct Scratch {
     int s = hc_malloc(ctx, bytes, out);
     if (s == HC_OK) ptrs.push_back(*out);
     return s;
+  }
+  // A block that only launches of this call touch, none of which declares it. A recording whose list will be rewritten hands no other block out twice and
+  // would keep one per call; of these it takes an earlier call's again, once more than `behind` of them have been given back. Its rewrite keeps the
+  // order of launches that share one (hc_pending::sums; launches without it are not moved).
+  int own(size_t bytes, size_t behind, void** out) {
+    int s = HC_OK;
+    std::unique_lock<std::mutex> lock(ctx->mu);
+    std::deque<void*>* spare = ctx->capturing && ctx->rewrite ? &ctx->capturing->spare[bucket_size(bytes)] : nullptr;
+    if (spare && spare->size() > behind) {
+      *out = spare->front();
+      spare->pop_front();
+    } else {
+      lock.unlock();
+      s = hc_malloc(ctx, bytes, out);
+    }
+    if (s == HC_OK) owned.push_back(*out);
+    return s;
+  }
+  void give_back(void* p) {
+    {
+      std::lock_guard<std::mutex> lock(ctx->mu);
+      auto block = ctx->live.find(p);
+      auto owner = ctx->block_owner.find(p);
+      if (ctx->rewrite && block != ctx->live.end() && owner != ctx->block_owner.end() && owner->second == ctx->capturing) {
+        ctx->capturing->spare[block->second].push_back(p);
+        return;
+      }
+    }
+    (void)hc_free(ctx, p);
   }
 };
 

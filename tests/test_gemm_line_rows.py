@@ -45,3 +45,24 @@ def test_what_follows_a_row_is_not_multiplied(hip_backend):
     want = np.full((m, n), 8000.0, np.float16)     # (8001 rounds to 8000 in fp16)
     want[5], want[9], want[:, 7] = np.inf, -np.inf, np.nan
     np.testing.assert_array_equal(got, want)
+
+
+def test_a_recording_shares_the_copies(hip_backend):
+    """Six products whose operands are copied to rows of whole lines, 14 MiB each: one pair of copies in a recording, and the bits of the calls."""
+    m, k, n, count = 900, 8001, 900, 6
+    a, b = operands(m, k, n)
+    with hip_backend.use():
+        xs, y = [Tensor(data=np.roll(a, i, axis=0)) for i in range(count)], Tensor(data=b)
+        program = lambda: [Tensor.matmul(x, False, y, True, False) for x in xs]
+        want = [t.numpy() for t in program()]
+        hip_backend.sync()
+        assert hip_backend._lib.hc_trim(hip_backend._ctx) == 0
+        with hip_backend.capture() as recording:
+            outs = program()
+        for _ in range(2):
+            recording.graph.launch()
+            assert all(np.array_equal(t.numpy(), v) for t, v in zip(outs, want))
+        del outs
+        recording.graph.destroy()
+        held = hip_backend.memStats()[1]
+        assert held <= 2 * (14 << 20) + count * (2 << 20), held

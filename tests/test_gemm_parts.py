@@ -146,6 +146,29 @@ def test_sums_in_another_order_than_their_parts(hip_backend, capfd, m, k, n):
         same_bits(hip_backend, program)
 
 
+def test_a_recording_shares_the_blocks_of_partial_sums(hip_backend):
+    """Forty products whose sums take 768 KiB each in a recording, what follows them merged in all orders: at most nine blocks, and the bits of the calls."""
+    m, k, n, count = 64, 3072, 256, 40
+    rng = np.random.default_rng(3)
+    tensor = lambda *shape: Tensor(data=rng.standard_normal(shape).astype(np.float32), dtype=DType.float16)
+    with hip_backend.use():
+        xs, w, row = [tensor(m, k) for _ in range(count)], tensor(k, n), tensor(n)
+
+        def program():
+            late = [Tensor.matmul(x, False, w, False, False) for x in xs[:20]]     # (their bias comes when the blocks have been used again)
+            return [Tensor.matmul(x, False, w, False, False) + row for x in xs[20:]] + [y + row for y in late]
+
+        same_bits(hip_backend, program)
+        hip_backend.sync()
+        assert hip_backend._lib.hc_trim(hip_backend._ctx) == 0
+        with hip_backend.capture() as recording:
+            outs = program()
+        del outs
+        recording.graph.destroy()
+        held = hip_backend.memStats()[1]      # what the recording had: the sums, and 32 KiB for every product and every addition
+        assert held <= 9 * (1 << 20) + 2 * count * (32 << 10), held
+
+
 @pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
 def test_an_infinity_or_a_nan_stays_in_its_row_and_column(hip_backend, dtype):
     m, k, n = 70, 3100, 66
