@@ -289,8 +289,10 @@ static PyObject* end(Call* call, PyObject* result) {
     if (!result) {                                                                     \
       PyObject *type, *value, *traceback;                                              \
       PyErr_Fetch(&type, &value, &traceback);                                          \
+      Py_BEGIN_ALLOW_THREADS                                                           \
       for (int i = 0; i < n; i++)                                                      \
         if (out[i]) c->hc_free(ctx, out[i]);                                           \
+      Py_END_ALLOW_THREADS                                                             \
       PyErr_Restore(type, value, traceback);                                           \
     }                                                                                  \
   }                                                                                    \

@@ -16,9 +16,10 @@ native = pytest.importorskip("honeycrisp_amd._native")
 TYPED = r"""
 #include <stdlib.h>
 #include "hchip.h"
-int live, calls, fail; long long seen[16]; hc_strides shape;
+int live, calls, fail, locked; long long seen[16]; hc_strides shape;
+int PyGILState_Check(void);
 int hc_malloc(hc_ctx* c, size_t n, void** p) { if (!c) return HC_ERR_INVALID; if (fail == 2 && live) return HC_ERR_ALLOC; *p = malloc(1); live++; return 0; }
-int hc_free(hc_ctx* c, void* p) { free(p); live--; return 0; }
+int hc_free(hc_ctx* c, void* p) { locked += PyGILState_Check(); free(p); live--; return 0; }
 int hc_binary_op(hc_ctx* c, int op, int t, const void* a, const hc_strides* sa, const void* b, const hc_strides* sb, void* o) {
   seen[0] = op; seen[1] = t; seen[2] = (long long)a; seen[3] = (long long)b; shape = *sa; calls++; return fail ? HC_ERR_UNSUPPORTED : 0; }
 int hc_fill(hc_ctx* c, int t, float f, int64_t i, void* o, size_t n) { seen[0] = t; seen[1] = (long long)(f * 4); seen[2] = i; seen[3] = n; calls++; return 0; }
@@ -64,7 +65,7 @@ def fake(lib):
     f = Fake()
     f._native = native.Context(lib.path, 4096, Data)
     f.Data = Data
-    for name in ("live", "calls", "fail"):
+    for name in ("live", "calls", "fail", "locked"):
         ctypes.c_int.in_dll(lib, name).value = 0
     return f
 
@@ -109,6 +110,8 @@ def test_a_refused_call_gives_its_results_back(lib, fake):
     with pytest.raises(Refused):
         fake._native.adamw(fake, 3, x, x, x, x, 1, 1, 1, 1, 1, 1, 2)
     assert value(lib, "live") == 1
+    del x
+    assert value(lib, "locked") == 0    # (the library may wait for the device, and that for a host function in Python)
 
 
 def test_what_is_no_argument_is_refused_before_the_library_sees_it(lib, fake):
