@@ -726,7 +726,7 @@ class HIPBackend(Backend):
 
     def batchedMatmul(self, matrixCount: int, a, transA: bool, b, transB: bool, transOut: bool, rows: int,
                       inner: int, cols: int, dtype: DType) -> HIPData:
-        return self._native.matmul(self, dtype, matrixCount, a, transA, b, transB, transOut, rows, inner, cols)
+        return self._native.matmul(self, dtype, matrixCount, a, int(transA), b, int(transB), int(transOut), rows, inner, cols)
 
     def triangular(self, a, batch: int, rows: int, cols: int, upper: bool, offset: int, dtype: DType):
         out = self.allocate(batch * rows * cols * dtype.byteSize)

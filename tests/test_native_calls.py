@@ -22,12 +22,14 @@ int hc_malloc(hc_ctx* c, size_t n, void** p) { if (!c) return HC_ERR_INVALID; if
 int hc_free(hc_ctx* c, void* p) { locked += PyGILState_Check(); free(p); live--; return 0; }
 int hc_binary_op(hc_ctx* c, int op, int t, const void* a, const hc_strides* sa, const void* b, const hc_strides* sb, void* o) {
   seen[0] = op; seen[1] = t; seen[2] = (long long)a; seen[3] = (long long)b; shape = *sa; calls++; return fail ? HC_ERR_UNSUPPORTED : 0; }
+int hc_matmul(hc_ctx* c, int t, int64_t n, const void* a, int ta, const void* b, int tb, int to, int64_t rows, int64_t inner, int64_t cols, void* o) {
+  seen[0] = ta; seen[1] = tb; seen[2] = to; seen[3] = rows; seen[4] = inner; seen[5] = cols; calls++; return fail ? 4 : 0; }
 int hc_fill(hc_ctx* c, int t, float f, int64_t i, void* o, size_t n) { seen[0] = t; seen[1] = (long long)(f * 4); seen[2] = i; seen[3] = n; calls++; return 0; }
 """
 # (without the header: they do not read their arguments)
 COUNTED = "extern int calls, fail;\n" + "".join("int %s() { calls++; return fail ? 4 : 0; }\n" % name for name in (
     "hc_binary_op_scalar hc_mul_add hc_add_mul hc_when hc_cast hc_pow hc_elemwise hc_reduce hc_cumulative hc_argsort hc_log_softmax "
-    "hc_log_softmax_grad hc_normalize hc_gather hc_scatter hc_adamw hc_matmul hc_broadcast").split())
+    "hc_log_softmax_grad hc_normalize hc_gather hc_scatter hc_adamw hc_broadcast").split())
 
 
 class Refused(Exception):
@@ -126,6 +128,22 @@ def test_what_is_no_argument_is_refused_before_the_library_sees_it(lib, fake):
         with pytest.raises(error):
             call()
     assert value(lib, "calls") == 0 and value(lib, "live") == 1
+
+
+@pytest.mark.filterwarnings("error")
+def test_flags_may_be_numbers_of_any_kind(lib, fake):
+    x = fake.made(8)
+    hip = backend_module.HIPBackend.__new__(backend_module.HIPBackend)
+    hip._ctx, hip._native, hip._dev = None, fake._native, lambda data: data
+    dims = backend_module.ReduceDims(2, 3, 1)
+    hip.matmul(x, np.bool_(True), x, 0.0, np.bool_(False), 2, 3, 4, DType.float16)
+    assert seen(lib, 6) == [1, 0, 0, 2, 3, 4]
+    hip.batchedMatmul(1, x, 0, x, np.True_, 1, 2, 3, 4, DType.float16)
+    assert seen(lib, 3) == [0, 1, 1]
+    with pytest.raises(TypeError):
+        hip.matmul(x, None, x, False, False, 2, 3, 4, DType.float16)
+    hip.argsort(x, dims, np.bool_(True), np.bool_(True), DType.float16)
+    hip.cumulativeSum(x, dims, np.bool_(True), 0.0, DType.float16)
 
 
 def test_other_data_goes_through_the_backend(lib, fake):
