@@ -378,7 +378,11 @@ class HIPBackend(Backend):
         if status != _lib.HC_OK:
             self._raise(status)
         self._ctx = ctx
-        self._native = _native.Context(_lib.LIB_PATH, ctx.value, HIPData)
+        try:
+            self._native = _native.Context(_lib.LIB_PATH, ctx.value, HIPData)
+        except BaseException:
+            self.close()
+            raise
         # hc_set_batching's current values (HCHIP_BATCHING in the environment gives a context its first)
         env = (os.environ.get("HCHIP_BATCHING") or "0").split(",")
         self._batching = (int(env[0]), int(env[1]) if len(env) > 1 else 0)
@@ -386,7 +390,8 @@ class HIPBackend(Backend):
     def close(self):
         if self._ctx:
             self._perm_cache.clear()
-            self._native.close()
+            if self._native is not None:
+                self._native.close()
             self._lib.hc_shutdown(self._ctx)
             self._ctx = None
 

@@ -178,3 +178,21 @@ def test_the_backend_says_what_is_missing(monkeypatch):
     monkeypatch.setattr(backend_module, "_native", None)
     with pytest.raises(ImportError, match="_native"):
         backend_module.HIPBackend()
+
+
+def test_a_library_without_the_calls_leaves_no_context_behind(monkeypatch):
+    class Library:
+        shut = []
+
+        def hc_init(self, device, out):
+            out._obj.value = 4096
+            return 0
+
+        def hc_shutdown(self, ctx):
+            self.shut.append(ctx.value)
+
+    monkeypatch.setattr(backend_module._lib, "load", Library)
+    monkeypatch.setattr(backend_module._lib, "LIB_PATH", "libc.so.6")
+    with pytest.raises(ImportError, match="hc_malloc"):
+        backend_module.HIPBackend()
+    assert Library.shut == [4096]
