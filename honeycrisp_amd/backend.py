@@ -371,7 +371,7 @@ class HIPBackend(Backend):
         self._capturing = False
         self._perm_cache, self._perm_cache_bytes = {}, 0
         if _native is None:
-            raise ImportError("honeycrisp_amd/_native.so is missing: build it with `python -m honeycrisp_amd.csrc.build`")
+            raise ImportError("honeycrisp_amd._native is not built for this Python: build it with `python -m honeycrisp_amd.csrc.build`")
         self._lib = _lib.load()
         ctx = c_void_p()
         status = self._lib.hc_init(device, byref(ctx))

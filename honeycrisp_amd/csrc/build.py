@@ -1,7 +1,7 @@
 """Build libhchip.so: gfx950 code objects via `hipcc --genco`, embedded into the host library.
 
 Usage: python -m honeycrisp_amd.csrc.build   (or build_all() from Python)
-Outputs, all in this directory: build/*.hsaco (intermediate) and libhchip.so.
+Outputs: build/*.hsaco (intermediate) and libhchip.so in this directory, ../_native.*.so and ../cpp/HCMatrixBench.
 """
 import os
 import re
@@ -183,11 +183,6 @@ def build_all(verbose=True):
     ])
     if verbose:
         print("built", os.path.relpath(LIB_PATH, HERE), os.path.getsize(LIB_PATH), "bytes")
-    native = os.path.join(os.path.dirname(HERE), "_native.so")
-    _run(["gcc", "-O2", "-std=gnu11", "-fPIC", "-shared", "-Wall", "-I" + sysconfig.get_path("include"), os.path.join(HERE, "native.c"),
-          "-o", native, "-ldl"])
-    if verbose:
-        print("built", os.path.relpath(native, HERE), os.path.getsize(native), "bytes")
     if LIB_PATH == os.path.join(HERE, "libhchip.so"):
         # C++ host mirror + HCMatrixBench (links the library just built, and the Linux stand-in for
         # Accelerate that its CPU leg calls the way the reference's CPUBackend calls Accelerate)
@@ -202,6 +197,12 @@ def build_all(verbose=True):
               "-L" + os.path.join(ROCM, "lib"), "-Wl,-rpath-link," + os.path.join(ROCM, "lib"), "-ldl", "-lm", "-lpthread"])
         if verbose:
             print("built", os.path.relpath(bench, HERE))
+    # What HIPBackend calls the library through (needs Python's headers, like nothing above)
+    native = os.path.join(os.path.dirname(HERE), "_native" + sysconfig.get_config_var("EXT_SUFFIX"))
+    _run(["gcc", "-O2", "-std=gnu11", "-fPIC", "-shared", "-Wall", "-I" + sysconfig.get_path("include"), os.path.join(HERE, "native.c"),
+          "-o", native, "-ldl"])
+    if verbose:
+        print("built", os.path.relpath(native, HERE), os.path.getsize(native), "bytes")
     return LIB_PATH
 
 

@@ -3,12 +3,14 @@ import ctypes
 import gc
 import os
 import subprocess
+import sysconfig
 import weakref
 
 import numpy as np
 import pytest
 
 from honeycrisp_amd import backend as backend_module
+from honeycrisp_amd.csrc import build
 from honeycrisp_amd.descriptors import BroadcastStrides, DType
 
 native = pytest.importorskip("honeycrisp_amd._native")
@@ -196,3 +198,13 @@ def test_a_library_without_the_calls_leaves_no_context_behind(monkeypatch):
     with pytest.raises(ImportError, match="hc_malloc"):
         backend_module.HIPBackend()
     assert Library.shut == [4096]
+
+
+def test_the_extension_is_built_last_and_for_one_python(monkeypatch):
+    """What needs neither Python's headers nor gcc does not fail with it, and another Python does not take it for its own."""
+    outputs = []
+    monkeypatch.setattr(build, "_run", lambda command: outputs.append(command[command.index("-o") + 1]))
+    monkeypatch.setattr(build, "build_kernel", lambda name, source, flags: name)
+    build.build_all(verbose=False)
+    assert os.path.basename(outputs[-1]) == "_native" + sysconfig.get_config_var("EXT_SUFFIX")
+    assert os.path.basename(outputs[-2]) == "HCMatrixBench"
