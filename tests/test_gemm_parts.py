@@ -1,4 +1,6 @@
 """Products of few tiles over a long K, computed in parts of K that are added up: the ends of tiles, parts and rows, every layout."""
+from ctypes import c_void_p
+
 import numpy as np
 import pytest
 
@@ -13,10 +15,22 @@ pytestmark = pytest.mark.gpu
 SHAPES = [(64, 3072, 64), (64, 3136, 80), (9, 3073, 461), (5, 4097, 821), (65, 3137, 63), (16, 3200, 4096), (200, 4099, 130), (512, 3136, 1024),
           (127, 8191, 33), (300, 5000, 256), (40, 3330, 1001), (520, 3200, 1024)]
 
+# one launch, by rows, K and columns of what is stored: more than half as many tiles as compute units; one output less than a tile; fp16 with few columns and
+# many rows; fp32 with no more parts than an output has chains in that launch
+WHOLE = {(520, 3200, 1024), (1024, 3200, 520), (65, 3137, 63), (63, 3137, 65)}
+WHOLE = {DType.float16: WHOLE | {(4096, 3200, 16)},
+         DType.float32: WHOLE | {(512, 3136, 1024), (1024, 3136, 512), (16, 3200, 4096), (4096, 3200, 16)}}
+SHORT = {DType.float16: "f16", DType.float32: "f32"}
+
+
+def error_bound(k, size, want, dtype):
+    """k additions in fp32, each off by half a last place of a partial sum, and one rounding to the result's type."""
+    return k * 2.0 ** -24 * size + (2.0 ** -11 * np.abs(want) + 2.0 ** -24 if dtype == DType.float16 else 0)
+
 
 @pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
 @pytest.mark.parametrize("m,k,n", SHAPES, ids=str)
-def test_against_float64(hip_backend, dtype, m, k, n):
+def test_against_float64(hip_backend, capfd, dtype, m, k, n):
     rng = np.random.default_rng(m * k + n)
     with hip_backend.use():
         for ta in (False, True):
@@ -29,10 +43,54 @@ def test_against_float64(hip_backend, dtype, m, k, n):
                     want, size = a @ b, np.abs(a) @ np.abs(b)
                     if to:
                         want, size = want.T, size.T
+                    names = kernels_of(hip_backend, capfd, lambda: Tensor.matmul(x, ta, y, tb, to))
+                    along = ("k" if tb else "m") + ("n" if ta else "k") if to else ("m" if ta else "k") + ("k" if tb else "n")
+                    edge = "_e" if m % 64 or n % 64 or k % (128 // np.dtype(dtype.numpy).itemsize) else ""
+                    in_parts = ["hc_gemm_%s_part_64x64_%s%s" % (SHORT[dtype], along, edge), "hc_gemm_part_sum_%s" % SHORT[dtype]]
+                    assert (names == in_parts) == (((n, k, m) if to else (m, k, n)) not in WHOLE[dtype]), (names, in_parts)
                     got = Tensor.matmul(x, ta, y, tb, to).numpy().astype(np.float64)
-                    # k additions in fp32, each off by half a last place of a partial sum, and one rounding to the result's type
-                    bound = k * 2.0 ** -24 * size + (2.0 ** -11 * np.abs(want) + 2.0 ** -24 if dtype == DType.float16 else 0)
-                    assert np.all(np.abs(got - want) <= bound), (ta, tb, to, np.max(np.abs(got - want) / size))
+                    assert np.all(np.abs(got - want) <= error_bound(k, size, want, dtype)), (ta, tb, to, np.max(np.abs(got - want) / size))
+
+
+@pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
+def test_operands_and_result_at_odd_elements(hip_backend, capfd, dtype):
+    m, k, n, guard, es = 65, 3137, 80, 33, np.dtype(dtype.numpy).itemsize
+    rng = np.random.default_rng(11)
+    with hip_backend.use():
+        for ta in (False, True):
+            for tb in (False, True):
+                a, b = (rng.standard_normal(shape).astype(dtype.numpy) for shape in ((k, m) if ta else (m, k), (n, k) if tb else (k, n)))
+                around = lambda x: hip_backend.upload(np.concatenate([np.full(guard, np.nan, dtype.numpy), x.ravel(), np.full(guard, np.nan, dtype.numpy)]))
+                x, y, out = around(a), around(b), around(np.zeros((m, n), dtype.numpy))
+                at = lambda data: c_void_p(data.ptr + guard * es)
+                call = lambda: hip_backend._check(hip_backend._lib.hc_matmul(hip_backend._ctx, dtype, 1, at(x), int(ta), at(y), int(tb), 0, m, k, n, at(out)))
+                names = kernels_of(hip_backend, capfd, call)
+                assert names[0] == "hc_gemm_%s_part_64x64_%s%s_e" % (SHORT[dtype], "m" if ta else "k", "k" if tb else "n"), names
+                call()
+                got = Tensor(dataHandle=out, shape=[m * n + 2 * guard], dtype=dtype).numpy().astype(np.float64)
+                assert np.isnan(got[:guard]).all() and np.isnan(got[-guard:]).all()
+                a, b = (a.T if ta else a).astype(np.float64), (b.T if tb else b).astype(np.float64)
+                got, want = got[guard:-guard].reshape(m, n), a @ b
+                assert np.all(np.abs(got - want) <= error_bound(k, np.abs(a) @ np.abs(b), want, dtype))
+
+
+# a few rows, a few columns, both (the columns are too many tiles for parts, one launch), and both over operands that were copied to whole lines first
+@pytest.mark.parametrize("dtype,m,k,n,parts,tb", [(DType.float16, 4104, 3200, 1024, "kn", False), (DType.float32, 4104, 4160, 1024, "kn", False),
+                                                  (DType.float16, 1024, 3200, 4104, "kk", True), (DType.float16, 2061, 3072, 2056, "kn", False),
+                                                  (DType.float16, 2061, 3201, 2053, "kk", True)], ids=str)
+def test_fringes_in_parts(hip_backend, capfd, dtype, m, k, n, parts, tb):
+    rng = np.random.default_rng(m + n)
+    a, b = (rng.standard_normal((m, k)) / np.sqrt(k)).astype(dtype.numpy), rng.standard_normal((n, k) if tb else (k, n)).astype(dtype.numpy)
+    with hip_backend.use():
+        x, y = Tensor(data=a), Tensor(data=b)
+        call = lambda: Tensor.matmul(x, False, y, tb, False)
+        names = kernels_of(hip_backend, capfd, call)
+        assert sum("_part_64x64_" + parts in name for name in names) == 1 and names.count("hc_gemm_part_sum_" + SHORT[dtype]) == 1, names
+        assert ("hc_copy_lines_b2" in names) == (k % 2 == 1)
+        got = call().numpy().astype(np.float64)
+    a, b = a.astype(np.float64), (b.T if tb else b).astype(np.float64)
+    want = a @ b
+    assert np.all(np.abs(got - want) <= error_bound(k, np.abs(a) @ np.abs(b), want, dtype))
 
 
 def same_bits(hip, fn):
@@ -91,7 +149,7 @@ def test_products_over_one_input_share_their_launches(hip_backend, capfd, dtype,
     tensor = lambda *shape: Tensor(data=rng.standard_normal(shape).astype(np.float32), dtype=dtype)
     with hip_backend.use():
         x, ws, rows = tensor(m, k), [tensor(k, n) for _ in range(count)], [tensor(n) for _ in range(count)]
-        if "hc_gemm_part_sum_%s" % {DType.float16: "f16", DType.float32: "f32"}[dtype] not in kernels_of(
+        if "hc_gemm_part_sum_%s" % SHORT[dtype] not in kernels_of(
                 hip_backend, capfd, lambda: Tensor.matmul(x, False, ws[0], False, False)):
             assert dtype == DType.float32 and m * n > 200000      # (longer chains than those of a workgroup's waves)
             return
