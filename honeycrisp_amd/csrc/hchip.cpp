@@ -2178,11 +2178,12 @@ extern "C" int hc_cumulative(hc_ctx* ctx, int op, int dtype, const void* in, voi
   // elements, one tile of a wave ([4096, 100] 3.6 / 4.7), nor many of up to 512 (fp16 [16384, 300] 11.1 / 13.5); and not a few rows so long that one
   // unit each takes longer than all units and a second launch: [8, 60000] 9.2 / 9.4, [8, 100000] 9.6 / 14.1, fp16 [8, 45000] 9.5 / 9.1 and [8, 60000]
   // 9.6 / 11.2, int64 [8, 20000] 8.9 / 7.3 and [8, 30000] 9.1 / 9.6. With a row for every fourth unit (int64: second) the totals' pass over the data
-  // costs more at any length: [64, 80000] 21 / 14, [128, 200000] 97 / 54, int64 [64, 60000] 22.1 / 21.5 and [64, 100000] 33 / 48.
+  // costs more at any length: [64, 80000] 22 / 14, [64, 4000000] 1158 / 815, [128, 400000] 221 / 100, fp16, half the bytes at the same arithmetic, [64, 80000]
+  // 21 / 15, [64, 200000] 49 / 42, [64, 4000000] 1201 / 961, [128, 400000] 186 / 80, int64 [128, 400000] 312 / 222, but [64, 60000] 22.1 / 21.5 and [64, 100000] 33 / 48.
   const uint64_t longest = dtype == HC_F32 ? 57344 : dtype == HC_F16 ? 49152 : 24576;
   if (inner == 1 && reduce > 256 && (reduce >= 512 || outer <= 2048) &&
       ((uint64_t)reduce <= longest || (uint64_t)outer >= cus / (dtype == HC_I64 ? 2 : 4))) {
-    // (1024 lanes while a unit has no more than one row of more than a quarter of a tile: [8, 4096] 3.9 / 3.1, [512, 2000] 3.9 / 4.1)
+    // (1024 lanes while a unit has fewer than two rows, each of more than a quarter of a tile: [8, 4096] 3.9 / 3.1, [512, 2000] 3.9 / 4.1)
     const bool wide = reduce > 1024 && (uint64_t)outer < 2 * cus;
     snprintf(name, sizeof(name), "hc_cumulative_%s_rowblock%s_%s", opn, wide ? "_wide" : "", tn);
     return launch(ctx, name, (uint64_t)outer, 1, &k, sizeof(k), wide ? 1024 : HCK_BLOCK);
