@@ -47,9 +47,32 @@ def test_against_float64(hip_backend, capfd, dtype, m, k, n):
                     along = ("k" if tb else "m") + ("n" if ta else "k") if to else ("m" if ta else "k") + ("k" if tb else "n")
                     edge = "_e" if m % 64 or n % 64 or k % (128 // np.dtype(dtype.numpy).itemsize) else ""
                     in_parts = ["hc_gemm_%s_part_64x64_%s%s" % (SHORT[dtype], along, edge), "hc_gemm_part_sum_%s" % SHORT[dtype]]
-                    assert (names == in_parts) == (((n, k, m) if to else (m, k, n)) not in WHOLE[dtype]), (names, in_parts)
+                    rows, cols = (n, m) if to else (m, n)
+                    whole = (rows, k, cols) in WHOLE[dtype] or (k < 4096 and (
+                        along == "mn" and min(m, n) <= 16 if dtype == DType.float32 else along == "kn" and rows >= 640 and cols < 64))
+                    assert (names == in_parts) == (not whole), (names, in_parts)
                     got = Tensor.matmul(x, ta, y, tb, to).numpy().astype(np.float64)
                     assert np.all(np.abs(got - want) <= error_bound(k, size, want, dtype)), (ta, tb, to, np.max(np.abs(got - want) / size))
+
+
+# both sides of the rule's lines below K = 4096: fp32 with both operands along M and N and 16 or 17 columns; fp16 with A along K and B along N, 640 rows and 63
+# columns, unless the rows start at odd halfs or the waves that split K are more than three quarters of the compute units
+@pytest.mark.parametrize("dtype,m,k,n,ta,parts", [
+    (DType.float32, 400, 4032, 16, True, False), (DType.float32, 400, 4096, 16, True, True), (DType.float32, 400, 4032, 17, True, True), (DType.float32, 400, 4032, 16, False, True),
+    (DType.float32, 16, 4032, 400, True, False), (DType.float16, 640, 4032, 48, False, False), (DType.float16, 639, 4032, 48, False, True),
+    (DType.float16, 640, 4096, 48, False, True), (DType.float16, 640, 4032, 64, False, True), (DType.float16, 640, 4031, 48, False, True),
+    (DType.float16, 1552, 4032, 48, False, True), (DType.float16, 1536, 4032, 63, False, False), (DType.float16, 640, 4032, 48, True, True)], ids=str)
+def test_short_products_of_few_columns(hip_backend, capfd, dtype, m, k, n, ta, parts):
+    rng = np.random.default_rng(n)
+    a, b = (rng.standard_normal((m, k)) / np.sqrt(k)).astype(dtype.numpy), rng.standard_normal((k, n)).astype(dtype.numpy)
+    with hip_backend.use():
+        x, y = Tensor(data=np.ascontiguousarray(a.T) if ta else a), Tensor(data=b)
+        call = lambda: Tensor.matmul(x, ta, y, False, False)
+        assert ("hc_gemm_part_sum_" + SHORT[dtype] in kernels_of(hip_backend, capfd, call)) == parts
+        got = call().numpy().astype(np.float64)
+    a, b = a.astype(np.float64), b.astype(np.float64)
+    want = a @ b
+    assert np.all(np.abs(got - want) <= error_bound(k, np.abs(a) @ np.abs(b), want, dtype))
 
 
 @pytest.mark.parametrize("dtype", [DType.float16, DType.float32], ids=lambda d: d.name)
